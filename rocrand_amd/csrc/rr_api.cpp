@@ -706,8 +706,9 @@ public:
         m_S = engines;
         if(!m_states)
         {
-            // two state buffers: a call reads one and leaves the advanced states in the other
-            if(hipMalloc(&m_states, 2 * state_words() * sizeof(uint32_t)) != hipSuccess)
+            // two state buffers: a call reads one and leaves the advanced states in the other;
+            // then the set-up's scratch
+            if(hipMalloc(&m_states, (2 * state_words() + INTER_INIT_SCRATCH) * sizeof(uint32_t)) != hipSuccess)
             {
                 m_states = nullptr;
                 return ROCRAND_STATUS_ALLOCATION_FAILED;
@@ -717,7 +718,9 @@ public:
         m_start = (uint32_t)(offset % m_S);
         uint32_t seeded[6];
         seed_state(seeded);
-        if(launch_interleaved_init(m_kind, cur_states(), seeded, m_start, offset / m_S, m_S, stream) != hipSuccess)
+        if(launch_interleaved_init(m_kind, cur_states(), m_states + 2 * state_words(), seeded, m_start, offset / m_S, m_S,
+                                   stream)
+           != hipSuccess)
             return ROCRAND_STATUS_LAUNCH_FAILURE;
         m_initialized = true;
         return ROCRAND_STATUS_SUCCESS;
@@ -805,7 +808,7 @@ private:
     unsigned long long m_seed        = 0;
     uint4              m_seed4       = {2, 8, 16, 128};
     bool               m_initialized = false;
-    uint32_t*          m_states      = nullptr; // 2 * state_words() words
+    uint32_t*          m_states      = nullptr; // 2 * state_words() words, then the set-up's scratch
     uint32_t           m_cur         = 0;       // which half holds the current states
     uint32_t           m_start       = 0;
     uint32_t           m_S           = INTERLEAVED_ENGINES; // engines

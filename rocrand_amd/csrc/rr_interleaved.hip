@@ -10,11 +10,12 @@
 //
 // Engine e is initialised by a jump-ahead kernel: the seeded state advanced by
 // e subsequences and then by offset/S + [e < offset mod S] steps, with matrix
-// powers (mod-m 3x3 for the MRGs, GF(2) for XORWOW / LFSR113) computed on the
-// host once per device (rr_tables.cpp).
+// powers (mod-m 3x3 for the MRGs, computed on the host once per device in
+// rr_tables.cpp; for XORWOW and LFSR113 see gf2_low_kernel).
 #include "rr_interleaved_dev.hpp"
 
 #include <algorithm>
+#include <mutex>
 
 namespace rr
 {
@@ -32,6 +33,130 @@ __global__ __launch_bounds__(256) void init_kernel(uint32_t* states, const devic
         return;
     ieng<K> g = seeded;
     g.init(t, e, base_off + (e < start ? 1u : 0u));
+    g.store(states, e, ns);
+}
+
+// XORWOW / LFSR113 engines.  With X = one subsequence and e = 256 hi + lo, the engine's
+// bits are X^(256 hi) X^lo M^(steps) (seeded state): 256 low jumps (of the state after
+// `steps` and after one more) are made once, a wavefront each, and every block of 256
+// engines then takes one matrix product with its own X^(256 hi), which its lanes share.
+// One shared-matrix product per engine takes 960 (XORWOW) VALU instructions and bounds it; the base-4
+// digits of e, up to three products each and different for each lane, took 19 of them
+// (150 us for 131072 engines; now 2.6 and 8.1 us).  The powers are made on the
+// device, once (gf2_powers_kernel).
+constexpr uint32_t GF2_LO = 256, GF2_HI = 1024; // hi beyond 1024 (DYNAMIC grids): base-4 digits from 4^9 on
+constexpr uint32_t GF2_STEPS = 32;              // M^(4^k)
+static_assert((uint64_t)GF2_LO * GF2_HI == 1ull << 18, "the digits of e / (LO * HI) start at 4^9");
+constexpr uint32_t GF2_POWERS = GF2_LO + GF2_HI + GF2_STEPS;
+__device__ uint32_t d_xorwow_powers[GF2_POWERS * 32 * 5 * 5];
+__device__ uint32_t d_lfsr_powers[GF2_POWERS * 32 * 4 * 4];
+
+// X^lo and M^(4^k) by columns for gf2_wave (word w of column c at [w * 32 N + c]),
+// X^(256 hi) by rows; thread r makes row r.
+template<int N>
+__global__ __launch_bounds__(192) void gf2_powers_kernel(const uint32_t* seq, const uint32_t* jump, uint32_t* powers)
+{
+    constexpr uint32_t    R = 32 * N;
+    __shared__ uint32_t   rows[R][N];
+    __shared__ alignas(16) uint32_t lds[R * N];
+    const uint32_t        m = blockIdx.x, r = threadIdx.x;
+    uint32_t              v[N];
+#pragma unroll
+    for(int k = 0; k < N; k++)
+        v[k] = (uint32_t)k == r / 32 ? 1u << r % 32 : 0u;
+    if(m < GF2_LO + GF2_HI)
+        gf2_jump_block<N>(v, seq, m < GF2_LO ? m : (uint64_t)(m - GF2_LO) * GF2_LO, lds);
+    else if(r < R)
+        for(int k = 0; k < N; k++)
+            v[k] = jump[((size_t)(m - GF2_LO - GF2_HI) * R + r) * N + k];
+    if(r < R)
+#pragma unroll
+        for(int k = 0; k < N; k++)
+            rows[r][k] = v[k];
+    __syncthreads();
+    uint32_t* out = powers + (size_t)m * R * N;
+    for(uint32_t i = r; i < R * N; i += blockDim.x)
+    {
+        if(m >= GF2_LO && m < GF2_LO + GF2_HI)
+        {
+            out[i] = rows[i / N][i % N];
+            continue;
+        }
+        const uint32_t w = i / R, c = i % R; // rows 32 w .. 32 w + 31 of column c
+        uint32_t       x = 0;
+        for(uint32_t b = 0; b < 32; b++)
+            x |= (rows[32 * w + b][c / 32] >> c % 32 & 1u) << b;
+        out[i] = x;
+    }
+}
+
+// v = m v for one wavefront and a wavefront-uniform v: lane l forms output bits l, l + 64,
+// ... as the parity of v with those columns, and the ballots are the output words.
+template<int N>
+__device__ __forceinline__ void gf2_wave(const uint32_t* m, uint32_t (&v)[N])
+{
+    constexpr uint32_t R = 32 * N;
+    const uint32_t     lane = threadIdx.x & 63u;
+    uint32_t           r[N + 1];
+#pragma unroll
+    for(uint32_t g = 0; g < (R + 63) / 64; g++)
+    {
+        const uint32_t c = 64 * g + lane < R ? 64 * g + lane : lane; // the last group's spare lanes repeat column `lane`
+        uint32_t       x = 0;
+#pragma unroll
+        for(int w = 0; w < N; w++)
+            x = xor_and(x, m[w * R + c], v[w]);
+        const uint64_t b = __ballot(__popc(x) & 1);
+        r[2 * g]         = (uint32_t)b;
+        if(2 * g + 1 < N + 1)
+            r[2 * g + 1] = (uint32_t)(b >> 32);
+    }
+#pragma unroll
+    for(int w = 0; w < N; w++)
+        v[w] = r[w];
+}
+
+// low[(which * N + w) * LO + lo]: word w of X^lo M^(steps + which) (seeded state).
+template<int N>
+struct gf2_vec
+{
+    uint32_t v[N];
+};
+template<int N>
+__global__ __launch_bounds__(256) void gf2_low_kernel(const uint32_t* powers, gf2_vec<N> seeded, uint64_t steps0,
+                                                      uint64_t steps1, uint32_t* low)
+{
+    constexpr size_t SZ = 32 * N * N;
+    const uint32_t   wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
+    const uint32_t   which = wave / GF2_LO, lo = wave % GF2_LO;
+    uint64_t         n = which ? steps1 : steps0;
+    for(int k = 0; n > 0; n >>= 2, k++)
+        for(uint32_t i = 0; i < (uint32_t)(n & 3u); i++)
+            gf2_wave<N>(powers + (GF2_LO + GF2_HI + k) * SZ, seeded.v);
+    gf2_wave<N>(powers + lo * SZ, seeded.v);
+    if((threadIdx.x & 63u) == 0)
+#pragma unroll
+        for(int w = 0; w < N; w++)
+            low[(which * N + w) * GF2_LO + lo] = seeded.v[w];
+}
+
+template<inter_kind K>
+__global__ __launch_bounds__(256) void gf2_init_kernel(uint32_t* states, const uint32_t* powers, const uint32_t* seq,
+                                                       ieng<K> seeded, uint32_t start, uint64_t steps0,
+                                                       uint64_t steps1, const uint32_t* low, uint32_t ns)
+{
+    constexpr int       N = ieng<K>::N;
+    constexpr size_t    SZ = 32 * N * N;
+    __shared__ alignas(16) uint32_t lds[SZ];
+    const uint32_t      e = blockIdx.x * GF2_LO + threadIdx.x; // ns is a multiple of 256
+    const uint32_t      which = e < start ? 1u : 0u;
+    ieng<K>             g = seeded;
+#pragma unroll
+    for(int w = 0; w < N; w++)
+        g.bits()[w] = low[(which * N + w) * GF2_LO + threadIdx.x];
+    g.count(which ? steps1 : steps0);
+    gf2_apply_block<N>(g.bits(), powers + (GF2_LO + blockIdx.x % GF2_HI) * SZ, 1, lds);
+    gf2_jump_block<N>(g.bits(), seq + 9 * SZ, blockIdx.x / GF2_HI, lds);
     g.store(states, e, ns);
 }
 
@@ -201,7 +326,7 @@ __global__ __launch_bounds__(256) void generate_chunked_kernel(interleaved_call 
     {
         // GF(2) jumps: k0 is the same for the whole block, which stages each matrix in
         // LDS once; every thread takes part (barriers) before idle ones leave
-        __shared__ uint32_t mat[ieng<K>::LDS_WORDS];
+        __shared__ alignas(16) uint32_t mat[ieng<K>::LDS_WORDS];
         eng.load(c.states, eid, S);
         eng.advance_block(t, k0 * IN, mat);
         if(idle)
@@ -368,9 +493,41 @@ hipError_t dispatch(out_kind o, const interleaved_call& c, hipStream_t s)
     return hipErrorInvalidValue;
 }
 
+// The powers of the current device, made on its first XORWOW / LFSR113 generator.
 template<inter_kind K>
-hipError_t launch_init_k(uint32_t* states, const uint32_t* seed_state, uint32_t start, uint64_t base_off,
-                         uint32_t ns, hipStream_t s)
+hipError_t get_gf2_powers(const device_tables& t, const uint32_t** out)
+{
+    constexpr int     N = ieng<K>::N;
+    static std::mutex mtx;
+    static uint32_t*  made[64] = {};
+    int               dev = 0;
+    hipError_t        err = hipGetDevice(&dev);
+    if(err != hipSuccess)
+        return err;
+    if(dev < 0 || dev >= 64)
+        return hipErrorInvalidDevice;
+    std::lock_guard<std::mutex> lock(mtx);
+    if(made[dev] == nullptr)
+    {
+        void* p = nullptr;
+        err     = K == inter_kind::xorwow ? hipGetSymbolAddress(&p, HIP_SYMBOL(d_xorwow_powers))
+                                          : hipGetSymbolAddress(&p, HIP_SYMBOL(d_lfsr_powers));
+        if(err != hipSuccess)
+            return err;
+        hipLaunchKernelGGL((gf2_powers_kernel<N>), dim3(GF2_POWERS), dim3(192), 0, 0,
+                           K == inter_kind::xorwow ? t.xorwow_seq : t.lfsr_seq,
+                           K == inter_kind::xorwow ? t.xorwow_jump : t.lfsr_jump, static_cast<uint32_t*>(p));
+        if((err = hipGetLastError()) != hipSuccess || (err = hipStreamSynchronize(0)) != hipSuccess)
+            return err;
+        made[dev] = static_cast<uint32_t*>(p);
+    }
+    *out = made[dev];
+    return hipSuccess;
+}
+
+template<inter_kind K>
+hipError_t launch_init_k(uint32_t* states, uint32_t* low, const uint32_t* seed_state, uint32_t start,
+                         uint64_t base_off, uint32_t ns, hipStream_t s)
 {
     device_tables t;
     hipError_t    err = get_device_tables(t);
@@ -378,28 +535,41 @@ hipError_t launch_init_k(uint32_t* states, const uint32_t* seed_state, uint32_t 
         return err;
     ieng<K> seeded;
     seeded.set(seed_state);
-    hipLaunchKernelGGL((init_kernel<K>), dim3((ns + 255) / 256), dim3(256), 0, s, states, t, seeded, start, base_off,
-                       ns);
+    if constexpr(K == inter_kind::xorwow || K == inter_kind::lfsr113)
+    {
+        constexpr int   N = ieng<K>::N;
+        const uint32_t* powers = nullptr;
+        if((err = get_gf2_powers<K>(t, &powers)) != hipSuccess)
+            return err;
+        const uint64_t steps0 = ieng<K>::steps(base_off), steps1 = ieng<K>::steps(base_off + 1);
+        gf2_vec<N>     v;
+        std::copy(seeded.bits(), seeded.bits() + N, v.v);
+        hipLaunchKernelGGL((gf2_low_kernel<N>), dim3(2 * GF2_LO / 4), dim3(256), 0, s, powers, v, steps0, steps1, low);
+        hipLaunchKernelGGL((gf2_init_kernel<K>), dim3(ns / GF2_LO), dim3(GF2_LO), 0, s, states, powers,
+                           K == inter_kind::xorwow ? t.xorwow_seq : t.lfsr_seq, seeded, start, steps0, steps1, low, ns);
+    }
+    else
+        hipLaunchKernelGGL((init_kernel<K>), dim3(ns / 256), dim3(256), 0, s, states, t, seeded, start, base_off, ns);
     return hipGetLastError();
 }
 
 } // namespace
 
-hipError_t launch_interleaved_init(inter_kind k, uint32_t* states, const uint32_t* seed_state, uint32_t start,
-                                   uint64_t base_offset, uint32_t engines, hipStream_t s)
+hipError_t launch_interleaved_init(inter_kind k, uint32_t* states, uint32_t* scratch, const uint32_t* seed_state,
+                                   uint32_t start, uint64_t base_offset, uint32_t engines, hipStream_t s)
 {
     if(engines == 0 || engines % 256 != 0)
         return hipErrorInvalidValue;
     switch(k)
     {
         case inter_kind::mrg32k3a:
-            return launch_init_k<inter_kind::mrg32k3a>(states, seed_state, start, base_offset, engines, s);
+            return launch_init_k<inter_kind::mrg32k3a>(states, scratch, seed_state, start, base_offset, engines, s);
         case inter_kind::mrg31k3p:
-            return launch_init_k<inter_kind::mrg31k3p>(states, seed_state, start, base_offset, engines, s);
+            return launch_init_k<inter_kind::mrg31k3p>(states, scratch, seed_state, start, base_offset, engines, s);
         case inter_kind::xorwow:
-            return launch_init_k<inter_kind::xorwow>(states, seed_state, start, base_offset, engines, s);
+            return launch_init_k<inter_kind::xorwow>(states, scratch, seed_state, start, base_offset, engines, s);
         case inter_kind::lfsr113:
-            return launch_init_k<inter_kind::lfsr113>(states, seed_state, start, base_offset, engines, s);
+            return launch_init_k<inter_kind::lfsr113>(states, scratch, seed_state, start, base_offset, engines, s);
     }
     return hipErrorInvalidValue;
 }

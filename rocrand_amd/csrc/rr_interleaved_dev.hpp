@@ -147,39 +147,71 @@ struct ieng<inter_kind::mrg31k3p> : ieng<inter_kind::mrg32k3a>
     }
 };
 
-// Base-4 digit expansion with matrix k = M^(c * 4^k) applied digit times
-// (rocrand_xorwow.h:186-200, rocrand_lfsr113.h jump()).
-template<int N>
-__device__ void gf2_jump(uint32_t* v, const uint32_t* mats, uint64_t n)
+// acc ^ (a & b) in one instruction (v_bitop3_b32)
+__device__ __forceinline__ uint32_t xor_and(uint32_t acc, uint32_t a, uint32_t b)
 {
-    for(int k = 0; n > 0; n >>= 2, k++)
-    {
-        const uint32_t d = (uint32_t)(n & 3u);
-        for(uint32_t i = 0; i < d; i++)
-            gf2_mat_vec<N>(mats + (size_t)k * 32 * N * N, v);
-    }
+    return __builtin_amdgcn_bitop3_b32(acc, a, b, 0x78);
 }
 
-// gf2_jump for a whole block whose lanes share `n` (block-uniform): each 4^k power is
-// staged once in LDS (`lds`: 32 N^2 words) and read from there by every lane, instead
-// of every wavefront fetching the same rows through the scalar or vector caches.
-// Every thread of the block must call it.
+// GF(2) matrix (row per input bit, N words per row; 16-byte aligned, the same for every
+// lane, normally in LDS) times each lane's vector, four rows per N 16-byte broadcast reads.
+template<int N>
+__device__ __forceinline__ void gf2_mat_vec_shared(const uint32_t* m, uint32_t* v)
+{
+    const uint4* q    = reinterpret_cast<const uint4*>(m);
+    uint32_t     r[N] = {};
+#pragma unroll
+    for(int i = 0; i < N; i++)
+    {
+        const uint32_t vi = v[i];
+#pragma unroll 2
+        for(int j = 0; j < 32; j += 4, q += N)
+        {
+            uint32_t w[4 * N];
+#pragma unroll
+            for(int k = 0; k < N; k++)
+            {
+                const uint4 t = q[k];
+                w[4 * k] = t.x, w[4 * k + 1] = t.y, w[4 * k + 2] = t.z, w[4 * k + 3] = t.w;
+            }
+#pragma unroll
+            for(int l = 0; l < 4; l++)
+            {
+                const uint32_t b = 0u - ((vi >> (j + l)) & 1u);
+#pragma unroll
+                for(int k = 0; k < N; k++)
+                    r[k] = xor_and(r[k], w[l * N + k], b);
+            }
+        }
+    }
+#pragma unroll
+    for(int k = 0; k < N; k++)
+        v[k] = r[k];
+}
+
+// v = m v for a whole block with one matrix, staged in LDS (`lds`: 32 N^2 words, 16-byte
+// aligned).  Every thread of the block must call it.
+template<int N>
+__device__ __forceinline__ void gf2_apply_block(uint32_t* v, const uint32_t* m, uint32_t times, uint32_t* lds)
+{
+    __syncthreads(); // the previous matrix is no longer read
+    for(int w = threadIdx.x; w < 32 * N * N; w += blockDim.x)
+        lds[w] = m[w];
+    __syncthreads();
+    for(uint32_t i = 0; i < times; i++)
+        gf2_mat_vec_shared<N>(lds, v);
+}
+
+// Base-4 digit expansion with matrix k = M^(c * 4^k) applied digit times
+// (rocrand_xorwow.h:186-200, rocrand_lfsr113.h jump()), for a whole block whose lanes
+// share `n` (block-uniform): each 4^k power is staged once in LDS and read from there by
+// every lane.  Every thread of the block must call it.
 template<int N>
 __device__ void gf2_jump_block(uint32_t* v, const uint32_t* mats, uint64_t n, uint32_t* lds)
 {
-    constexpr int SZ = 32 * N * N;
     for(int k = 0; n > 0; n >>= 2, k++)
-    {
-        const uint32_t d = (uint32_t)(n & 3u);
-        if(d == 0)
-            continue;
-        __syncthreads(); // the previous matrix is no longer read
-        for(int w = threadIdx.x; w < SZ; w += blockDim.x)
-            lds[w] = mats[(size_t)k * SZ + w];
-        __syncthreads();
-        for(uint32_t i = 0; i < d; i++)
-            gf2_mat_vec<N>(lds, v);
-    }
+        if((n & 3u) != 0)
+            gf2_apply_block<N>(v, mats + (size_t)k * 32 * N * N, (uint32_t)(n & 3u), lds);
 }
 
 template<>
@@ -208,24 +240,18 @@ struct ieng<inter_kind::xorwow>
             s.x[j] = w[1 + j];
     }
     __device__ uint32_t next() { return xorwow_next(s); }
-    __device__ void init(const device_tables& t, uint32_t e, uint64_t off)
-    {
-        gf2_jump<5>(s.x, t.xorwow_seq, e);
-        gf2_jump<5>(s.x, t.xorwow_jump, off);
-        s.d += (uint32_t)off * 362437u; // rocrand_xorwow.h:134-145
-    }
-    // k steps ahead: the 4^j powers for the xorshift part, the Weyl counter linearly
-    __device__ void advance(const device_tables& t, uint64_t k)
-    {
-        gf2_jump<5>(s.x, t.xorwow_jump, k);
-        s.d += (uint32_t)k * 362437u;
-    }
+    static constexpr int N = 5;
+    // the part that jumps as a GF(2) vector, and the Weyl counter's part of k steps
+    // (rocrand_xorwow.h:134-145; a subsequence of 2^67 steps leaves the counter)
+    __host__ __device__ uint32_t* bits() { return s.x; }
+    __host__ __device__ void      count(uint64_t k) { s.d += (uint32_t)k * 362437u; }
+    static uint64_t               steps(uint64_t k) { return k; }
     static constexpr int LDS_WORDS = 32 * 5 * 5;
     // the same for a block sharing k (every thread calls it)
     __device__ void advance_block(const device_tables& t, uint64_t k, uint32_t* lds)
     {
         gf2_jump_block<5>(s.x, t.xorwow_jump, k, lds);
-        s.d += (uint32_t)k * 362437u;
+        count(k);
     }
 };
 
@@ -252,13 +278,11 @@ struct ieng<inter_kind::lfsr113>
             s.z[j] = w[j];
     }
     __device__ uint32_t next() { return lfsr113_next(s); }
-    __device__ void init(const device_tables& t, uint32_t e, uint64_t off)
-    {
-        // lfsr113.hpp:45-62: the step count travels as an unsigned int.
-        gf2_jump<4>(s.z, t.lfsr_seq, (uint32_t)e);
-        gf2_jump<4>(s.z, t.lfsr_jump, (uint32_t)off);
-    }
-    __device__ void advance(const device_tables& t, uint64_t k) { gf2_jump<4>(s.z, t.lfsr_jump, k); }
+    static constexpr int N = 4;
+    __host__ __device__ uint32_t* bits() { return s.z; }
+    __host__ __device__ void      count(uint64_t) {}
+    // lfsr113.hpp:45-62: the step count travels as an unsigned int
+    static uint64_t steps(uint64_t k) { return (uint32_t)k; }
     static constexpr int LDS_WORDS = 32 * 4 * 4;
     __device__ void advance_block(const device_tables& t, uint64_t k, uint32_t* lds)
     {

@@ -70,8 +70,12 @@ constexpr int inter_state_words(inter_kind k)
     return k == inter_kind::lfsr113 ? 4 : 6;
 }
 
+// Scratch words of an engine set-up (the 2 x 256 low jumps of XORWOW and LFSR113, 5 words).
+constexpr size_t INTER_INIT_SCRATCH = 2 * 256 * 5;
+
 hipError_t launch_interleaved_init(inter_kind k,
                                    uint32_t*  states,
+                                   uint32_t*  scratch, // INTER_INIT_SCRATCH words
                                    const uint32_t* seed_state, // one engine's seeded state
                                    uint32_t   start,
                                    uint64_t   base_offset,

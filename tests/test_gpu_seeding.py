@@ -50,3 +50,35 @@ def test_mt19937_seeded_on_two_streams():
     torch.cuda.synchronize()
     for b, seed in zip(bufs, seeds):
         assert np.array_equal(b.cpu().numpy(), _want(O.MT19937, n, seed=seed))
+
+
+@pytest.mark.parametrize("rng", [R.XORWOW, R.LFSR113], ids=["xorwow", "lfsr113"])
+def test_gf2_engine_states_under_new_seeds(rng):
+    """Two words of every engine: no steps, one step more below `offset mod S`, every digit of
+    the step count (past 2^32 steps LFSR113 counts modulo 2^32)."""
+    S = 131072
+    g, n = R.PRNG(rng), 2 * S + 3
+    for seed, offset in ((0, 0), (1, S - 1), (0xFFFFFFFFFFFFFFFF, S), (5, 27 * S + 77), (6, (1 << 50) + 12345),
+                         (7, 0xFFFFFFFFFFFFFFFF)):
+        print(f"case {rng} seed={seed:#x} offset={offset:#x}", flush=True)
+        g.seed = seed
+        g.offset = offset
+        got = _words(g, n)
+        torch.cuda.synchronize()
+        assert np.array_equal(got.cpu().numpy(), _want(rng, n, seed=seed, offset=offset))
+
+
+@pytest.mark.parametrize("rng", [R.XORWOW, R.LFSR113], ids=["xorwow", "lfsr113"])
+@pytest.mark.parametrize("blocks", [256, 1024, 2048])
+def test_gf2_engine_states_on_other_grids(rng, blocks):
+    """Engine counts below the DEFAULT grid's, at the end of the high jumps' table (2^18) and past it."""
+    S = 256 * blocks
+    R.set_dynamic_grid(rng, 256, blocks)
+    try:
+        g = R.PRNG(rng, seed=77, offset=5 * S + 3)
+        g.set_ordering(R.ORDERING_PSEUDO_DYNAMIC)
+        got = _words(g, S + 9)
+        torch.cuda.synchronize()
+    finally:
+        R.set_dynamic_grid(rng, 0, 0)
+    assert np.array_equal(got.cpu().numpy(), _want(rng, S + 9, seed=77, offset=5 * S + 3, grid=(256, blocks)))
