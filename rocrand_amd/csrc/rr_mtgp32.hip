@@ -31,8 +31,6 @@
 
 #include <algorithm>
 #include <mutex>
-#include <string.h>
-#include <vector>
 
 extern "C" const unsigned char rr_mtgp32_params_begin[];
 extern "C" const unsigned char rr_mtgp32_params_end[];
@@ -67,6 +65,56 @@ const mtgp_param* params()
     static_assert(sizeof(mtgp_param) == 36 * 4, "layout of mtgp32_11213.bin");
     return reinterpret_cast<const mtgp_param*>(rr_mtgp32_params_begin);
 }
+
+// The parameter sets on the device (uploaded once per device).
+__device__ mtgp_param d_params[MTGP_GENS];
+
+// rocrand_make_state_mtgp32 (rocrand_mtgp32.h:362-390) and rocrand_mtgp32_init_state
+// (:130-145), one wavefront per generator: the seeding recurrence is a chain of 350 uniform
+// steps (scalar instructions), of which lane l keeps words l, l + 64, ...  Bound by that
+// chain (13 us a seed; 512 x 351 words made on the host, copied and waited for, took 380).
+__global__ __launch_bounds__(64) void mtgp_seed_kernel(mtgp_state* states, const mtgp_param* params, uint32_t seed)
+{
+    const uint32_t    b = blockIdx.x, lane = threadIdx.x;
+    const mtgp_param& p = params[b];
+    mtgp_state&       g = states[b];
+    const uint32_t    hidden = p.tbl[4] ^ (p.tbl[8] << 16);
+    uint32_t          tmp    = hidden;
+    tmp += tmp >> 16;
+    tmp += tmp >> 8;
+    const uint32_t fill = (tmp & 0xffu) * 0x01010101u;
+    uint32_t       x    = __builtin_amdgcn_readfirstlane(seed + b + 1);
+    uint32_t       mine = x; // word 0
+    for(uint32_t k = 1; k < MTGP_N; k++)
+    {
+        x = (k == 1 ? hidden : fill) ^ (1812433253u * (x ^ (x >> 30)) + k);
+        if(k % 64 == 0)
+            g.status[k - 64 + lane] = mine;
+        mine = k % 64 == lane ? x : mine;
+    }
+    constexpr uint32_t last = MTGP_N / 64 * 64;
+    for(uint32_t i = last + lane; i < MTGP_RING; i += 64)
+        g.status[i] = i < MTGP_N ? mine : 0u;
+    if(lane == 0)
+    {
+        g.offset = 0;
+        g.pos    = p.pos;
+        g.sh1    = p.sh1;
+        g.sh2    = p.sh2;
+        g.mask   = params[0].mask;
+    }
+    if(lane < 16)
+    {
+        g.tbl[lane] = p.tbl[lane];
+        g.tmp[lane] = p.tmp[lane];
+    }
+}
+
+// d_params of the current device, checked and uploaded on the first call there: the kernel
+// evaluates the recurrence table from its entries at 1, 2, 4 and 8 (the tempering table is
+// linear too and checked with it), and its unmasked ring reads reach off + 255 + pos with
+// off < 1024.
+rocrand_status device_params(const mtgp_param*& out);
 
 struct mtgp_call
 {
@@ -239,6 +287,36 @@ hipError_t dispatch(out_kind o, const mtgp_call& c, hipStream_t s)
     return hipErrorInvalidValue;
 }
 
+rocrand_status device_params(const mtgp_param*& out)
+{
+    static std::mutex  mtx;
+    static mtgp_param* ready[64] = {};
+    int                dev = 0;
+    if(hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
+        return ROCRAND_STATUS_INTERNAL_ERROR;
+    std::lock_guard<std::mutex> lock(mtx);
+    if(ready[dev] == nullptr)
+    {
+        const mtgp_param* p = params();
+        for(unsigned i = 0; i < MTGP_GENS; i++)
+        {
+            if(p[i].pos == 0 || p[i].pos + MTGP_BLOCK > MTGP_N)
+                return ROCRAND_STATUS_INTERNAL_ERROR;
+            for(uint32_t k = 0; k < 16; k++)
+                if(p[i].tbl[k] != mtgp_lin16(k, p[i].tbl[1], p[i].tbl[2], p[i].tbl[4], p[i].tbl[8])
+                   || p[i].tmp[k] != mtgp_lin16(k, p[i].tmp[1], p[i].tmp[2], p[i].tmp[4], p[i].tmp[8]))
+                    return ROCRAND_STATUS_INTERNAL_ERROR;
+        }
+        void* d = nullptr;
+        if(hipGetSymbolAddress(&d, HIP_SYMBOL(d_params)) != hipSuccess
+           || hipMemcpy(d, p, sizeof(mtgp_param) * MTGP_GENS, hipMemcpyHostToDevice) != hipSuccess)
+            return ROCRAND_STATUS_ALLOCATION_FAILED;
+        ready[dev] = static_cast<mtgp_param*>(d);
+    }
+    out = ready[dev];
+    return ROCRAND_STATUS_SUCCESS;
+}
+
 // mtgp32.hpp:308-617
 class mtgp32_generator final : public rocrand_generator_base_type
 {
@@ -267,45 +345,14 @@ public:
             m_states = nullptr;
             return ROCRAND_STATUS_ALLOCATION_FAILED;
         }
-        // rocrand_make_state_mtgp32 (rocrand_mtgp32.h:362-390) and
-        // rocrand_mtgp32_init_state (:130-145)
-        std::vector<mtgp_state> h(MTGP_GENS);
-        const mtgp_param*       p    = params();
-        const uint64_t          s64  = m_seed ^ (m_seed >> 32);
-        for(unsigned i = 0; i < MTGP_GENS; i++)
-        {
-            // the kernel evaluates the recurrence table from its entries at 1, 2, 4 and 8 (the
-            // tempering table is linear too and checked with it), and its
-            // unmasked ring reads reach off + 255 + pos with off < 1024
-            if(p[i].pos == 0 || p[i].pos + MTGP_BLOCK > MTGP_N)
-                return ROCRAND_STATUS_INTERNAL_ERROR;
-            for(uint32_t k = 0; k < 16; k++)
-                if(p[i].tbl[k] != mtgp_lin16(k, p[i].tbl[1], p[i].tbl[2], p[i].tbl[4], p[i].tbl[8])
-                   || p[i].tmp[k] != mtgp_lin16(k, p[i].tmp[1], p[i].tmp[2], p[i].tmp[4], p[i].tmp[8]))
-                    return ROCRAND_STATUS_INTERNAL_ERROR;
-            mtgp_state& g = h[i];
-            memset(&g, 0, sizeof(g));
-            const uint32_t hidden = p[i].tbl[4] ^ (p[i].tbl[8] << 16);
-            uint32_t       tmp    = hidden;
-            tmp += tmp >> 16;
-            tmp += tmp >> 8;
-            memset(g.status, (int)(tmp & 0xff), sizeof(uint32_t) * MTGP_N);
-            g.status[0] = (uint32_t)s64 + i + 1;
-            g.status[1] = hidden;
-            for(unsigned k = 1; k < MTGP_N; k++)
-                g.status[k] ^= 1812433253u * (g.status[k - 1] ^ (g.status[k - 1] >> 30)) + k;
-            g.offset = 0;
-            g.pos    = p[i].pos;
-            g.sh1    = p[i].sh1;
-            g.sh2    = p[i].sh2;
-            g.mask   = p[0].mask;
-            memcpy(g.tbl, p[i].tbl, sizeof(g.tbl));
-            memcpy(g.tmp, p[i].tmp, sizeof(g.tmp));
-        }
-        if(hipMemcpyAsync(m_states, h.data(), sizeof(mtgp_state) * MTGP_GENS, hipMemcpyHostToDevice, stream)
-               != hipSuccess
-           || hipStreamSynchronize(stream) != hipSuccess)
-            return ROCRAND_STATUS_ALLOCATION_FAILED;
+        const mtgp_param* params = nullptr;
+        rocrand_status    st     = device_params(params);
+        if(st != ROCRAND_STATUS_SUCCESS)
+            return st;
+        hipLaunchKernelGGL(mtgp_seed_kernel, dim3(MTGP_GENS), dim3(64), 0, stream, static_cast<mtgp_state*>(m_states),
+                           params, (uint32_t)(m_seed ^ (m_seed >> 32)));
+        if(hipGetLastError() != hipSuccess)
+            return ROCRAND_STATUS_LAUNCH_FAILURE;
         m_initialized = true;
         return ROCRAND_STATUS_SUCCESS;
     }

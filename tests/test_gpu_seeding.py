@@ -82,3 +82,15 @@ def test_gf2_engine_states_on_other_grids(rng, blocks):
     finally:
         R.set_dynamic_grid(rng, 0, 0)
     assert np.array_equal(got.cpu().numpy(), _want(rng, S + 9, seed=77, offset=5 * S + 3, grid=(256, blocks)))
+
+
+def test_mtgp32_states_under_new_seeds():
+    """Every generator's first words under the seeds at the ends of the range."""
+    g, n = R.PRNG(R.MTGP32), 3 * 512 * 256
+    for seed in (0, 1, 0xFFFFFFFF, 0x8000000000000000, 0xFFFFFFFFFFFFFFFF, 0x0123456789ABCDEF):
+        print(f"case mtgp32 seed={seed:#x}", flush=True)
+        g.seed = seed
+        got = _words(g, n)
+        torch.cuda.synchronize()
+        assert np.array_equal(got.cpu().numpy(), _want(O.MTGP32, n, seed=seed))
+
