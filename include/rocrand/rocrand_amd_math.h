@@ -36,102 +36,140 @@ constexpr float  R_SQRT2          = 1.4142135f;
 // Float transcendentals evaluated in double and rounded once, written for the
 // arguments the transforms produce, with short fixed polynomials instead of the
 // general-purpose library routines:
-//   logf_tab (Box-Muller radius, u a positive normal float): u = 2^k z with
-//        z in [0.699, 1.398), ln u = k ln 2 - ln(1/c_i) + log1p(z/c_i - 1) over the 64-entry
-//        table of rocrand_amd_mathtab.h, |z/c_i - 1| < 2^-7, series to r^6 (relative error < 2^-44);
-//   sin/cos for x in [0, 8): reduction by pi/32 (two parts, fused), sin/cos(k pi/32) from
-//        rocrand_amd_mathtab.h and Taylor series to r^7 / r^6 on |r| <= pi/64;
-//   expf_acc: reduction by ln2/32 (two parts), 2^(j/32) from rocrand_amd_mathtab.h, Taylor series
-//        of exp(r) - 1 to r^5 on |r| <= ln2/64, scaling by 2^e in double.
-// A host C twin of these routines (exact division in place of the refined reciprocal)
-// rounds to the correctly rounded float result for every float in [2^-32, 1] but one
-// (logf_tab; that one lies within 2^-48 of a rounding boundary), every float in (0, 7]
-// (sin, cos) and every float in (-105, 90) but two (exp).
-// So each differs from the host libm's float result by at most the host's own error
-// (< 1 ulp).
-constexpr double RR_LN2     = 6.93147180559945286227e-01; // ln 2 rounded to double
+//   neg2log (Box-Muller radius, u a positive normal float in [2^-32, 1]): one table load
+//        indexed by u's exponent and 6 leading mantissa bits, |u a - 1| < 2^-7, series to
+//        r^4 (relative error < 2^-30) or r^6 (< 2^-44);
+//   sin/cos of a Box-Muller angle: table entry from the word that the angle came from, the
+//        difference exact in float, series to a^5 / a^6 on |a| < 0.0124 (errors < 2^-47);
+//   expf_acc: reduction by ln2/32, 2^(j/32) from rocrand_amd_mathtab.h, series of
+//        exp(r) - 1 to r^5 on |r| < 0.0109, scaling by 2^e in double.
+// The r^6 log, sin/cos and exp round to the correctly rounded float result but next to a
+// rounding boundary (relative distance 2^-44 or less), so each differs from the host
+// libm's float result by at most the host's own error (< 1 ulp).
 
-// ln u for a positive normal float u (the Box-Muller uniforms lie in [2^-32, 1]).
-__device__ __forceinline__ float logf_tab(float u)
+// Host and device compile the same code (the tests' host twins check it), with these in
+// place of the device's intrinsics; the hardware's reciprocal square roots are good to
+// 2^-24 (double) and one ulp (float).
+__host__ __device__ __forceinline__ uint32_t rr_float_bits(float x)
 {
-    ROCRAND_AMD_FP_EXACT
-    const uint32_t ix  = __float_as_uint(u);
-    const uint32_t tmp = ix - RR_LOGTAB_OFF;
-    const uint32_t i   = (tmp >> (23 - RR_LOGTAB_BITS)) & ((1u << RR_LOGTAB_BITS) - 1u);
-    const int      k   = (int)tmp >> 23;
-    const float    z   = __uint_as_float(ix - (tmp & 0xff800000u));
-    const double2  t   = rr_logtab[i];
-    const double   r   = __builtin_fma((double)z, t.x, -1.0);
-    const double   r2  = r * r;
-    double         p   = __builtin_fma(r, -1.0 / 6, 1.0 / 5);
-    p                  = __builtin_fma(p, r, -0.25);
-    p                  = __builtin_fma(p, r, 1.0 / 3);
-    p                  = __builtin_fma(p, r, -0.5);
-    const double hi    = __builtin_fma((double)k, RR_LN2, t.y);
-    return (float)(hi + __builtin_fma(p, r2, r));
+    uint32_t b;
+    __builtin_memcpy(&b, &x, sizeof(b));
+    return b;
+}
+__host__ __device__ __forceinline__ double rr_rsq(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rsq(x);
+#else
+    return (double)(float)(1.0 / __builtin_sqrt(x));
+#endif
+}
+__host__ __device__ __forceinline__ float rr_rsqf(float x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rsqf(x);
+#else
+    return (float)(1.0 / __builtin_sqrt((double)x));
+#endif
 }
 
-// sin and cos of x in [0, 8), rounded to float: x = q pi/32 + r (two-part reduction,
-// |r| <= pi/64), then the angle-addition formulas with sin/cos(k pi/32), k = q mod 64,
-// from rocrand_amd_mathtab.h and Taylor series of sin r (to r^7) and cos r (to r^6).  Where
-// sin x or cos x is near 0 the table entry is an exact 0 / +-1, so the sum does not cancel.
-__device__ __forceinline__ void sincosf_acc(float xf, float* s, float* c)
+// -2 ln u for a float u in [2^-32, 1]: the exponent and 6 leading mantissa bits index
+// rr_bm_logtab (a = 2^-k / c, b = 2 ln a), r = u a - 1 (one rounding-free fused operation)
+// and -2 ln u = b - 2 log1p(r), to r^4 or r^6.  u = 1 gives -0, as the reference's
+// -2.0f * logf(1.0f).
+template<int DEG>
+__host__ __device__ __forceinline__ double neg2log(float u)
 {
     ROCRAND_AMD_FP_EXACT
-    const double  x  = (double)xf;
-    const double  q  = __builtin_rint(x * RR_SC_INV_STEP);
-    const int     k  = (int)q & ((1 << RR_SCTAB_BITS) - 1);
-    double        r  = __builtin_fma(-q, RR_SC_STEP_HI, x);
-    r                = __builtin_fma(-q, RR_SC_STEP_LO, r);
-    const double2 t  = rr_sctab[k];
-    const double  r2 = r * r;
-    double        ps = __builtin_fma(r2, -1.0 / 5040, 1.0 / 120);
-    ps               = __builtin_fma(ps, r2, -1.0 / 6);
-    const double  sr = __builtin_fma(r * r2, ps, r);
-    double        pc = __builtin_fma(r2, -1.0 / 720, 1.0 / 24);
-    pc               = __builtin_fma(pc, r2, -0.5);
-    const double  cr = __builtin_fma(r2, pc, 1.0);
-    *s               = (float)__builtin_fma(t.x, cr, t.y * sr);
-    *c               = (float)__builtin_fma(t.y, cr, -(t.x * sr));
+    const uint32_t off = ((rr_float_bits(u) >> 17) << 4) - RR_BM_EMIN * 64u * 16u; // entry (exponent, i)
+    const double2  t   = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(rr_bm_logtab) + off);
+    const double   r   = __builtin_fma((double)u, t.x, -1.0);
+    double         p;
+    if constexpr(DEG == 4)
+        p = __builtin_fma(r, 0.5, -2.0 / 3);
+    else
+    {
+        p = __builtin_fma(r, 1.0 / 3, -2.0 / 5);
+        p = __builtin_fma(p, r, 0.5);
+        p = __builtin_fma(p, r, -2.0 / 3);
+    }
+    p = __builtin_fma(p, r, 1.0);
+    p = __builtin_fma(p, r, -2.0);
+    return __builtin_fma(p, r, t.y);
 }
 
-// sqrtf for 0 and positive normal floats: the hardware square root (within 1 ulp) and
-// the two fused-multiply-add checks of its neighbours that make it correctly rounded --
-// the same instructions as the compiler's sqrtf without its rescaling of tiny inputs
-// (below 2^-96) and of infinities, which the Box-Muller radius (0 or >= 2^-24) never is.
-__device__ __forceinline__ float sqrtf_radius(float x)
+// logf of u, correctly rounded (an exact scaling of neg2log's rounding).
+__host__ __device__ __forceinline__ float logf_unit(float u)
+{
+    return -0.5f * (float)neg2log<6>(u);
+}
+
+// sqrtf, correctly rounded, for 0 and floats from 2^-96 up: the hardware reciprocal square
+// root, then one step from the exact residual x - s^2 (equal to the correctly rounded root
+// for every float of [2^-30, 2^8), checked exhaustively on gfx950; the compiler's sqrtf
+// adds a rescaling of tiny inputs and takes twice as many instructions).
+__host__ __device__ __forceinline__ float sqrtf_unit(float x)
 {
     ROCRAND_AMD_FP_EXACT
-    const float s  = __builtin_amdgcn_sqrtf(x);
-    const float sm = __uint_as_float(__float_as_uint(s) - 1u);
-    const float sp = __uint_as_float(__float_as_uint(s) + 1u);
-    float       r  = __builtin_fmaf(-sm, s, x) <= 0.0f ? sm : s;
-    r              = __builtin_fmaf(-sp, s, x) > 0.0f ? sp : r;
-    return r;
+    const float y = rr_rsqf(__builtin_fmaxf(x, 0x1p-96f));
+    const float s = x * y;
+    const float e = __builtin_fmaf(-s, s, x);
+    return __builtin_fmaf(e, 0.5f * y, s);
 }
 
+// The transforms' tables, by default the constant arrays; a kernel may pass copies in LDS.
+// A gather of 64 lanes from 16-byte entries through the vector cache takes about 40 cycles
+// of the CU's one address path however few lines it touches, which bounds a transform that
+// makes four of them per lane; from LDS it takes about half and that path stays free.
+struct math_tables
+{
+    const double2* nsc  = rr_nsc_tab;
+    const double2* sc   = rr_bm_sctab;
+    const double*  ex   = rr_exptab;
+    const double*  plog = rr_plog_tab[0];
+    const double*  psc  = rr_psc_tab[0];
+};
 
+// sin and cos of a Box-Muller angle v, each rounded to float: qoff = 16 q selects q =
+// round(128 v / pi), which the callers take from the word the angle came from.
+__host__ __device__ __forceinline__ void sincosf_unit(float v, uint32_t qoff, float& s, float& c,
+                                                      const math_tables& tab = math_tables{})
+{
+    ROCRAND_AMD_FP_EXACT
+    const double2 t  = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(tab.sc) + qoff);
+    const double  a  = (double)__builtin_fmaf(-(float)qoff, RR_BM_ANGLE_STEP * 0.0625f, v);
+    const double  a2 = a * a;
+    const double  sa = __builtin_fma(a * a2, __builtin_fma(a2, 1.0 / 120, -1.0 / 6), a);
+    double        ca = __builtin_fma(a2, -1.0 / 720, 1.0 / 24);
+    ca               = __builtin_fma(a2, __builtin_fma(a2, ca, -0.5), 1.0);
+    s                = (float)__builtin_fma(t.x, ca, t.y * sa);
+    c                = (float)__builtin_fma(t.y, ca, -(t.x * sa));
+}
 
 // exp of a float, rounded to float: x = (32 e + j) ln2/32 + r, exp x = 2^e 2^(j/32) exp(r)
 // with the 2^(j/32) table of rocrand_amd_mathtab.h.  Arguments are clamped to [-110, 100]
-// first (the float result is then 0 or +inf already), which keeps |32 e + j| < 2^13.
-__device__ __forceinline__ float expf_acc(float xf)
+// first (the float result is then 0 or +inf already); a NaN passes through the clamp.
+__host__ __device__ __forceinline__ float expf_acc(float xf, const math_tables& tab = math_tables{})
 {
     ROCRAND_AMD_FP_EXACT
-    const double x  = (double)xf;
-    const double xc = x < -110.0 ? -110.0 : (x > 100.0 ? 100.0 : x);
-    const double kd = __builtin_rint(xc * RR_EXP_INV_STEP);
-    const int    k  = (int)kd;
-    double       r  = __builtin_fma(-kd, RR_EXP_STEP_HI, xc);
-    r               = __builtin_fma(-kd, RR_EXP_STEP_LO, r);
-    double p        = __builtin_fma(r, 1.0 / 120, 1.0 / 24);
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float xc = __builtin_elementwise_maximum(__builtin_elementwise_minimum(xf, 100.0f), -110.0f);
+#else
+    const float xc = xf < -110.0f ? -110.0f : (xf > 100.0f ? 100.0f : xf);
+#endif
+    const float  kf = __builtin_rintf(xc * (float)RR_EXP_INV_STEP);
+    const int    k  = (int)kf;
+    const double r  = __builtin_fma((double)kf, -(RR_EXP_STEP_HI + RR_EXP_STEP_LO), (double)xc);
+    double       p  = __builtin_fma(r, 1.0 / 120, 1.0 / 24);
     p               = __builtin_fma(p, r, 1.0 / 6);
     p               = __builtin_fma(p, r, 0.5);
     p               = __builtin_fma(p, r, 1.0);
-    p               = p * r;
-    const double t  = rr_exptab[k & ((1 << RR_EXPTAB_BITS) - 1)];
-    const float  y  = (float)__builtin_amdgcn_ldexp(__builtin_fma(t, p, t), k >> RR_EXPTAB_BITS);
-    return xf != xf ? xf : y;
+    const double t  = tab.ex[k & ((1 << RR_EXPTAB_BITS) - 1)];
+#if defined(__HIP_DEVICE_COMPILE__)
+    return (float)__builtin_amdgcn_ldexp(__builtin_fma(t * r, p, t), k >> RR_EXPTAB_BITS);
+#else
+    return (float)__builtin_ldexp(__builtin_fma(t * r, p, t), k >> RR_EXPTAB_BITS);
+#endif
 }
 
 // ---------------------------------------------------------------- double functions
@@ -365,45 +403,40 @@ __device__ __forceinline__ double mrg_f64(uint32_t v)
 
 // The Box-Muller pair sin(v) sqrt(-2 ln u), cos(v) sqrt(-2 ln u) for a float u in
 // [2^-32, 1] and a float angle v in (0, 2 pi], evaluated in double and rounded to float
-// once.  qoff = 16 q selects the angle table entry for q = round(128 v / pi), which the
+// once.  qoff = 16 q selects the angle table entry for q = round(256 v / pi), which the
 // callers take from the word the angle came from (integer operations).
-//   -2 ln u: u's exponent and 6 leading mantissa bits index rr_bm_logtab (a = 2^-k / c,
-//     b = 2 ln a), r = u a - 1 (|r| < 2^-7) and -2 ln u = b + r (-2 + r (1 + r (-2/3 + r/2)))
-//     (log1p to r^4, relative error below 2^-35; u = 1 gives b = -0 and r = 0, so -0 as the
-//     reference's -2.0f * logf(1.0f));
-//   sqrt: the hardware double reciprocal square root (relative error below 2^-22) and one
-//     coupled Newton step (error below 2^-42); the radius keeps the sign of a zero;
-//   sin/cos: v = q P + a with P = pi/128 to 15 bits, a = v - q P exact in float
-//     (|a| < 0.0124), sin a to a^3 and cos a to a^4 (relative errors below 2^-32 and 2^-44),
-//     then the angle-addition formulas with sin(q P), cos(q P) from rr_bm_sctab.
-// The pair before its rounding is within 2^-30 of exact, so each output is within 0.51
+//   x = -2 ln u: neg2log<4>;
+//   angle: v = q P + a with P = pi/256 to 15 bits, a = v - q P exact in float (|a| < 0.0063),
+//     and sin v = cos a (S + C tan a), cos v = cos a (C - S tan a) with S, C = sin, cos of
+//     q P from rr_nsc_tab (halved) and tan a = a + g a^3 (g the best for that range, a little
+//     over 1/3: relative error 2^-34);
+//   radius times cos a: with y the hardware's reciprocal square root of x and t = x y, one
+//     Newton step gives 2 sqrt(x) = t (3 - t y) to 2^-46, and as 3 - t y is 2 to 2^-23,
+//     2 sqrt(x) cos a = t (3 - a^2 - t y) to 2^-33: the cosine costs no product of its own.
+//     The doubling is the table's half; the radius keeps the sign of a zero.
+// The pair before its rounding is within 2^-30 of exact, so each output is within 0.505
 // ulp of the exact value, and within 2 ulp of the reference's float pipeline (logf, sqrtf,
-// sinf/cosf and the product: four roundings, rocrand_normal.h:51-66).  UNIT rounds
+// sinf/cosf and the product: four roundings, rocrand_normal.h:51-66).  About 34 VALU
+// operations a pair (38 with sin and cos as sums of products with sin a and cos a and a
+// separate radius; XORWOW normal f32, 2^27 values, with its table in LDS: 3.30 -> 3.87
+// TB/s).  UNIT rounds
 // sin(v) s + 0 instead of sin(v) s: the output of mean + 1 * x at mean +0 (a zero is +0).
 template<bool UNIT = false>
-__device__ __forceinline__ void box_muller_dd(float u, float v, uint32_t qoff, float& r0, float& r1)
+__host__ __device__ __forceinline__ void box_muller_dd(float u, float v, uint32_t qoff, float& r0, float& r1,
+                                                       const math_tables& tab = math_tables{})
 {
     ROCRAND_AMD_FP_EXACT
-    const uint32_t loff = (__float_as_uint(u) >> 13) & 0x1fff0u; // 16 * (exponent * 64 + i)
-    const double2  lt   = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(rr_bm_logtab)
-                                                         - RR_BM_EMIN * 64u * 16u + loff);
-    const double   r    = __builtin_fma((double)u, lt.x, -1.0);
-    double         p    = __builtin_fma(r, 0.5, -2.0 / 3);
-    p                   = __builtin_fma(p, r, 1.0);
-    p                   = __builtin_fma(p, r, -2.0);
-    const double   x    = __builtin_fma(p, r, lt.y);
-    const double   y    = __builtin_amdgcn_rsq(__builtin_fmax(x, 0x1p-126));
-    const double   t    = x * y;
-    const double   h    = __builtin_fma(-t, y, 1.0);
-    const double   s    = __builtin_fma(t * h, 0.5, t);
-
-    const double2 st = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(rr_bm_sctab) + qoff);
-    const double  a  = (double)__builtin_fmaf(-(float)qoff, RR_BM_ANGLE_STEP * 0.0625f, v);
-    const double  a2 = a * a;
-    const double  sa = a * __builtin_fma(a2, -1.0 / 6, 1.0);
-    const double  ca = __builtin_fma(a2, __builtin_fma(a2, 1.0 / 24, -0.5), 1.0);
-    const double  sn = __builtin_fma(st.x, ca, st.y * sa);
-    const double  cs = __builtin_fma(st.y, ca, -(st.x * sa));
+    const double  x  = neg2log<4>(u);
+    const double2 st = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(tab.nsc) + qoff);
+    const double  a  = (double)__builtin_fmaf(-(float)qoff, RR_NSC_STEP * 0.0625f, v);
+    const double  c3 = __builtin_fma(-a, a, 3.0);
+    constexpr double g = 1.0 / 3 + 4.3e-6;
+    const double  ta = a * __builtin_fma(c3, -g, 1.0 + 3.0 * g); // a (1 + g a^2)
+    const double  y  = rr_rsq(__builtin_fmax(x, 0x1p-126));
+    const double  t  = x * y;
+    const double  s  = t * __builtin_fma(-t, y, c3);
+    const double  sn = __builtin_fma(st.y, ta, st.x);
+    const double  cs = __builtin_fma(-st.x, ta, st.y);
     if constexpr(UNIT)
     {
         r0 = (float)__builtin_fma(sn, s, 0.0);
@@ -418,35 +451,38 @@ __device__ __forceinline__ void box_muller_dd(float u, float v, uint32_t qoff, f
 
 // rocrand_normal.h:51-66: u = 2^-32 + x 2^-32, angle 2^-32 2pi + y 2^-32 2pi (rounded as
 // the reference rounds them), then the pair above; the angle is about 2 pi (y + 1) 2^-32,
-// so q = round(y 2^-24).
+// so q = round(y 2^-23) (and for the 257-entry table of the stepwise pair, round(y 2^-24)).
 template<bool UNIT = false>
-__device__ __forceinline__ void box_muller(uint32_t x, uint32_t y, float& r0, float& r1)
+__device__ __forceinline__ void box_muller(uint32_t x, uint32_t y, float& r0, float& r1,
+                                           const math_tables& tab = math_tables{})
 {
     ROCRAND_AMD_FP_EXACT
     const float u = uniform_f32(x);
     const float v = R_2POW32_INV_2PI + (float)y * R_2POW32_INV_2PI;
-    box_muller_dd<UNIT>(u, v, ((y >> 20) + 8u) & ~15u, r0, r1);
+    box_muller_dd<UNIT>(u, v, ((y >> 19) + 8u) & ~15u, r0, r1, tab);
 }
 
 // The same pair through the reference's own steps -- logf, sqrtf, sinf/cosf, each rounded
 // to float (correctly) -- for the log-normal transforms: exp magnifies a one-ulp change
 // of the variate to several ulps of the output, and these steps reproduce the reference
 // host path's variate bit for bit wherever its libm rounds correctly.
-__device__ __forceinline__ void box_muller_uv_stepwise(float u, float v, float& r0, float& r1)
+__device__ __forceinline__ void box_muller_uv_stepwise(float u, float v, uint32_t qoff, float& r0, float& r1,
+                                                       const math_tables& tab)
 {
     ROCRAND_AMD_FP_EXACT
-    const float s = sqrtf_radius(-2.0f * logf_tab(u));
+    const float s = sqrtf_unit((float)neg2log<6>(u));
     float       sn, cs;
-    sincosf_acc(v, &sn, &cs);
+    sincosf_unit(v, qoff, sn, cs, tab);
     r0 = sn * s;
     r1 = cs * s;
 }
-__device__ __forceinline__ void box_muller_stepwise(uint32_t x, uint32_t y, float& r0, float& r1)
+__device__ __forceinline__ void box_muller_stepwise(uint32_t x, uint32_t y, float& r0, float& r1,
+                                                    const math_tables& tab = math_tables{})
 {
     ROCRAND_AMD_FP_EXACT
     const float u = uniform_f32(x);
     const float v = R_2POW32_INV_2PI + (float)y * R_2POW32_INV_2PI;
-    box_muller_uv_stepwise(u, v, r0, r1);
+    box_muller_uv_stepwise(u, v, ((y >> 20) + 8u) & ~15u, r0, r1, tab);
 }
 // rocrand_normal.h:76-96 (host branch: sin(w * pi), not sincospi).
 __device__ __forceinline__ void box_muller_double(uint32_t a, uint32_t b, uint32_t c, uint32_t d, double& r0,
@@ -464,33 +500,121 @@ __device__ __forceinline__ void box_muller_double(uint32_t a, uint32_t b, uint32
     r0 = sn * s;
     r1 = cs * s;
 }
+// The double Box-Muller pair evaluated as double-doubles and rounded once, for a double u
+// in [2^-53, 1] and a double angle t in (0, 2 pi + 2^-48]; qoff = 32 q selects the angle
+// table entry for q = round(128 t / pi), which the callers take from the angle's word.
+//   x = -2 ln u: u = 2^k m, a = a multiple of 2^-8 next to 1/m (rr_plog_tab), so r = m a - 1
+//     is exact (|r| < 2^-7.3), and x = (-2 k ln 2 + 2 ln a) - 2 r + r^2 (1 - 2/3 r + ...):
+//     the first two terms add exactly in their heads, the sums with 2 r and with the rest
+//     (to r^8, small enough to be a double) leave their rounding errors in the tail;
+//   sqrt: t1 = sqrt(x) to 2^-46 from the hardware's reciprocal square root and a step, and
+//     the exact residual x - t1^2 gives the tail;
+//   angle: a = t - q P is exact for P = pi/128 rounded to double; sin and cos of q P as
+//     double-doubles, the products with a and the sums carried with their errors.
+// Relative error below 2^-58 before the rounding: within 0.52 ulp of the exact value, where
+// the reference's steps (log, sqrt, sin/cos and product, rounded one by one) may be 1.8
+// ulp off, and within 2 ulp of those.  115 VALU instructions with its uniforms and the
+// affine step; taking those steps one by one, each correctly rounded, costs 243 (XORWOW
+// normal f64, 2^27 values: 2.10 -> 3.57 TB/s, MRG32k3a 2.07 -> 3.56, Philox 1.98 -> 3.14).
+__host__ __device__ __forceinline__ void box_muller_pair_double(double u, double t, uint32_t qoff, double& r0,
+                                                                double& r1, const math_tables& tab)
+{
+    ROCRAND_AMD_FP_EXACT
+    // x = xh + xl
+    const uint64_t ix  = rr_double_to_bits(u);
+    const uint32_t hw  = (uint32_t)(ix >> 32), tmp = hw - RR_DLOG_OFF;
+    const double   k   = (double)((int32_t)tmp >> 20);
+    const double   m   = rr_bits_to_double(((uint64_t)(hw - (tmp & 0xfff00000u)) << 32) | (uint32_t)ix);
+    const double*  lt  = reinterpret_cast<const double*>(reinterpret_cast<const char*>(tab.plog)
+                                                       + ((tmp >> 8) & 0xfe0u));
+    const double   r   = __builtin_fma(m, lt[0], -1.0);
+    double         p   = __builtin_fma(r, 1.0 / 4, -2.0 / 7);
+    p                  = __builtin_fma(p, r, 1.0 / 3);
+    p                  = __builtin_fma(p, r, -2.0 / 5);
+    p                  = __builtin_fma(p, r, 1.0 / 2);
+    p                  = __builtin_fma(p, r, -2.0 / 3);
+    p                  = __builtin_fma(p, r, 1.0);
+    const double s0    = __builtin_fma(k, RR_PLOG_M2LN2_HI, lt[1]);
+    const double sl    = __builtin_fma(k, RR_PLOG_M2LN2_LO, lt[2]);
+    const double x1    = __builtin_fma(-2.0, r, s0);
+    const double q     = __builtin_fma(r * r, p, sl);
+    const double xh    = x1 + q;
+    const double xl    = __builtin_fma(-2.0, r, -(x1 - s0)) + (q - (xh - x1));
+    // sqrt(x) = th + tl
+    const double y     = rr_rsq(__builtin_fmax(xh, 0x1p-126));
+    const double h     = 0.5 * y;
+    const double g     = xh * y;
+    const double th    = __builtin_fma(__builtin_fma(-g, g, xh), h, g);
+    const double tl    = (__builtin_fma(-th, th, xh) + xl) * h;
+    // a = t - q P; sin a = a + sa, cos a = 1 + ca
+    const double* T    = reinterpret_cast<const double*>(reinterpret_cast<const char*>(tab.psc) + qoff);
+    const double  S = T[0], Sl = T[1], C = T[2], Cl = T[3];
+    const double  a    = __builtin_fma((double)qoff, -RR_PSC_STEP / 32, t);
+    const double  a2   = a * a;
+    const double  sa   = a * a2 * __builtin_fma(a2, __builtin_fma(a2, -1.0 / 5040, 1.0 / 120), -1.0 / 6);
+    const double  ca   = a2 * __builtin_fma(a2, __builtin_fma(a2, -1.0 / 720, 1.0 / 24), -0.5);
+    // sin t = S cos a + C sin a = sn + se
+    const double  p1   = C * a;
+    const double  sn   = S + p1;
+    double        se   = p1 - (sn - S);
+    se                 = __builtin_fma(S, ca, se);
+    se                 = __builtin_fma(C, sa, se);
+    se                 = __builtin_fma(Cl, a, se + __builtin_fma(C, a, -p1) + Sl);
+    // cos t = C cos a - S sin a = cs + ce
+    const double  p2   = S * a;
+    const double  cs   = C - p2;
+    double        ce   = (C - cs) - p2;
+    ce                 = __builtin_fma(C, ca, ce);
+    ce                 = __builtin_fma(-S, sa, ce);
+    ce                 = __builtin_fma(-Sl, a, ce - __builtin_fma(S, a, -p2) + Cl);
+    // the products, rounded once
+    const double  q0   = sn * th, q1 = cs * th;
+    r0 = q0 + __builtin_fma(se, th, __builtin_fma(sn, tl, __builtin_fma(sn, th, -q0)));
+    r1 = q1 + __builtin_fma(ce, th, __builtin_fma(cs, tl, __builtin_fma(cs, th, -q1)));
+}
+// The pair of four words: u = (v1 + 1) 2^-53 and w = (v2 + 1) 2^-52 rounded to double, each
+// from its word's halves in two exact fused operations and one rounding (rocrand_normal.h:76-96);
+// the angle is about 2 pi v2 2^-53, and v2's high word is d >> 11.
+__host__ __device__ __forceinline__ void normal_pair_double(uint32_t a, uint32_t b, uint32_t c, uint32_t d, double& r0,
+                                                            double& r1, const math_tables& tab = math_tables{})
+{
+    ROCRAND_AMD_FP_EXACT
+    const double u = __builtin_fma((double)(b >> 11), 0x1p-21,
+                                   __builtin_fma((double)(a ^ (b << 21)), R_2POW53_INV_DBL, R_2POW53_INV_DBL));
+    const double w = __builtin_fma((double)(d >> 11), 0x1p-20,
+                                   __builtin_fma((double)(c ^ (d << 21)), 0x1p-52, 0x1p-52));
+    box_muller_pair_double(u, w * R_PI_DBL, (((d >> 11) + 4096u) >> 8) & ~31u, r0, r1, tab);
+}
 // rocrand_normal.h:108-135, host (float math) branch.
-__device__ __forceinline__ void box_muller_half(uint32_t x16, uint32_t y16, float& h0, float& h1)
+__device__ __forceinline__ void box_muller_half(uint32_t x16, uint32_t y16, float& h0, float& h1,
+                                                const math_tables& tab)
 {
     ROCRAND_AMD_FP_EXACT
     const float u = R_2POW16_INV + (float)(x16 & 0xffffu) * R_2POW16_INV;
     const float v = R_2POW16_INV_2PI + (float)(y16 & 0xffffu) * R_2POW16_INV_2PI;
-    const float s = sqrtf_radius(-2.0f * logf_tab(u));
-    float       sn, cs;
-    sincosf_acc(v, &sn, &cs);
-    h0 = __half2float(__float2half(sn * s));
-    h1 = __half2float(__float2half(cs * s));
+    float       r0, r1; // the angle is about 2 pi (y16 + 1) 2^-16
+    box_muller_uv_stepwise(u, v, (((y16 & 0xffffu) >> 4) + 8u) & ~15u, r0, r1, tab);
+    h0 = __half2float(__float2half(r0));
+    h1 = __half2float(__float2half(r1));
 }
 // rocrand_normal.h:138-154
 // The MRG outputs y in [1, m] scale by about 2^-32 (MRG32k3a) or 2^-31 (MRG31k3p), so
-// q = round(y 2^-24) or round(y 2^-23).
+// q = round(y 2^-23) or round(y 2^-22) (stepwise pair: round(y 2^-24) or round(y 2^-23)).
 template<int MRG, bool UNIT = false>
-__device__ __forceinline__ void mrg_box_muller(uint32_t x, uint32_t y, float& r0, float& r1)
+__device__ __forceinline__ void mrg_box_muller(uint32_t x, uint32_t y, float& r0, float& r1,
+                                               const math_tables& tab = math_tables{})
+{
+    ROCRAND_AMD_FP_EXACT
+    constexpr int SH = MRG == 32 ? 19 : 18;
+    box_muller_dd<UNIT>(mrg_f32<MRG>(x), mrg_f32<MRG>(y) * R_2PI, ((y >> SH) + 8u) & ~15u, r0, r1, tab);
+}
+template<int MRG>
+__device__ __forceinline__ void mrg_box_muller_stepwise(uint32_t x, uint32_t y, float& r0, float& r1,
+                                                        const math_tables& tab = math_tables{})
 {
     ROCRAND_AMD_FP_EXACT
     constexpr int SH = MRG == 32 ? 20 : 19;
-    box_muller_dd<UNIT>(mrg_f32<MRG>(x), mrg_f32<MRG>(y) * R_2PI, ((y >> SH) + 8u) & ~15u, r0, r1);
-}
-template<int MRG>
-__device__ __forceinline__ void mrg_box_muller_stepwise(uint32_t x, uint32_t y, float& r0, float& r1)
-{
-    ROCRAND_AMD_FP_EXACT
-    box_muller_uv_stepwise(mrg_f32<MRG>(x), mrg_f32<MRG>(y) * R_2PI, r0, r1);
+    box_muller_uv_stepwise(mrg_f32<MRG>(x), mrg_f32<MRG>(y) * R_2PI, ((y >> SH) + 8u) & ~15u, r0, r1, tab);
 }
 // rocrand_normal.h:156-172: float-precision uniforms widened to double.
 template<int MRG>
@@ -504,6 +628,16 @@ __device__ __forceinline__ void mrg_box_muller_double(uint32_t x, uint32_t y, do
     sincos_cr(v * R_PI_DBL, sn, cs);
     r0 = sn * s;
     r1 = cs * s;
+}
+// The pair of rocrand_normal.h:156-172 evaluated as double-doubles and rounded once.
+template<int MRG>
+__device__ __forceinline__ void mrg_normal_pair_double(uint32_t x, uint32_t y, double& r0, double& r1,
+                                                       const math_tables& tab)
+{
+    ROCRAND_AMD_FP_EXACT
+    constexpr int SH = MRG == 32 ? 19 : 18;
+    const double  v  = (double)mrg_f32<MRG>(y) * 2.0;
+    box_muller_pair_double((double)mrg_f32<MRG>(x), v * R_PI_DBL, ((y >> SH) + 16u) & ~31u, r0, r1, tab);
 }
 // rocrand_normal.h:199-221 roc_d_erfinv and :263-268 normal_distribution_double.
 __device__ __forceinline__ double roc_d_erfinv(double x)
@@ -526,23 +660,21 @@ __device__ __forceinline__ double normal_double_1(double p)
     return (double)R_SQRT2 * roc_d_erfinv(2.0 * p - 1.0);
 }
 
-// rocrand_normal.h:174-197 roc_f_erfinv, float arithmetic rounded step by step.
+// rocrand_normal.h:174-197 roc_f_erfinv, float arithmetic rounded step by step.  x is 0 or
+// the difference of two floats of [0, 1], so (1 - x)(1 + x) is 0 or in [2^-23, 1]; at 0
+// (the logarithm is -inf) the reference returns 0.  The roots' arguments are 0 or at least
+// ulp(4.33).
 __device__ __forceinline__ float roc_f_erfinv(float x)
 {
     ROCRAND_AMD_FP_EXACT
-    const float sgn = (x < 0.0f) ? -1.0f : 1.0f;
-    x               = (1.0f - x) * (1.0f + x);
-    // (1 - x)(1 + x) is a positive normal float or 0 here (|x| <= 1)
-    const float lnx = x > 0.0f ? logf_tab(x) : -__builtin_inff();
-    if(isnan(lnx))
-        return 1.0f;
-    if(isinf(lnx))
-        return 0.0f;
+    const float     z   = (1.0f - x) * (1.0f + x);
+    const float     lnx = logf_unit(z > 0.0f ? z : 1.0f);
     constexpr float c1  = 2.0f / (3.141592653f * 0.147f);
     constexpr float c2  = 1.0f / 0.147f;
     const float     tt1 = c1 + 0.5f * lnx;
     const float     tt2 = c2 * lnx;
-    return sgn * sqrtf(-tt1 + sqrtf(tt1 * tt1 - tt2));
+    const float     w   = sqrtf_unit(-tt1 + sqrtf_unit(tt1 * tt1 - tt2));
+    return z > 0.0f ? __builtin_copysignf(w, x) : 0.0f;
 }
 
 // Uniforms of a direction value (rocrand_uniform.h:63-116 on the 32- or 64-bit value).

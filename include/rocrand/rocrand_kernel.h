@@ -9,8 +9,9 @@
  * rocrand_log_normal*, rocrand_poisson* and rocrand_discrete*.  A state initialised with
  * (seed, subsequence, offset) produces the words of the reference state initialised the
  * same way; the engine arithmetic and the float transforms are the library's own
- * (rocrand_amd_engines.h, rocrand_amd_math.h), so a thread's normals equal the bulk
- * generator's for the same words.  Jump matrices: rocrand_amd_jumptables.h.
+ * (rocrand_amd_engines.h, rocrand_amd_math.h), so a thread's float normals equal the bulk
+ * generator's for the same words; its double normals take the reference's steps one by one
+ * (the log-normals share them), within 2 ulp of the bulk generator's.  Jump matrices: rocrand_amd_jumptables.h.
  *
  * Sobol32/64 and their scrambled forms take the caller's direction vectors and scramble
  * constants (rocrand_get_direction_vectors32/64, rocrand_get_scramble_constants32/64).

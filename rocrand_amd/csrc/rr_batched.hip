@@ -110,6 +110,9 @@ __global__ __launch_bounds__(256) void batch_counter_kernel(const counter_call* 
 {
     using namespace ctr_dev;
     const uint64_t* staged = nullptr;
+    math_tables     tab;
+    if constexpr(counter_stages<K, D>())
+        stage_tables<D>(tab);
     for(uint32_t ti = blockIdx.x; ti < ntiles; ti += gridDim.x)
     {
         const batch_tile tl = read_const(tiles, ti);
@@ -118,6 +121,7 @@ __global__ __launch_bounds__(256) void batch_counter_kernel(const counter_call* 
         counter_call c = dist_kind<D>::value == out_kind::poisson ? calls[tl.stream] : read_const(calls, tl.stream);
         const uint64_t rmask = (uint64_t)c.ref_stride - 1;
         stage_tile_table<D>(c.params, staged);
+        const kernel_params kp{c.params, tab};
         const size_t end = tl.first + tl.count;
         if(fast_ok<K>(c))
         {
@@ -134,21 +138,21 @@ __global__ __launch_bounds__(256) void batch_counter_kernel(const counter_call* 
                 const uint32_t q  = (nch + 3) / 4;
                 const uint32_t m0 = wave * q;
                 if(m0 < nch)
-                    fast_run<K, D, true>(c, vb0 + 64 * (int64_t)m0, std::min(q, nch - m0), lo, hi);
+                    fast_run<K, D, true>(c, kp, vb0 + 64 * (int64_t)m0, std::min(q, nch - m0), lo, hi);
             }
             else
             {
                 for(uint32_t m = wave; m < nch; m += 4)
-                    fast_run<K, D, false>(c, vb0 + 64 * (int64_t)m, 1, lo, hi);
+                    fast_run<K, D, false>(c, kp, vb0 + 64 * (int64_t)m, 1, lo, hi);
             }
         }
         else
         {
             for(size_t v = tl.first + threadIdx.x; v < end; v += 256)
-                generic_vec<K, D>(c, v, rmask);
+                generic_vec<K, D>(c, kp, v, rmask);
         }
         if(tl.first == 0 && threadIdx.x == 0)
-            head_tail<K, D>(c, rmask);
+            head_tail<K, D>(c, kp, rmask);
     }
 }
 
@@ -165,11 +169,14 @@ __global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* call
     constexpr int OUT   = D::out_w;
     constexpr int BYTES = OUT * (int)sizeof(out_t);
     const uint64_t* staged = nullptr;
+    math_tables     tab;
+    stage_tables<D>(tab);
     for(uint32_t ti = blockIdx.x; ti < ntiles; ti += gridDim.x)
     {
         const batch_tile tl = read_const(tiles, ti);
         inter_call       c  = read_const(calls, tl.stream);
         stage_tile_table<D>(c.params, staged);
+        const kernel_params kp{c.params, tab};
         // The tile's engines start `lead` lanes into the block (the stream's first tile
         // only), so that a wavefront's stores start on a 128-byte line of the output.
         const uint32_t lead = (uint32_t)((tl.first + c.shift) & 255u);
@@ -211,7 +218,7 @@ __global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* call
 #pragma unroll
             for(int i = 0; i < IN; i++)
                 in[i] = g.next();
-            D::apply(in, o, c.params);
+            D::apply(in, o, kp);
             store_uniform_base<BYTES>(base, off, lim, o);
         }
         for(; index < c.vec_n; index += S, base += (size_t)S * BYTES)
@@ -219,7 +226,7 @@ __global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* call
 #pragma unroll
             for(int i = 0; i < IN; i++)
                 in[i] = g.next();
-            D::apply(in, o, c.params);
+            D::apply(in, o, kp);
             store_uniform_base<BYTES>(base, off, lim, o);
         }
         // the engine that would produce vec index vec_n writes the head, then the tail
@@ -231,7 +238,7 @@ __global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* call
 #pragma unroll
                 for(int i = 0; i < IN; i++)
                     in[i] = g.next();
-                D::apply(in, o, c.params);
+                D::apply(in, o, kp);
                 for(uint32_t j = 0; j < (uint32_t)OUT; j++)
                     if(j < c.head)
                         data[j] = o[j];
@@ -241,7 +248,7 @@ __global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* call
 #pragma unroll
                 for(int i = 0; i < IN; i++)
                     in[i] = g.next();
-                D::apply(in, o, c.params);
+                D::apply(in, o, kp);
                 for(uint32_t j = 0; j < (uint32_t)OUT; j++)
                     if(j < c.tail)
                         data[c.n - c.tail + j] = o[j];

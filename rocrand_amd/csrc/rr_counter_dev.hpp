@@ -108,11 +108,12 @@ __device__ __forceinline__ void store_vec(void* dst, const uint32_t* u)
     }
 }
 
-// Head and tail of a call (at most FULL-1 outputs each), written by one thread.
+// Head and tail of a call (at most FULL-1 outputs each), written by one thread.  `kp` =
+// the call's parameters with the kernel's tables, here and below.
 // stride_mask = c.ref_stride - 1 (the stride is a power of two), passed by the caller: a
 // read of the field here keeps the batched kernels' per-tile copy of the call in scratch.
 template<ctr_kind K, class D>
-__device__ void head_tail(const counter_call& c, uint64_t stride_mask)
+__device__ void head_tail(const counter_call& c, const kernel_params& kp, uint64_t stride_mask)
 {
     using T                    = ctr_traits<K>;
     using W                    = typename T::word;
@@ -136,7 +137,8 @@ __device__ void head_tail(const counter_call& c, uint64_t stride_mask)
 #pragma unroll
                 for(int i = 0; i < IN; i++)
                     in[i] = r.next(c.key);
-                D::apply(in, tmp, c.params);
+                D::apply(in, tmp, kp);
+#pragma unroll
                 for(int o = 0; o < OUT; o++)
                     if((uint32_t)(s * OUT + o) < c.head)
                         data[s * OUT + o] = tmp[o];
@@ -155,7 +157,8 @@ __device__ void head_tail(const counter_call& c, uint64_t stride_mask)
 #pragma unroll
                 for(int i = 0; i < IN; i++)
                     in[i] = r.next(c.key);
-                D::apply(in, tmp, c.params);
+                D::apply(in, tmp, kp);
+#pragma unroll
                 for(int o = 0; o < OUT; o++)
                     if((uint32_t)(s * OUT + o) < c.tail)
                         data[c.n - c.tail + s * OUT + o] = tmp[o];
@@ -168,7 +171,7 @@ __device__ void head_tail(const counter_call& c, uint64_t stride_mask)
 
 // One vec of a call, any position (two engine blocks when the stream starts mid-block).
 template<ctr_kind K, class D>
-__device__ __forceinline__ void generic_vec(const counter_call& c, size_t v, uint64_t stride_mask)
+__device__ __forceinline__ void generic_vec(const counter_call& c, const kernel_params& kp, size_t v, uint64_t stride_mask)
 {
     using T                    = ctr_traits<K>;
     using W                    = typename T::word;
@@ -208,7 +211,7 @@ __device__ __forceinline__ void generic_vec(const counter_call& c, size_t v, uin
     out_t o[FULL];
 #pragma unroll
     for(int s = 0; s < OPT; s++)
-        D::apply(words + s * IN, o + s * OUT, c.params);
+        D::apply(words + s * IN, o + s * OUT, kp);
     uint32_t u[BYTES / 4];
     __builtin_memcpy(u, o, BYTES);
     store_vec<BYTES>(vec_data + v * FULL, u);
@@ -228,7 +231,8 @@ __device__ __forceinline__ void generic_vec(const counter_call& c, size_t v, uin
 // chunk ahead (chunks + 1 block evaluations in all).  Every lane of the wavefront calls
 // this.
 template<ctr_kind K, class D, bool SUB>
-__device__ __forceinline__ void fast_run(const counter_call& c, int64_t vb, uint32_t chunks, int64_t lo, int64_t end)
+__device__ __forceinline__ void fast_run(const counter_call& c, const kernel_params& kp, int64_t vb, uint32_t chunks,
+                                         int64_t lo, int64_t end)
 {
     using T                = ctr_traits<K>;
     using W                = typename T::word;
@@ -261,22 +265,39 @@ __device__ __forceinline__ void fast_run(const counter_call& c, int64_t vb, uint
         T::block(ctr, c.key, w);
     };
 
-    W cur[DIM];
-    block_at(vb + lane, cur);
-    for(uint32_t k = 0; k < chunks; k++)
-    {
-        const int64_t base = vb + 64 * (int64_t)k;
-        if(base >= end)
-            break;
-        const int64_t v     = base + lane;
-        const bool    ahead = SUB || k + 1 < chunks;
-        W             nxt[DIM];
-        if(ahead)
-            block_at(v + 64, nxt);
-        W words[DIM];
-        if constexpr(SUB)
+    auto put = [&](int64_t v, const W* words) {
+        if(v >= lo && v < end)
         {
-            W nb[DIM];
+            out_t o[FULL];
+#pragma unroll
+            for(int s = 0; s < OPT; s++)
+                D::apply(words + s * IN, o + s * OUT, kp);
+            uint32_t u[BYTES / 4];
+            __builtin_memcpy(u, o, BYTES);
+            store_vec<BYTES>(vec_data + v * FULL, u);
+        }
+    };
+    W cur[DIM];
+    if constexpr(!SUB)
+    {
+        for(uint32_t k = 0; k < chunks; k++)
+        {
+            const int64_t v = vb + 64 * (int64_t)k + lane;
+            block_at(v, cur);
+            put(v, cur);
+        }
+    }
+    else
+    {
+        block_at(vb + lane, cur);
+        for(uint32_t k = 0; k < chunks; k++)
+        {
+            const int64_t base = vb + 64 * (int64_t)k;
+            if(base >= end)
+                break;
+            const int64_t v = base + lane;
+            W             nxt[DIM], nb[DIM], words[DIM];
+            block_at(v + 64, nxt);
 #pragma unroll
             for(int i = 0; i < DIM; i++)
             {
@@ -286,25 +307,7 @@ __device__ __forceinline__ void fast_run(const counter_call& c, int64_t vb, uint
                 nb[i] = (W)__builtin_amdgcn_update_dpp(first_next, (int)cur[i], 0x130, 0xf, 0xf, false);
             }
             interleave<W, DIM>(cur, nb, sub, words);
-        }
-        else
-        {
-#pragma unroll
-            for(int i = 0; i < DIM; i++)
-                words[i] = cur[i];
-        }
-        if(v >= lo && v < end)
-        {
-            out_t o[FULL];
-#pragma unroll
-            for(int s = 0; s < OPT; s++)
-                D::apply(words + s * IN, o + s * OUT, c.params);
-            uint32_t u[BYTES / 4];
-            __builtin_memcpy(u, o, BYTES);
-            store_vec<BYTES>(vec_data + v * FULL, u);
-        }
-        if(ahead)
-        {
+            put(v, words);
 #pragma unroll
             for(int i = 0; i < DIM; i++)
                 cur[i] = nxt[i];
@@ -318,7 +321,7 @@ __device__ __forceinline__ void fast_run(const counter_call& c, int64_t vb, uint
 // offset 2^20 + 7 measured 3.10 TB/s with it, 3.98 this way).  `first` is the wavefront's
 // first vec; every lane of the wavefront calls this.
 template<ctr_kind K, class D>
-__device__ __forceinline__ void fast_tile63(const counter_call& c, size_t first, size_t end)
+__device__ __forceinline__ void fast_tile63(const counter_call& c, const kernel_params& kp, size_t first, size_t end)
 {
     using T                = ctr_traits<K>;
     using W                = typename T::word;
@@ -362,7 +365,7 @@ __device__ __forceinline__ void fast_tile63(const counter_call& c, size_t first,
         out_t o[FULL];
 #pragma unroll
         for(int s = 0; s < OPT; s++)
-            D::apply(words + s * IN, o + s * OUT, c.params);
+            D::apply(words + s * IN, o + s * OUT, kp);
         uint32_t u[BYTES / 4];
         __builtin_memcpy(u, o, BYTES);
         store_vec<BYTES>(vec_data + v * FULL, u);
@@ -377,6 +380,15 @@ __device__ __forceinline__ void fast_tile63(const counter_call& c, size_t first,
         else
             finish(std::integral_constant<uint32_t, 3>{});
     }
+}
+
+// Whether a counter engine's kernels stage the transform's tables in LDS: Philox, whose
+// float transforms are bound by their gathers.  ThreeFry's rounds and the double pair leave
+// the kernel bound by arithmetic, and staging cost them 2% to 10%.
+template<ctr_kind K, class D>
+constexpr bool counter_stages()
+{
+    return K == ctr_kind::philox4x32 && dist_tables<D>::any && !dist_tables<D>::pair;
 }
 
 // Whether fast_run applies to a call.

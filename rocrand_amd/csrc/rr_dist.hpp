@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -91,6 +92,12 @@ struct dist_params
     int         unit; // mf is +0 and sf is 1 (the standard normal)
 };
 
+// The parameters as a kernel's transforms see them: with its tables (math_tables).
+struct kernel_params : dist_params
+{
+    math_tables tab;
+};
+
 // Family of the engine feeding the transform: generic 32-bit words, generic
 // 64-bit words (ThreeFry x64), or MRG (raw values in [1, m1], remapped).
 enum class word_family : int
@@ -134,6 +141,62 @@ struct dist_kind<dist<F, K, B>>
     static constexpr out_kind value = K;
 };
 
+// Which tables a transform gathers from (the log's, 33 KiB, stay in constant memory).
+template<class D>
+struct dist_tables
+{
+    static constexpr out_kind K   = dist_kind<D>::value;
+    static constexpr bool     one = std::is_same<D, dist<word_family::w32, K, true>>::value; // erfinv doubles
+    static constexpr bool nsc  = K == out_kind::normal_f32;
+    static constexpr bool sc   = K == out_kind::lognormal_f32 || K == out_kind::normal_f16 || K == out_kind::lognormal_f16;
+    static constexpr bool ex   = K == out_kind::lognormal_f32 || K == out_kind::lognormal_f16;
+    static constexpr bool pair = K == out_kind::normal_f64 && !one;
+    static constexpr bool any  = nsc || sc || ex || pair;
+};
+
+template<class T>
+__device__ __forceinline__ void copy_table(T* lds, const T* tab, uint32_t n)
+{
+    for(uint32_t i = threadIdx.x; i < n; i += blockDim.x)
+        lds[i] = tab[i];
+}
+
+// The block's copies of the tables that D gathers from, in LDS.  Every thread of the block
+// calls this before any leaves.
+template<class D>
+__device__ __forceinline__ void stage_tables(math_tables& t)
+{
+    using N = dist_tables<D>;
+    if constexpr(N::nsc)
+    {
+        __shared__ double2 s[513];
+        copy_table(s, rr_nsc_tab, 513);
+        t.nsc = s;
+    }
+    if constexpr(N::sc)
+    {
+        __shared__ double2 s[257];
+        copy_table(s, rr_bm_sctab, 257);
+        t.sc = s;
+    }
+    if constexpr(N::ex)
+    {
+        __shared__ double s[1 << RR_EXPTAB_BITS];
+        copy_table(s, rr_exptab, 1 << RR_EXPTAB_BITS);
+        t.ex = s;
+    }
+    if constexpr(N::pair)
+    {
+        __shared__ double2 s[2 * 257], l[2 * 128];
+        copy_table(s, reinterpret_cast<const double2*>(rr_psc_tab), 2 * 257);
+        copy_table(l, reinterpret_cast<const double2*>(rr_plog_tab), 2 * 128);
+        t.psc  = reinterpret_cast<const double*>(s);
+        t.plog = reinterpret_cast<const double*>(l);
+    }
+    if constexpr(N::any)
+        __syncthreads();
+}
+
 // Generic 32-bit engines (uniform.hpp:37-120, normal.hpp:45-108, log_normal.hpp:45-108).
 #define RR_DIST(F, K, IW, OW, T) \
     template<bool B>              \
@@ -142,7 +205,7 @@ struct dist_kind<dist<F, K, B>>
         static constexpr int in_w = IW, out_w = OW; \
         using out_t               = T;              \
         template<class W>                           \
-        __device__ __forceinline__ static void apply(const W* in, T* out, const dist_params& p)
+        __device__ __forceinline__ static void apply(const W* in, T* out, const kernel_params& p)
 
 RR_DIST(word_family::w32, out_kind::u32, 1, 1, uint32_t) { (void)p; out[0] = (uint32_t)in[0]; } };
 RR_DIST(word_family::w32, out_kind::u8, 1, 4, uint8_t)
@@ -172,21 +235,21 @@ RR_DIST(word_family::w32, out_kind::uniform_f16, 1, 2, __half)
 RR_DIST(word_family::w32, out_kind::normal_f32, 2, 2, float)
 {
     float r0, r1;
-    box_muller<B>((uint32_t)in[0], (uint32_t)in[1], r0, r1);
+    box_muller<B>((uint32_t)in[0], (uint32_t)in[1], r0, r1, p.tab);
     rr_affine<B>(r0, r1, out, p);
 } };
 RR_DIST(word_family::w32, out_kind::lognormal_f32, 2, 2, float)
 {
     float r0, r1;
-    box_muller_stepwise((uint32_t)in[0], (uint32_t)in[1], r0, r1);
-    out[0] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r0, p.sf)));
-    out[1] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r1, p.sf)));
+    box_muller_stepwise((uint32_t)in[0], (uint32_t)in[1], r0, r1, p.tab);
+    out[0] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r0, p.sf)), p.tab);
+    out[1] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r1, p.sf)), p.tab);
 } };
 RR_DIST(word_family::w32, out_kind::normal_f16, 1, 2, __half)
 {
     float h0, h1;
     const uint32_t v = (uint32_t)in[0];
-    box_muller_half(v, v >> 16, h0, h1);
+    box_muller_half(v, v >> 16, h0, h1, p.tab);
     const float m = __half2float(p.mh), s = __half2float(p.sh);
     out[0] = __float2half(__fadd_rn(m, __fmul_rn(s, h0)));
     out[1] = __float2half(__fadd_rn(m, __fmul_rn(s, h1)));
@@ -195,10 +258,10 @@ RR_DIST(word_family::w32, out_kind::lognormal_f16, 1, 2, __half)
 {
     float h0, h1;
     const uint32_t v = (uint32_t)in[0];
-    box_muller_half(v, v >> 16, h0, h1);
+    box_muller_half(v, v >> 16, h0, h1, p.tab);
     const float m = __half2float(p.mh), s = __half2float(p.sh);
-    out[0] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h0))));
-    out[1] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h1))));
+    out[0] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h0)), p.tab));
+    out[1] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h1)), p.tab));
 } };
 RR_DIST(word_family::w32, out_kind::poisson, 1, 1, uint32_t)
 {
@@ -221,10 +284,10 @@ struct dist<word_family::w32, out_kind::normal_f64, false>
     static constexpr int in_w = 4, out_w = 2;
     using out_t               = double;
     template<class W>
-    __device__ __forceinline__ static void apply(const W* in, double* out, const dist_params& p)
+    __device__ __forceinline__ static void apply(const W* in, double* out, const kernel_params& p)
     {
         double r0, r1;
-        box_muller_double((uint32_t)in[0], (uint32_t)in[1], (uint32_t)in[2], (uint32_t)in[3], r0, r1);
+        normal_pair_double((uint32_t)in[0], (uint32_t)in[1], (uint32_t)in[2], (uint32_t)in[3], r0, r1, p.tab);
         out[0] = __dadd_rn(p.md, __dmul_rn(r0, p.sd));
         out[1] = __dadd_rn(p.md, __dmul_rn(r1, p.sd));
     }
@@ -235,7 +298,7 @@ struct dist<word_family::w32, out_kind::lognormal_f64, false>
     static constexpr int in_w = 4, out_w = 2;
     using out_t               = double;
     template<class W>
-    __device__ __forceinline__ static void apply(const W* in, double* out, const dist_params& p)
+    __device__ __forceinline__ static void apply(const W* in, double* out, const kernel_params& p)
     {
         double r0, r1;
         box_muller_double((uint32_t)in[0], (uint32_t)in[1], (uint32_t)in[2], (uint32_t)in[3], r0, r1);
@@ -249,7 +312,7 @@ struct dist<word_family::w32, out_kind::normal_f64, true>
     static constexpr int in_w = 1, out_w = 1;
     using out_t               = double;
     template<class W>
-    __device__ __forceinline__ static void apply(const W* in, double* out, const dist_params& p)
+    __device__ __forceinline__ static void apply(const W* in, double* out, const kernel_params& p)
     {
         const double v = normal_double_1(__dadd_rn(R_2POW32_INV_DBL, __dmul_rn((double)(uint32_t)in[0], R_2POW32_INV_DBL)));
         out[0] = __dadd_rn(p.md, __dmul_rn(v, p.sd));
@@ -261,7 +324,7 @@ struct dist<word_family::w32, out_kind::lognormal_f64, true>
     static constexpr int in_w = 1, out_w = 1;
     using out_t               = double;
     template<class W>
-    __device__ __forceinline__ static void apply(const W* in, double* out, const dist_params& p)
+    __device__ __forceinline__ static void apply(const W* in, double* out, const kernel_params& p)
     {
         const double v = normal_double_1(__dadd_rn(R_2POW32_INV_DBL, __dmul_rn((double)(uint32_t)in[0], R_2POW32_INV_DBL)));
         out[0] = exp_cr(__dadd_rn(p.md, __dmul_rn(v, p.sd)));
@@ -303,22 +366,22 @@ RR_DIST(word_family::w64, out_kind::normal_f32, 1, 2, float)
 {
     float r0, r1;
     const uint64_t v = (uint64_t)in[0];
-    box_muller<B>((uint32_t)v, (uint32_t)(v >> 32), r0, r1);
+    box_muller<B>((uint32_t)v, (uint32_t)(v >> 32), r0, r1, p.tab);
     rr_affine<B>(r0, r1, out, p);
 } };
 RR_DIST(word_family::w64, out_kind::lognormal_f32, 1, 2, float)
 {
     float r0, r1;
     const uint64_t v = (uint64_t)in[0];
-    box_muller_stepwise((uint32_t)v, (uint32_t)(v >> 32), r0, r1);
-    out[0] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r0, p.sf)));
-    out[1] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r1, p.sf)));
+    box_muller_stepwise((uint32_t)v, (uint32_t)(v >> 32), r0, r1, p.tab);
+    out[0] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r0, p.sf)), p.tab);
+    out[1] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r1, p.sf)), p.tab);
 } };
 RR_DIST(word_family::w64, out_kind::normal_f64, 2, 2, double)
 {
     double r0, r1;
     const uint64_t a = (uint64_t)in[0], b = (uint64_t)in[1];
-    box_muller_double((uint32_t)a, (uint32_t)(a >> 32), (uint32_t)b, (uint32_t)(b >> 32), r0, r1);
+    normal_pair_double((uint32_t)a, (uint32_t)(a >> 32), (uint32_t)b, (uint32_t)(b >> 32), r0, r1, p.tab);
     out[0] = __dadd_rn(p.md, __dmul_rn(r0, p.sd));
     out[1] = __dadd_rn(p.md, __dmul_rn(r1, p.sd));
 } };
@@ -334,7 +397,7 @@ RR_DIST(word_family::w64, out_kind::normal_f16, 1, 2, __half)
 {
     float h0, h1;
     const uint64_t v = (uint64_t)in[0];
-    box_muller_half((uint32_t)v, (uint32_t)(v >> 32), h0, h1);
+    box_muller_half((uint32_t)v, (uint32_t)(v >> 32), h0, h1, p.tab);
     const float m = __half2float(p.mh), s = __half2float(p.sh);
     out[0] = __float2half(__fadd_rn(m, __fmul_rn(s, h0)));
     out[1] = __float2half(__fadd_rn(m, __fmul_rn(s, h1)));
@@ -343,10 +406,10 @@ RR_DIST(word_family::w64, out_kind::lognormal_f16, 1, 2, __half)
 {
     float h0, h1;
     const uint64_t v = (uint64_t)in[0];
-    box_muller_half((uint32_t)v, (uint32_t)(v >> 32), h0, h1);
+    box_muller_half((uint32_t)v, (uint32_t)(v >> 32), h0, h1, p.tab);
     const float m = __half2float(p.mh), s = __half2float(p.sh);
-    out[0] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h0))));
-    out[1] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h1))));
+    out[0] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h0)), p.tab));
+    out[1] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h1)), p.tab));
 } };
 RR_DIST(word_family::w64, out_kind::poisson, 1, 1, uint32_t)
 {
@@ -386,20 +449,20 @@ RR_DIST(word_family::w64, out_kind::poisson, 1, 1, uint32_t)
     RR_DIST(F, out_kind::normal_f32, 2, 2, float)                                                \
     {                                                                                            \
         float r0, r1;                                                                            \
-        mrg_box_muller<M, B>((uint32_t)in[0], (uint32_t)in[1], r0, r1);                          \
+        mrg_box_muller<M, B>((uint32_t)in[0], (uint32_t)in[1], r0, r1, p.tab);                          \
         rr_affine<B>(r0, r1, out, p);                                                            \
     } };                                                                                         \
     RR_DIST(F, out_kind::lognormal_f32, 2, 2, float)                                             \
     {                                                                                            \
         float r0, r1;                                                                            \
-        mrg_box_muller_stepwise<M>((uint32_t)in[0], (uint32_t)in[1], r0, r1);                             \
-        out[0] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r0, p.sf)));                                     \
-        out[1] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r1, p.sf)));                                     \
+        mrg_box_muller_stepwise<M>((uint32_t)in[0], (uint32_t)in[1], r0, r1, p.tab);                             \
+        out[0] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r0, p.sf)), p.tab);                                     \
+        out[1] = expf_acc(__fadd_rn(p.mf, __fmul_rn(r1, p.sf)), p.tab);                                     \
     } };                                                                                         \
     RR_DIST(F, out_kind::normal_f64, 2, 2, double)                                               \
     {                                                                                            \
         double r0, r1;                                                                           \
-        mrg_box_muller_double<M>((uint32_t)in[0], (uint32_t)in[1], r0, r1);                      \
+        mrg_normal_pair_double<M>((uint32_t)in[0], (uint32_t)in[1], r0, r1, p.tab);                     \
         out[0] = __dadd_rn(p.md, __dmul_rn(r0, p.sd));                                           \
         out[1] = __dadd_rn(p.md, __dmul_rn(r1, p.sd));                                           \
     } };                                                                                         \
@@ -414,7 +477,7 @@ RR_DIST(word_family::w64, out_kind::poisson, 1, 1, uint32_t)
     {                                                                                            \
         float h0, h1;                                                                            \
         const uint32_t v = mrg_uint<M>((uint32_t)in[0]);                                         \
-        box_muller_half(v, v >> 16, h0, h1);                                                     \
+        box_muller_half(v, v >> 16, h0, h1, p.tab);                                                     \
         const float m = __half2float(p.mh), s = __half2float(p.sh);                              \
         out[0] = __float2half(__fadd_rn(m, __fmul_rn(s, h0)));                                   \
         out[1] = __float2half(__fadd_rn(m, __fmul_rn(s, h1)));                                   \
@@ -423,10 +486,10 @@ RR_DIST(word_family::w64, out_kind::poisson, 1, 1, uint32_t)
     {                                                                                            \
         float h0, h1;                                                                            \
         const uint32_t v = mrg_uint<M>((uint32_t)in[0]);                                         \
-        box_muller_half(v, v >> 16, h0, h1);                                                     \
+        box_muller_half(v, v >> 16, h0, h1, p.tab);                                                     \
         const float m = __half2float(p.mh), s = __half2float(p.sh);                              \
-        out[0] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h0))));                             \
-        out[1] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h1))));                             \
+        out[0] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h0)), p.tab));                             \
+        out[1] = __float2half(expf_acc(__fadd_rn(m, __fmul_rn(s, h1)), p.tab));                             \
     } };                                                                                         \
     RR_DIST(F, out_kind::poisson, 1, 1, uint32_t)                                                \
     {                                                                                            \

@@ -164,16 +164,16 @@ __global__ __launch_bounds__(256) void gf2_init_kernel(uint32_t* states, const u
 // table above lambda 4000) and samples from there.  Every thread of the block calls this
 // before any thread leaves.
 template<class D>
-__device__ __forceinline__ void stage_poisson_table(interleaved_call& c)
+__device__ __forceinline__ void stage_poisson_table(kernel_params& p)
 {
     if constexpr(dist_kind<D>::value == out_kind::poisson)
     {
         extern __shared__ uint64_t lds_packed[];
-        const uint32_t             size = c.params.huge ? 0u : c.params.pt.size;
+        const uint32_t             size = p.huge ? 0u : p.pt.size;
         for(uint32_t i = threadIdx.x; i < size; i += blockDim.x)
-            lds_packed[i] = c.params.pt.packed[i];
+            lds_packed[i] = p.pt.packed[i];
         __syncthreads();
-        c.params.pt.packed = lds_packed;
+        p.pt.packed = lds_packed;
     }
 }
 
@@ -206,7 +206,9 @@ __global__ __launch_bounds__(256) void generate_kernel(interleaved_call c)
     constexpr int BYTES  = OUT * (int)sizeof(out_t);
     static_assert(BYTES == 4 || BYTES == 8 || BYTES == 16, "vec size");
 
-    stage_poisson_table<D>(c);
+    kernel_params kp{c.params, {}};
+    stage_poisson_table<D>(kp);
+    stage_tables<D>(kp.tab);
     const uint32_t S = c.S;
     // engines over lanes shifted by lane_shift, so that each wavefront's stores start on
     // a 128-byte line; the last lane_shift engines wrap round to block 0's first lanes
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(256) void generate_kernel(interleaved_call c)
 #pragma unroll
         for(int i = 0; i < IN; i++)
             in[i] = g.next();
-        D::apply(in, o, c.params);
+        D::apply(in, o, kp);
         store_uniform_base<BYTES>(base, off, lim, o);
     }
     for(; index < c.vec_n; index += S, base += (size_t)S * BYTES)
@@ -253,7 +255,7 @@ __global__ __launch_bounds__(256) void generate_kernel(interleaved_call c)
 #pragma unroll
         for(int i = 0; i < IN; i++)
             in[i] = g.next();
-        D::apply(in, o, c.params);
+        D::apply(in, o, kp);
         store_uniform_base<BYTES>(base, off, lim, o);
     }
     // The engine that would produce vec index vec_n also writes the head and
@@ -265,7 +267,7 @@ __global__ __launch_bounds__(256) void generate_kernel(interleaved_call c)
 #pragma unroll
             for(int i = 0; i < IN; i++)
                 in[i] = g.next();
-            D::apply(in, o, c.params);
+            D::apply(in, o, kp);
             for(uint32_t j = 0; j < (uint32_t)OUT; j++)
                 if(j < c.head)
                     data[j] = o[j];
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(256) void generate_kernel(interleaved_call c)
 #pragma unroll
             for(int i = 0; i < IN; i++)
                 in[i] = g.next();
-            D::apply(in, o, c.params);
+            D::apply(in, o, kp);
             for(uint32_t j = 0; j < (uint32_t)OUT; j++)
                 if(j < c.tail)
                     data[c.n - c.tail + j] = o[j];
@@ -313,7 +315,9 @@ __global__ __launch_bounds__(256) void generate_chunked_kernel(interleaved_call 
     const uint32_t     id  = lane_engine((blockIdx.x % BPC) * 256 + threadIdx.x, c.lane_shift, S);
     if(j >= J)
         return; // the whole block
-    stage_poisson_table<D>(c);
+    kernel_params kp{c.params, {}};
+    stage_poisson_table<D>(kp);
+    stage_tables<D>(kp.tab);
     // vec-steps of this engine: vec indices id, id + S, ... below vec_n
     const uint64_t steps  = id < c.vec_n ? (c.vec_n - id + S - 1) / S : 0;
     const uint64_t k0     = (uint64_t)j * C;
@@ -366,7 +370,7 @@ __global__ __launch_bounds__(256) void generate_chunked_kernel(interleaved_call 
 #pragma unroll
         for(int i = 0; i < IN; i++)
             in[i] = eng.next();
-        D::apply(in, o, c.params);
+        D::apply(in, o, kp);
         store_uniform_base<BYTES>(base, off, lim, o);
     }
     for(; k < cnt; k++, base += (size_t)S * BYTES)
@@ -374,7 +378,7 @@ __global__ __launch_bounds__(256) void generate_chunked_kernel(interleaved_call 
 #pragma unroll
         for(int i = 0; i < IN; i++)
             in[i] = eng.next();
-        D::apply(in, o, c.params);
+        D::apply(in, o, kp);
         store_uniform_base<BYTES>(base, off, lim, o);
     }
     if(!ending)
@@ -386,7 +390,7 @@ __global__ __launch_bounds__(256) void generate_chunked_kernel(interleaved_call 
 #pragma unroll
             for(int i = 0; i < IN; i++)
                 in[i] = eng.next();
-            D::apply(in, o, c.params);
+            D::apply(in, o, kp);
             for(uint32_t q = 0; q < (uint32_t)OUT; q++)
                 if(q < c.head)
                     data[q] = o[q];
@@ -396,7 +400,7 @@ __global__ __launch_bounds__(256) void generate_chunked_kernel(interleaved_call 
 #pragma unroll
             for(int i = 0; i < IN; i++)
                 in[i] = eng.next();
-            D::apply(in, o, c.params);
+            D::apply(in, o, kp);
             for(uint32_t q = 0; q < (uint32_t)OUT; q++)
                 if(q < c.tail)
                     data[c.n - c.tail + q] = o[q];

@@ -453,6 +453,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void m
     const unsigned special = mt_special[lane];
     alignas(16) out_t o[OUT];
     uint32_t     in[IN];
+    // the transforms' tables stay in constant memory: copies in LDS would leave room for
+    // three blocks per CU
+    const kernel_params kp{c.params, {}};
 
     // LDS indices of this thread's inputs, the same every round: local word
     // j = quarter + 4m (m < MW) reads eoff[m][i] for input i (held in registers: every
@@ -506,7 +509,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void m
 #pragma unroll
                     for(int i = 0; i < IN; i++)
                         in[i] = mt_temper(BATCH ? w[BATCH ? m : 0][i] : st[eoff[m][i]]);
-                    D::apply(in, o, c.params);
+                    D::apply(in, o, kp);
                     out_t* dst = rbase + (size_t)j * MT_STRIDE * OUT;
                     if constexpr(BYTES == 4)
                         *reinterpret_cast<uint32_t*>(dst) = *reinterpret_cast<const uint32_t*>(o);
@@ -527,7 +530,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void m
 #pragma unroll
             for(int i = 0; i < IN; i++)
                 in[i] = mt_temper(st[lds_at(mt_element(lane, special, j * IN + i), gl)]);
-            D::apply(in, o, c.params);
+            D::apply(in, o, kp);
             if(v < c.vec_n)
             {
                 out_t* dst = vec_data + v * OUT;

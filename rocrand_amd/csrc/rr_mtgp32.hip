@@ -156,6 +156,7 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
     const uint32_t pos = g->pos, sh1 = g->sh1, sh2 = g->sh2, mask = g->mask;
     if(t < 16)
         ttbl[t] = g->tmp[t];
+    kernel_params kp{c.params, {}};
     // Poisson: the block samples from its copy of the packed alias table in dynamic LDS
     // (a per-lane load from global memory would wait for the block's earlier stores)
     if constexpr(dist_kind<D>::value == out_kind::poisson)
@@ -164,10 +165,11 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
         const uint32_t             size = c.params.huge ? 0u : c.params.pt.size;
         for(uint32_t i = t; i < size; i += MTGP_BLOCK)
             lds_packed[i] = c.params.pt.packed[i];
-        c.params.pt.packed = lds_packed;
+        kp.pt.packed = lds_packed;
     }
     const uint32_t p1 = g->tbl[1], p2 = g->tbl[2], p4 = g->tbl[4], p8 = g->tbl[8];
     uint32_t       off = g->offset;
+    stage_tables<D>(kp.tab);
     __syncthreads();
 
     // one block-step: this thread's tempered word
@@ -209,7 +211,7 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
 #pragma unroll
         for(int i = 0; i < IN; i++)
             in[i] = step();
-        D::apply(in, o, c.params);
+        D::apply(in, o, kp);
         out_t* const dst = bptr + t * OUT;
         if constexpr(BYTES == 2)
             *reinterpret_cast<uint16_t*>(dst) = *reinterpret_cast<const uint16_t*>(o);
@@ -226,7 +228,7 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
 #pragma unroll
         for(int i = 0; i < IN; i++)
             in[i] = step();
-        D::apply(in, o, c.params);
+        D::apply(in, o, kp);
         if(index < c.vec_n)
             for(int j = 0; j < OUT; j++)
                 vec_data[index * OUT + j] = o[j];
@@ -237,7 +239,7 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
 #pragma unroll
         for(int i = 0; i < IN; i++)
             in[i] = step();
-        D::apply(in, o, c.params);
+        D::apply(in, o, kp);
         if(index == up)
             for(uint32_t j = 0; j < (uint32_t)OUT; j++)
                 if(j < c.head)

@@ -68,7 +68,7 @@ RR_SOB(out_kind::poisson, uint32_t)
 // sobol_*_distribution functors (uniform.hpp:351-442, normal.hpp:303-364,
 // log_normal.hpp:310-370, poisson.hpp:49-108 with the CDF method).
 template<out_kind K, class V>
-__device__ __forceinline__ typename sob_out<K>::type sob_apply(V x, const dist_params& p)
+__device__ __forceinline__ typename sob_out<K>::type sob_apply(V x, const kernel_params& p)
 {
     constexpr int B = sizeof(V) * 8;
     if constexpr(K == out_kind::u8)
@@ -92,12 +92,12 @@ __device__ __forceinline__ typename sob_out<K>::type sob_apply(V x, const dist_p
     else if constexpr(K == out_kind::normal_f16)
         return __float2half(__fadd_rn(__half2float(p.mh), __fmul_rn(sob_normal_f32(x), __half2float(p.sh))));
     else if constexpr(K == out_kind::lognormal_f32)
-        return expf_acc(__fadd_rn(p.mf, __fmul_rn(p.sf, sob_normal_f32(x))));
+        return expf_acc(__fadd_rn(p.mf, __fmul_rn(p.sf, sob_normal_f32(x))), p.tab);
     else if constexpr(K == out_kind::lognormal_f64)
         return exp_cr(__dadd_rn(p.md, __dmul_rn(p.sd, sob_normal_f64(x))));
     else if constexpr(K == out_kind::lognormal_f16)
         return __float2half(
-            expf_acc(__fadd_rn(__half2float(p.mh), __fmul_rn(__half2float(p.sh), sob_normal_f32(x)))));
+            expf_acc(__fadd_rn(__half2float(p.mh), __fmul_rn(__half2float(p.sh), sob_normal_f32(x))), p.tab));
     else
     {
         if(p.huge)
@@ -138,6 +138,15 @@ __global__ __launch_bounds__(256) void sobol_kernel(const sobol_call c)
                 lds_cdf[i] = c.params.pt.cdf[i];
             __syncthreads();
         }
+    }
+
+    kernel_params kp{c.params, {}};
+    if constexpr(K == out_kind::lognormal_f32 || K == out_kind::lognormal_f16)
+    {
+        __shared__ double ex[1 << RR_EXPTAB_BITS];
+        copy_table(ex, rr_exptab, 1 << RR_EXPTAB_BITS);
+        kp.tab.ex = ex;
+        __syncthreads();
     }
 
     // the wavefront index as a scalar, so that the group index below, its Gray-code
@@ -190,7 +199,7 @@ __global__ __launch_bounds__(256) void sobol_kernel(const sobol_call c)
     for(uint32_t m = 0; m < c.groups_per_wave; m++)
     {
         if(e >= 0 && (uint64_t)e < c.size)
-            store_one(out + e, sob_apply<K, V>((hi ? Wn : Wc) ^ L, c.params));
+            store_one(out + e, sob_apply<K, V>((hi ? Wn : Wc) ^ L, kp));
         e += 64;
         Wc = Wn;
         An = (An + 1u) & 0x03ffffffu;

@@ -1,6 +1,8 @@
 """Write include/rocrand/rocrand_amd_mathtab.h: the tables of the float-argument logarithm
 (Box-Muller radius), sine and cosine (Box-Muller angle) and exponential (log-normal
-outputs) evaluated in double.
+outputs) evaluated in double.  The first logarithm table and the first sine and cosine table
+serve arguments of any origin (tests/fastmath_twin.c); the transforms take the Box-Muller
+tables below, indexed by the bits their arguments came from.
 
 Logarithm, 64 entries: a positive normal float u is split as u = 2^k z with z in
 [0x3f330000, 0x3fb30000) (about [0.699, 1.398)), so that k = 0 around u = 1.  Entry i
@@ -35,7 +37,21 @@ Box-Muller sine and cosine, 257 entries: angles q P, q = 0..256, P = pi/128 roun
 float of 15 significant bits (q P and v - q P are exact in float for the angles v the
 transform sees, |v - q P| < 0.0124); entry q holds sin(q P), cos(q P) rounded to double.
 
-Double-precision logarithm, exponential and sine/cosine (the double transforms' steps,
+Float normals, sine and cosine, 513 entries: angles q P, q = 0..512, P = pi/256 rounded to 15
+significant bits (q P and v - q P exact in float as above, |v - q P| < 0.0063); entry q holds
+sin(q P)/2, cos(q P)/2 rounded to double (the radius comes out doubled).
+
+Double-precision Box-Muller pair (evaluated as double-doubles and rounded once):
+  log, 128 entries: x = 2^k m split as below; entry i holds a = a multiple of 2^-8 next to
+    1/c (exactly 1 for the interval that contains 1), so that m a - 1 is exact in double,
+    and 2 ln a as a head that is a multiple of 2^-42 (-0 where a = 1) and a tail; -2 ln 2 is
+    split the same way, so k (-2 ln 2) + 2 ln a adds exactly in the heads.
+  sin/cos, 257 entries: sin(q P) and cos(q P), q = 0..256, P = pi/128 rounded to double
+    (t - q P, |t - q P| < 2^-6, is a multiple of 2^-58 or of t's last bit where that is
+    smaller, so exact in double), as double-doubles; an entry next to a zero of the function
+    (q P is within 2^-51 of it) is all tail.
+
+Double-precision logarithm, exponential and sine/cosine (the double log-normals' steps,
 each evaluated in double-double and rounded once):
   log, 128 entries: x = 2^k m with the high word of m in [0x3fe6a09e, 0x3ff6a09e)
     (m in [sqrt(1/2), sqrt(2))); entry i covers the m whose high word minus 0x3fe6a09e has
@@ -135,6 +151,43 @@ def bm_sincos_entries():
     return [(float(mpmath.sin(q * p)), float(mpmath.cos(q * p))) for q in range(257)]
 
 
+def rounded_to(x, bits):
+    m, e = mpmath.frexp(x)
+    return mpmath.nint(m * 2**bits) * mpmath.power(2, e - bits)
+
+
+def normal_sincos_entries():
+    p = rounded_to(mpmath.pi / 256, 15)
+    return [(float(mpmath.sin(q * p) / 2), float(mpmath.cos(q * p) / 2)) for q in range(513)]
+
+
+def pair_log_split(x):
+    head = float(mpmath.nint(x * 2**42) / 2**42)
+    return head, float(x - mpmath.mpf(head))
+
+
+def pair_log_entries():
+    out = []
+    for i in range(128):
+        lo = mpmath.mpf(f64_from_high(DLOG_OFF + i * 0x2000))
+        hi = mpmath.mpf(f64_from_high(DLOG_OFF + (i + 1) * 0x2000))
+        if lo <= 1 < hi:
+            out.append((1.0, -0.0, 0.0))
+            continue
+        a = float(mpmath.nint(2 / (lo + hi) * 256) / 256)
+        out.append((a, *pair_log_split(2 * mpmath.log(mpmath.mpf(a)))))
+    return out
+
+
+def pair_sincos_entries():
+    p = mpmath.mpf(float(mpmath.pi / 128))
+
+    def tail_if_zero(x):
+        return (0.0, float(x)) if abs(x) < mpmath.power(2, -30) else dd(x)
+
+    return [(*tail_if_zero(mpmath.sin(q * p)), *tail_if_zero(mpmath.cos(q * p))) for q in range(257)]
+
+
 DLOG_OFF = 0x3FE6A09E
 
 
@@ -222,6 +275,12 @@ def main():
     bm_log_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}}}," for a, b in bm_log_entries())
     bm_sc_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}}}," for a, b in bm_sincos_entries())
     bm_p = bm_angle_step()
+    nsc_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}}}," for a, b in normal_sincos_entries())
+    nsc_p = float(rounded_to(mpmath.pi / 256, 15))
+    plog_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}, {c.hex()}, 0.0}}," for a, b, c in pair_log_entries())
+    psc_rows = "\n".join(f"    {{{', '.join(x.hex() for x in row)}}}," for row in pair_sincos_entries())
+    m2ln2 = pair_log_split(-2 * mpmath.log(2))
+    psc_p = float(mpmath.pi / 128)
     text = f"""// rocrand_amd_mathtab.h -- generated by rocrand_amd/data/make_math_tables.py; do not edit.
 // Tables of the double-evaluated float logarithm, sine/cosine and exponential (rocrand_amd_math.h).
 #pragma once
@@ -272,6 +331,24 @@ constexpr float RR_BM_ANGLE_STEP = {bm_p.hex()}f; // pi/128 to 15 bits
 // {{sin(q RR_BM_ANGLE_STEP), cos(q RR_BM_ANGLE_STEP)}}, q = 0..256
 RR_MATH_TABLE const double2 rr_bm_sctab[257] = {{
 {bm_sc_rows}
+}};
+
+// Float normals' angle: {{sin(q RR_NSC_STEP)/2, cos(q RR_NSC_STEP)/2}}, q = 0..512
+constexpr float RR_NSC_STEP = {nsc_p.hex()}f; // pi/256 to 15 bits
+RR_MATH_TABLE const double2 rr_nsc_tab[513] = {{
+{nsc_rows}
+}};
+
+// Double Box-Muller pair: {{a, 2 ln a (head, tail), 0}} for m in [sqrt(1/2), sqrt(2))
+RR_MATH_TABLE const double rr_plog_tab[128][4] = {{
+{plog_rows}
+}};
+constexpr double RR_PLOG_M2LN2_HI = {m2ln2[0].hex()}; // -2 ln 2
+constexpr double RR_PLOG_M2LN2_LO = {m2ln2[1].hex()};
+constexpr double RR_PSC_STEP = {psc_p.hex()}; // pi/128 rounded to double
+// {{sin(q RR_PSC_STEP), cos(q RR_PSC_STEP)}} (heads, tails), q = 0..256
+RR_MATH_TABLE const double rr_psc_tab[257][4] = {{
+{psc_rows}
 }};
 
 // Double-precision log: {{1/c, -ln(1/c) (head, tail), 0}} for m in [sqrt(1/2), sqrt(2))

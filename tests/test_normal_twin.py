@@ -1,0 +1,42 @@
+"""The normal and log-normal transforms' functions (include/rocrand/rocrand_amd_math.h)
+compiled for the host from the same source as the device (tests/normal_twin.cpp): the float
+log, sin, cos and exp are the correctly rounded ones (but next to a rounding boundary, at
+most one in a million here), the float pair is within 0.505 ulp and the double pair within
+0.52 ulp of exact, both within 2 ulp of the reference's steps over this libm."""
+import os
+import subprocess
+
+import pytest
+
+from test_dmath_twin import GCC_LIB, HERE, HIPCC, ROOT
+
+
+@pytest.fixture(scope="module")
+def rows(tmp_path_factory):
+    if not os.path.exists(HIPCC) or not os.path.exists(os.path.join(GCC_LIB, "include", "quadmath.h")):
+        pytest.skip("hipcc or libquadmath not available")
+    exe = tmp_path_factory.mktemp("ntwin") / "normal_twin"
+    subprocess.run([HIPCC, "-std=c++17", "-O2", "-ffp-contract=off", f"-I{os.path.join(ROOT, 'include')}",
+                    "-isystem", os.path.join(GCC_LIB, "include"), "-x", "hip", "--offload-arch=gfx950",
+                    os.path.join(HERE, "normal_twin.cpp"), "-o", str(exe), f"-L{GCC_LIB}", "-lquadmath"],
+                   check=True, capture_output=True)
+    out = subprocess.run([str(exe), "400000"], check=True, capture_output=True, text=True).stdout
+    return {ln.split()[0]: [int(v) for v in ln.split()[1:]] for ln in out.strip().splitlines()}
+
+
+@pytest.mark.parametrize("name", ["log", "sincos", "exp"])
+def test_float_functions_correctly_rounded(rows, name):
+    bad, total = rows[name]
+    assert total > 1_000_000
+    assert bad <= total * 1e-6
+    assert rows["special"] == [1, 1, 1, 1]
+
+
+@pytest.mark.parametrize("name,most", [("pair_f32", 505000), ("pair_f64", 520000)])
+def test_pairs(rows, name, most):
+    n, worst, beyond = rows[name]
+    assert n == 800000
+    assert worst <= most
+    assert beyond == 0
+    # the steps rounded one by one are further off: the comparison is not vacuous
+    assert rows["steps_f64"][0] >= 1_000_000
