@@ -9,10 +9,10 @@
 //   * MRG32k3a: a tile is up to 256 of a stream's engines.  A lane initialises its engine
 //     (the stream's seeded state advanced by offset / S + [engine < offset mod S] steps,
 //     jumped by the engine index in subsequences, as the per-call init kernel does) and
-//     then writes that engine's vecs v = id, id + S, ... (rr_interleaved_dev.hpp).  The
-//     tile's first engine state is computed on the host, so a lane applies one radix-table
-//     entry (its offset within the tile) rather than two.  Only the engines a stream uses
-//     are set up: min(S, vec_n + 1) instead of S per call.
+//     then writes that engine's vecs v = id, id + S, ... (rr_interleaved_dev.hpp).  A kernel
+//     of one thread per tile computes the tiles' first engine states beforehand, so a lane
+//     applies one radix-table entry (its offset within the tile) rather than two.  Only the
+//     engines a stream uses are set up: min(S, vec_n + 1) instead of S per call.
 // The plan records the group launches in a HIP graph once; a launch replays it.  The
 // grid size of each group is chosen by timing a few candidates on the first plan of a
 // given shape (kept in a process-wide cache).
@@ -45,15 +45,25 @@ struct batch_tile
     uint64_t first;
 };
 
+// Engines [first, first + count) of an MRG32k3a stream (first < S = 2^17, count <= 256), all
+// before or all past the wrap of (engine + start) mod S.
+struct inter_tile
+{
+    uint32_t stream; // index among all of the batch's MRG32k3a streams
+    uint32_t span;   // first | (count - 1) << 17
+    __host__ __device__ uint32_t first() const { return span & (INTERLEAVED_ENGINES - 1); }
+    __host__ __device__ uint32_t count() const { return (span >> 17) + 1; }
+};
+static_assert(INTERLEAVED_ENGINES == 1u << 17, "span layout");
+
 // One MRG32k3a stream: a fresh generator's single call.  Engine e's state is
-// A^(e * 2^76) A^(offset/S + [e < offset mod S]) (seeded state); the step part is the
-// same for every engine, so it is applied once on the host: base[0] = A^(offset/S) seeded,
-// base[1] = A base[0], and a lane only jumps by its subsequence.
+// A^(e * 2^76) A^(offset/S + [e < offset mod S]) (seeded state).
 struct inter_call
 {
-    uint32_t    base[2][6];
-    uint32_t    start;    // offset mod S
-    uint32_t    shift;    // vecs between the last 128-byte line boundary and vec 0
+    uint32_t    seeded[6];
+    uint32_t    start; // offset mod S
+    uint32_t    shift; // vecs between the last 128-byte line boundary and vec 0
+    uint64_t    steps; // offset / S
     void*       data;
     size_t      n, mis, vec_n;
     uint32_t    head, tail;
@@ -103,17 +113,17 @@ __device__ __forceinline__ T read_const(const T* p, size_t i)
     return r;
 }
 
-template<ctr_kind K, class D>
-__global__ __launch_bounds__(256) void batch_counter_kernel(const counter_call* calls,
-                                                            const batch_tile*   tiles,
-                                                            uint32_t            ntiles)
+// Tiles first, first + stride, ... below `end` of a Philox group, on one block.
+template<ctr_kind K, class D, bool STAGE>
+__device__ __forceinline__ void counter_tiles_run(const counter_call* calls, const batch_tile* tiles, uint32_t first,
+                                                  uint32_t last, uint32_t stride)
 {
     using namespace ctr_dev;
     const uint64_t* staged = nullptr;
     math_tables     tab;
-    if constexpr(counter_stages<K, D>())
+    if constexpr(STAGE)
         stage_tables<D>(tab);
-    for(uint32_t ti = blockIdx.x; ti < ntiles; ti += gridDim.x)
+    for(uint32_t ti = first; ti < last; ti += stride)
     {
         const batch_tile tl = read_const(tiles, ti);
         // (the Poisson kernel keeps a vector copy: with the descriptor in SGPRs its
@@ -156,12 +166,46 @@ __global__ __launch_bounds__(256) void batch_counter_kernel(const counter_call* 
     }
 }
 
-template<inter_kind K, class D>
-__global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* calls,
-                                                          const batch_tile* tiles,
-                                                          const uint32_t*   tile_states,
-                                                          uint32_t          ntiles,
-                                                          const device_tables t)
+template<ctr_kind K, class D>
+__global__ __launch_bounds__(256) void batch_counter_kernel(const counter_call* calls,
+                                                            const batch_tile*   tiles,
+                                                            uint32_t            ntiles)
+{
+    counter_tiles_run<K, D, ctr_dev::counter_stages<K, D>()>(calls, tiles, blockIdx.x, ntiles, gridDim.x);
+}
+
+// States of the tiles' first engines, one thread per tile of the batch: the seeded state
+// advanced by the stream's steps and jumped to engine (first + start) mod S.
+// Bound by one radix product per thread (9.5 us for a call's 5,000 tiles, 10.5 us for a
+// plan's 400,000); made on the host, they were most of the 80 ms that laying out 4096 streams
+// of 10^3 to 10^7 values took (14 ms now).
+__global__ __launch_bounds__(256) void batch_states_kernel(const inter_call* calls, const inter_tile* tiles,
+                                                           uint32_t ntiles, uint32_t* states, const device_tables t)
+{
+    using namespace inter_dev;
+    const uint32_t ti = blockIdx.x * 256u + threadIdx.x;
+    if(ti >= ntiles)
+        return;
+    const inter_tile           tl = tiles[ti];
+    const inter_call&          c  = calls[tl.stream];
+    const uint32_t             e  = tl.first() + c.start; // < 2 S
+    ieng<inter_kind::mrg32k3a> g;
+    g.set(c.seeded);
+    g.advance(t, c.steps + (e >= S ? 1u : 0u));
+    g.sub(t, e >= S ? e - S : e);
+#pragma unroll
+    for(int q = 0; q < 3; q++)
+    {
+        states[(size_t)ti * 6 + q]     = g.s.g1[q];
+        states[(size_t)ti * 6 + 3 + q] = g.s.g2[q];
+    }
+}
+
+// Tiles first, first + stride, ... below `end` of an MRG32k3a group, on one block.
+template<inter_kind K, class D, bool STAGE>
+__device__ __forceinline__ void inter_tiles_run(const inter_call* calls, const inter_tile* tiles,
+                                                const uint32_t* tile_states, uint32_t first, uint32_t last,
+                                                uint32_t stride, const device_tables& t)
 {
     using namespace inter_dev;
     using out_t         = typename D::out_t;
@@ -170,36 +214,29 @@ __global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* call
     constexpr int BYTES = OUT * (int)sizeof(out_t);
     const uint64_t* staged = nullptr;
     math_tables     tab;
-    stage_tables<D>(tab);
-    for(uint32_t ti = blockIdx.x; ti < ntiles; ti += gridDim.x)
+    if constexpr(STAGE)
+        stage_tables<D>(tab);
+    for(uint32_t ti = first; ti < last; ti += stride)
     {
-        const batch_tile tl = read_const(tiles, ti);
+        const inter_tile tl = read_const(tiles, ti);
         inter_call       c  = read_const(calls, tl.stream);
         stage_tile_table<D>(c.params, staged);
         const kernel_params kp{c.params, tab};
-        // The tile's engines start `lead` lanes into the block (the stream's first tile
-        // only), so that a wavefront's stores start on a 128-byte line of the output.
-        const uint32_t lead = (uint32_t)((tl.first + c.shift) & 255u);
-        if(threadIdx.x < lead || threadIdx.x - lead >= tl.count)
+        // The tile's engines start `lead` lanes into the block, so that a wavefront's stores
+        // start on a 128-byte line of the output.
+        const uint32_t lead = (tl.first() + c.shift) & 255u;
+        const uint32_t jl   = threadIdx.x - lead; // offset from the tile's first engine
+        if(threadIdx.x < lead || jl >= tl.count())
             continue;
-        const uint32_t id = (uint32_t)tl.first + threadIdx.x - lead;
-        // engine (id + start) mod S; the host gave the state of the tile's first engine
-        // (first + start, or first + start - S when the whole tile has wrapped), so a lane
-        // is X^j from it, j = its offset from that engine; in the tile that wraps, the
-        // wrapped lanes are X^(j - w) from base[1] (engine 0 with the extra step)
-        const uint32_t e0 = (uint32_t)tl.first + c.start;
-        const uint32_t jl = threadIdx.x - lead; // offset from the tile's first engine
-        const uint32_t w  = e0 < S ? S - e0 : 0u;
-        const bool     wr = e0 < S && jl >= w;
+        const uint32_t id = tl.first() + jl;
         uint32_t       w6[6];
 #pragma unroll
         for(int q = 0; q < 6; q++)
-            w6[q] = wr ? c.base[1][q] : read_const(tile_states, (size_t)ti * 6 + q);
+            w6[q] = read_const(tile_states, (size_t)ti * 6 + q);
         ieng<K> g;
         g.set(w6);
-        const uint32_t j = wr ? jl - w : jl;
-        if(j != 0u)
-            g.sub_entry(t, j);
+        if(jl != 0u)
+            g.sub_entry(t, jl);
         out_t* const data     = static_cast<out_t*>(c.data);
         out_t* const vec_data = data + c.mis;
         alignas(16) out_t o[OUT];
@@ -207,7 +244,7 @@ __global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* call
         // The tile's last engine takes the fewest vec-steps: that many run for every lane
         // under a scalar counter, storing from a tile-uniform base (buffer stores), and the
         // rest (at most one) per lane.
-        const uint32_t     id_last = (uint32_t)tl.first + tl.count - 1;
+        const uint32_t     id_last = tl.first() + tl.count() - 1;
         const uint32_t     ucnt    = id_last < c.vec_n ? (uint32_t)((c.vec_n - id_last + S - 1) / S) : 0u;
         const uint32_t     off     = id * (uint32_t)BYTES;
         constexpr uint32_t lim     = S * (uint32_t)BYTES;
@@ -257,20 +294,14 @@ __global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* call
     }
 }
 
-// The device's radix jump (rr_interleaved_dev.hpp mrg_sub_jump) on the host, MRG32k3a.
-void host_entry_apply(const uint32_t* entry, uint32_t x[6])
+template<inter_kind K, class D>
+__global__ __launch_bounds__(256) void batch_inter_kernel(const inter_call* calls,
+                                                          const inter_tile* tiles,
+                                                          const uint32_t*   tile_states,
+                                                          uint32_t          ntiles,
+                                                          const device_tables t)
 {
-    mat3_vec_fold<32, 209>(entry, x);
-    mat3_vec_fold<32, 22853>(entry + 9, x + 3);
-}
-void host_sub_jump(const uint32_t* radix, uint32_t e, uint32_t x[6])
-{
-    const uint32_t lo = e & (uint32_t)(MRG_RADIX_LO - 1);
-    const uint32_t hi = (e >> MRG_RADIX_LO_BITS) & (uint32_t)(MRG_RADIX_HI - 1);
-    if(lo != 0u)
-        host_entry_apply(radix + lo * MRG_RADIX_WORDS, x);
-    if(hi != 0u)
-        host_entry_apply(radix + (MRG_RADIX_LO + hi) * MRG_RADIX_WORDS, x);
+    inter_tiles_run<K, D, true>(calls, tiles, tile_states, blockIdx.x, ntiles, gridDim.x, t);
 }
 
 out_kind kind_of(rocrand_batch_kind k)
@@ -290,25 +321,26 @@ out_kind kind_of(rocrand_batch_kind k)
 
 // `lds` = bytes of dynamic LDS for the group's largest Poisson table (0 otherwise);
 // `tile_states` = MRG32k3a groups' per-tile engine states (6 words a tile), else null.
-using launcher = hipError_t (*)(const void* calls, const batch_tile* tiles, const uint32_t* tile_states,
+using launcher = hipError_t (*)(const void* calls, const void* tiles, const uint32_t* tile_states,
                                 uint32_t ntiles, uint32_t blocks, uint32_t lds, const device_tables& t,
                                 hipStream_t s);
 
 template<ctr_kind K, class D>
-hipError_t launch_counter_group(const void* calls, const batch_tile* tiles, const uint32_t*, uint32_t ntiles,
+hipError_t launch_counter_group(const void* calls, const void* tiles, const uint32_t*, uint32_t ntiles,
                                 uint32_t blocks, uint32_t lds, const device_tables&, hipStream_t s)
 {
     hipLaunchKernelGGL((batch_counter_kernel<K, D>), dim3(blocks), dim3(256), lds, s,
-                       static_cast<const counter_call*>(calls), tiles, ntiles);
+                       static_cast<const counter_call*>(calls), static_cast<const batch_tile*>(tiles), ntiles);
     return hipGetLastError();
 }
 
 template<inter_kind K, class D>
-hipError_t launch_inter_group(const void* calls, const batch_tile* tiles, const uint32_t* tile_states,
+hipError_t launch_inter_group(const void* calls, const void* tiles, const uint32_t* tile_states,
                               uint32_t ntiles, uint32_t blocks, uint32_t lds, const device_tables& t, hipStream_t s)
 {
     hipLaunchKernelGGL((batch_inter_kernel<K, D>), dim3(blocks), dim3(256), lds, s,
-                       static_cast<const inter_call*>(calls), tiles, tile_states, ntiles, t);
+                       static_cast<const inter_call*>(calls), static_cast<const inter_tile*>(tiles), tile_states,
+                       ntiles, t);
     return hipGetLastError();
 }
 
@@ -335,25 +367,73 @@ launcher pick_launcher(bool philox, out_kind k)
 #undef RR_PICK
 }
 
+// All groups of a small batch in one launch, one tile per block.
+struct small_batch
+{
+    struct part
+    {
+        const void*     calls;
+        const void*     tiles;
+        const uint32_t* states;
+        uint32_t        end;  // one past the part's last block
+        uint32_t        kind; // out_kind, + 32 for MRG32k3a
+    };
+    part     parts[16]; // at most 8 kinds of 2 engines
+    uint32_t n;
+};
+
+__global__ __launch_bounds__(256) void batch_small_kernel(const small_batch b, const device_tables t)
+{
+    constexpr word_family W = word_family::w32, M = word_family::mrg32;
+    constexpr ctr_kind    P = ctr_kind::philox4x32;
+    constexpr inter_kind  R = inter_kind::mrg32k3a;
+    uint32_t i = 0, begin = 0;
+    while(i + 1 < b.n && blockIdx.x >= b.parts[i].end)
+        begin = b.parts[i++].end;
+    const small_batch::part& p  = b.parts[i];
+    const uint32_t           ti = blockIdx.x - begin;
+#define RR_PART(KIND)                                                                                            \
+    case (uint32_t)KIND:                                                                                         \
+        counter_tiles_run<P, dist<W, KIND>, false>(static_cast<const counter_call*>(p.calls),                    \
+                                                   static_cast<const batch_tile*>(p.tiles), ti, ti + 1, 1);      \
+        break;                                                                                                   \
+    case 32u + (uint32_t)KIND:                                                                                   \
+        inter_tiles_run<R, dist<M, KIND>, false>(static_cast<const inter_call*>(p.calls),                        \
+                                                 static_cast<const inter_tile*>(p.tiles), p.states, ti, ti + 1, 1, t); \
+        break;
+    switch(p.kind)
+    {
+        RR_PART(out_kind::u32)
+        RR_PART(out_kind::uniform_f32)
+        RR_PART(out_kind::uniform_f64)
+        RR_PART(out_kind::normal_f32)
+        RR_PART(out_kind::normal_f64)
+        RR_PART(out_kind::lognormal_f32)
+        RR_PART(out_kind::lognormal_f64)
+        RR_PART(out_kind::poisson)
+    }
+#undef RR_PART
+}
+
 struct group
 {
     bool                      philox;
     out_kind                  kind;
     launcher                  fn;
-    std::vector<counter_call> ccalls;
-    std::vector<inter_call>   icalls;
-    std::vector<batch_tile>   tiles;
-    std::vector<uint32_t>     tile_states; // MRG32k3a: first engine state of each tile
+    std::vector<counter_call> ccalls; // Philox
+    std::vector<batch_tile>   tiles;  // Philox
+    std::vector<inter_tile>   itiles; // MRG32k3a
     size_t                    bytes_out = 0;
     size_t                    calls_at  = 0; // offsets in the descriptor image
     size_t                    tiles_at  = 0;
     size_t                    states_at = 0;
     void*                     d_calls   = nullptr;
-    batch_tile*               d_tiles   = nullptr;
+    void*                     d_tiles   = nullptr;
     const uint32_t*           d_states  = nullptr;
     uint32_t                  blocks    = 2048;
     uint32_t                  tile_vecs = CTR_TILE_VECS; // Philox: vecs per tile
     uint32_t                  lds_bytes = 0; // largest Poisson table of the group, packed
+    uint32_t ntiles() const { return (uint32_t)(philox ? tiles.size() : itiles.size()); }
 };
 
 // Philox tiles of a group: each stream's vecs in runs of `tile` whose boundaries fall on
@@ -395,15 +475,20 @@ std::tuple<int, int, int> tune_key(const group& g)
 }
 
 // A batch on the host: groups, the distinct Poisson tables, and the layout of the one
-// descriptor image (tables, then each group's calls and tiles) that goes to the device.
+// descriptor image that goes to the device: tables, each Philox group's calls and tiles, the
+// MRG32k3a calls and tiles of all groups, and, made there, the tiles' states.
 struct batch_layout
 {
     std::vector<group>                     groups;
+    std::vector<inter_call>                icalls;
     std::vector<std::vector<double>>       prob;
     std::vector<std::vector<unsigned int>> alias;
     std::vector<std::vector<uint64_t>>     packed;
     std::vector<size_t>                    prob_at, alias_at, packed_at;
-    size_t                                 bytes = 0;
+    size_t                                 icalls_at = 0, itiles_at = 0, states_at = 0;
+    uint32_t                               nitiles = 0;
+    size_t                                 upload = 0; // bytes made on the host
+    size_t                                 bytes  = 0;
 
     static size_t align(size_t x) { return (x + 255) / 256 * 256; }
 
@@ -419,19 +504,38 @@ struct batch_layout
             packed_at.push_back(at);
             at = align(at + packed[i].size() * sizeof(uint64_t));
         }
+        icalls_at = at;
+        at        = align(at + icalls.size() * sizeof(inter_call));
+        itiles_at = at;
         for(auto& g : groups)
-        {
-            g.calls_at = at;
-            at = align(at + (g.philox ? g.ccalls.size() * sizeof(counter_call) : g.icalls.size() * sizeof(inter_call)));
-            g.tiles_at = at;
-            at         = align(at + g.tiles.size() * sizeof(batch_tile));
-            g.states_at = at;
-            at          = align(at + g.tile_states.size() * sizeof(uint32_t));
-        }
+            if(!g.philox)
+            {
+                g.calls_at = icalls_at;
+                g.tiles_at = at;
+                at += g.itiles.size() * sizeof(inter_tile);
+            }
+        nitiles = (uint32_t)((at - itiles_at) / sizeof(inter_tile));
+        at      = align(at);
+        for(auto& g : groups)
+            if(g.philox)
+            {
+                g.calls_at = at;
+                at         = align(at + g.ccalls.size() * sizeof(counter_call));
+                g.tiles_at = at;
+                at         = align(at + g.tiles.size() * sizeof(batch_tile));
+            }
+        upload    = at;
+        states_at = at;
+        for(auto& g : groups)
+            if(!g.philox)
+            {
+                g.states_at = at;
+                at += g.itiles.size() * 6 * sizeof(uint32_t);
+            }
         bytes = std::max<size_t>(at, 256);
     }
 
-    // Writes the image for device address `dev` into `host` (bytes long): Poisson table
+    // Writes the image for device address `dev` into `host` (`upload` bytes): Poisson table
     // references (held as table indices until now) become device pointers.
     void pack(char* host, char* dev)
     {
@@ -449,40 +553,93 @@ struct batch_layout
             prm.pt.alias   = reinterpret_cast<const unsigned int*>(dev + alias_at[t]);
             prm.pt.packed  = reinterpret_cast<const uint64_t*>(dev + packed_at[t]);
         };
+        for(auto& c : icalls)
+            fix(c.params);
+        if(!icalls.empty())
+            memcpy(host + icalls_at, icalls.data(), icalls.size() * sizeof(inter_call));
         for(auto& g : groups)
         {
+            g.d_calls = dev + g.calls_at;
+            g.d_tiles = dev + g.tiles_at;
             if(g.philox)
             {
                 for(auto& c : g.ccalls)
                     fix(c.params);
                 memcpy(host + g.calls_at, g.ccalls.data(), g.ccalls.size() * sizeof(counter_call));
+                memcpy(host + g.tiles_at, g.tiles.data(), g.tiles.size() * sizeof(batch_tile));
             }
             else
             {
-                for(auto& c : g.icalls)
-                    fix(c.params);
-                memcpy(host + g.calls_at, g.icalls.data(), g.icalls.size() * sizeof(inter_call));
+                g.d_states = reinterpret_cast<const uint32_t*>(dev + g.states_at);
+                if(!g.itiles.empty())
+                    memcpy(host + g.tiles_at, g.itiles.data(), g.itiles.size() * sizeof(inter_tile));
             }
-            memcpy(host + g.tiles_at, g.tiles.data(), g.tiles.size() * sizeof(batch_tile));
-            memcpy(host + g.states_at, g.tile_states.data(), g.tile_states.size() * sizeof(uint32_t));
-            g.d_calls  = dev + g.calls_at;
-            g.d_tiles  = reinterpret_cast<batch_tile*>(dev + g.tiles_at);
-            g.d_states = g.tile_states.empty() ? nullptr : reinterpret_cast<const uint32_t*>(dev + g.states_at);
         }
+    }
+
+    // The tiles' states, once the image is at `dev`.
+    hipError_t make_states(char* dev, const device_tables& t, hipStream_t s) const
+    {
+        if(nitiles == 0)
+            return hipSuccess;
+        hipLaunchKernelGGL(batch_states_kernel, dim3((nitiles + 255) / 256), dim3(256), 0, s,
+                           reinterpret_cast<const inter_call*>(dev + icalls_at),
+                           reinterpret_cast<const inter_tile*>(dev + itiles_at), nitiles,
+                           reinterpret_cast<uint32_t*>(dev + states_at), t);
+        return hipGetLastError();
     }
 };
 
-hipError_t run_groups(const std::vector<group>& groups, const device_tables& tables, hipStream_t s)
+// A batch of at most this many tiles goes in one launch (batch_small_kernel): its groups
+// would not fill the chip one by one, and six launches of 10 us each, in a row, are what
+// 256 streams of 10^2.5 to 10^5 values took.  They now take 9.5 us for the states and 33 us
+// for the one launch; the whole call went from 304 to 66 us, most of that host work.
+// Above, a group's own launch fills the chip and has its own tuned grid.
+constexpr uint32_t SMALL_TILES = 8192;
+
+uint64_t batch_tiles(const std::vector<group>& groups)
 {
+    uint64_t n = 0;
+    for(const auto& g : groups)
+        n += g.ntiles();
+    return n;
+}
+
+hipError_t run_small(const std::vector<group>& groups, const device_tables& tables, hipStream_t s, bool& done)
+{
+    if(batch_tiles(groups) > SMALL_TILES)
+        return hipSuccess;
+    small_batch b{};
+    uint32_t    total = 0, lds = 0;
     for(const auto& g : groups)
     {
-        if(g.tiles.empty())
+        if(g.ntiles() == 0)
             continue;
-        const uint32_t blocks = std::min<uint32_t>(g.blocks, (uint32_t)g.tiles.size());
-        hipError_t     e      = g.fn(g.d_calls, g.d_tiles, g.d_states, (uint32_t)g.tiles.size(), blocks, g.lds_bytes, tables, s);
-        if(e != hipSuccess)
-            return e;
+        total += g.ntiles();
+        lds            = std::max(lds, g.lds_bytes);
+        b.parts[b.n++] = {g.d_calls, g.d_tiles, g.d_states, total, (uint32_t)g.kind + (g.philox ? 0u : 32u)};
     }
+    done = true;
+    if(total == 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(batch_small_kernel, dim3(total), dim3(256), lds, s, b, tables);
+    return hipGetLastError();
+}
+
+hipError_t run_group(const group& g, const device_tables& tables, hipStream_t s)
+{
+    return g.fn(g.d_calls, g.d_tiles, g.d_states, g.ntiles(), std::min(g.blocks, g.ntiles()), g.lds_bytes, tables, s);
+}
+
+hipError_t run_groups(const std::vector<group>& groups, const device_tables& tables, hipStream_t s)
+{
+    bool       done = false;
+    hipError_t e    = run_small(groups, tables, s, done);
+    if(e != hipSuccess || done)
+        return e;
+    for(const auto& g : groups)
+        if(g.ntiles() != 0 && (e = run_group(g, tables, s)) != hipSuccess)
+            return e;
     return hipSuccess;
 }
 
@@ -522,15 +679,18 @@ struct fork_join
 hipError_t run_groups_forked(const std::vector<group>& groups, const device_tables& tables, hipStream_t cap,
                              const fork_join& fj)
 {
-    hipError_t e = hipEventRecord(fj.fork, cap);
+    bool       done = false;
+    hipError_t e    = run_small(groups, tables, cap, done);
+    if(e != hipSuccess || done)
+        return e;
+    e = hipEventRecord(fj.fork, cap);
     for(size_t i = 0; i < groups.size() && e == hipSuccess; i++)
     {
         const group& g = groups[i];
-        if(g.tiles.empty())
+        if(g.ntiles() == 0)
             continue;
-        const uint32_t blocks = std::min<uint32_t>(g.blocks, (uint32_t)g.tiles.size());
         if((e = hipStreamWaitEvent(fj.side[i], fj.fork, 0)) != hipSuccess
-           || (e = g.fn(g.d_calls, g.d_tiles, g.d_states, (uint32_t)g.tiles.size(), blocks, g.lds_bytes, tables, fj.side[i])) != hipSuccess
+           || (e = run_group(g, tables, fj.side[i])) != hipSuccess
            || (e = hipEventRecord(fj.done[i], fj.side[i])) != hipSuccess
            || (e = hipStreamWaitEvent(cap, fj.done[i], 0)) != hipSuccess)
             break;
@@ -598,20 +758,33 @@ public:
         pending_.push_back(std::make_pair(b, ev));
     }
 
+    // Takes back the blocks whose events have fired (a caller whose streams are drained and
+    // about to be destroyed: an event cannot be asked once its stream is gone).
+    void collect()
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        reclaim();
+    }
+
 private:
     void reclaim()
     {
         size_t keep = 0;
         for(size_t i = 0; i < pending_.size(); i++)
         {
-            if(hipEventQuery(pending_[i].second) == hipSuccess)
+            const hipError_t e = hipEventQuery(pending_[i].second);
+            if(e == hipSuccess)
             {
                 const block& b = pending_[i].first;
                 free_[std::make_pair(b.device, b.size)].push_back(b);
                 events_[b.device].push_back(pending_[i].second);
+                continue;
             }
-            else
-                pending_[keep++] = pending_[i];
+            // An event whose stream is gone or is being captured cannot be asked: its block
+            // stays out of use, and the error is not left for the next launch to report.
+            if(e != hipErrorNotReady)
+                (void)hipGetLastError();
+            pending_[keep++] = pending_[i];
         }
         pending_.resize(keep);
     }
@@ -689,8 +862,9 @@ struct rocrand_batch_plan_st
 namespace
 {
 
-// Validates the streams and lays out the batch on the host (no device calls).
-rocrand_status build(batch_layout& L, const rocrand_batch_stream* streams, size_t count)
+// Validates the streams and lays out the batch on the host (no device calls).  `fine` lets
+// a small batch take smaller Philox tiles.
+rocrand_status build(batch_layout& L, const rocrand_batch_stream* streams, size_t count, bool fine = true)
 {
     // Poisson alias tables, one per distinct lambda (poisson.hpp:110-161, discrete.hpp:189-265)
     std::map<double, alias_table>         tables;
@@ -756,7 +930,7 @@ rocrand_status build(batch_layout& L, const rocrand_batch_stream* streams, size_
         group&         g  = L.groups[git->second];
         if(k == out_kind::poisson && !prm.huge)
             g.lds_bytes = std::max<uint32_t>(g.lds_bytes, prm.pt.size * (uint32_t)sizeof(uint64_t));
-        const uint32_t si = (uint32_t)(philox ? g.ccalls.size() : g.icalls.size());
+        const uint32_t si = (uint32_t)(philox ? g.ccalls.size() : L.icalls.size());
         dist_shape     s{};
         if(philox)
         {
@@ -776,19 +950,8 @@ rocrand_status build(batch_layout& L, const rocrand_batch_stream* streams, size_
             rocrand_status st = interleaved_seed_state(b.rng_type, b.seed, k, seeded, ik, s);
             if(st != ROCRAND_STATUS_SUCCESS)
                 return st;
-            // base[0] = A^(offset / S) seeded, base[1] = A base[0] (host step tables A^(2^i))
-            const uint32_t* steps = host_mrg_table(32, 0);
-            uint64_t        v     = b.offset / INTERLEAVED_ENGINES;
-            for(int i = 0; v > 0; v >>= 1, i++)
-                if(v & 1)
-                {
-                    mat3_vec_fold<32, 209>(steps + (i * 2 + 0) * 9, seeded);
-                    mat3_vec_fold<32, 22853>(steps + (i * 2 + 1) * 9, seeded + 3);
-                }
-            std::copy(seeded, seeded + 6, c.base[0]);
-            mat3_vec_fold<32, 209>(steps + 0 * 9, seeded);
-            mat3_vec_fold<32, 22853>(steps + 1 * 9, seeded + 3);
-            std::copy(seeded, seeded + 6, c.base[1]);
+            std::copy(seeded, seeded + 6, c.seeded);
+            c.steps = b.offset / INTERLEAVED_ENGINES;
             const uintptr_t addr = reinterpret_cast<uintptr_t>(b.output);
             c.start    = (uint32_t)(b.offset % INTERLEAVED_ENGINES);
             c.data     = b.output;
@@ -803,61 +966,54 @@ rocrand_status build(batch_layout& L, const rocrand_batch_stream* streams, size_
                 const unsigned  vbytes = s.out_w * s.esz;
                 c.shift = 128u % vbytes == 0 ? (uint32_t)((vaddr / vbytes) % (128u / vbytes)) : 0u;
             }
-            g.icalls.push_back(c);
+            L.icalls.push_back(c);
             const bool   extra = s.out_w > 1 && (c.head > 0 || c.tail > 0);
             const size_t lanes = std::min<size_t>(INTERLEAVED_ENGINES, c.vec_n + (extra ? 1 : 0));
-            // Tile states: X^(first + start) base[0] while the tile's first engine has not
-            // wrapped, X^(first + start - S) base[1] after; consecutive tiles of a region
-            // differ by X^256 (radix entry 256).
-            const uint32_t* radix = host_mrg_radix(32);
-            uint32_t        x[6];
-            bool            have = false, wrapped = false;
             // Tiles on the grid shifted by c.shift: tile t covers engines [256 t - shift,
-            // 256 (t + 1) - shift) of the used ones, its first (active) engine `e`.
-            size_t e = 0, prev = 0;
-            for(size_t t = 0; e < lanes; t++)
+            // 256 (t + 1) - shift) of the used ones, cut where engine + start wraps.
+            const size_t wrap = c.start == 0 ? lanes : std::min<size_t>(lanes, INTERLEAVED_ENGINES - c.start);
+            for(size_t e = 0, t = 1; e < lanes;)
             {
-                const size_t end = std::min<size_t>((t + 1) * MRG_TILE - c.shift, lanes); // > e
-                g.tiles.push_back(batch_tile{si, (uint32_t)(end - e), e});
-                const uint64_t e0 = e + c.start;
-                if(!have || (!wrapped && e0 >= INTERLEAVED_ENGINES))
-                {
-                    wrapped = e0 >= INTERLEAVED_ENGINES;
-                    std::copy(c.base[wrapped ? 1 : 0], c.base[wrapped ? 1 : 0] + 6, x);
-                    host_sub_jump(radix, (uint32_t)(wrapped ? e0 - INTERLEAVED_ENGINES : e0), x);
-                    have = true;
-                }
-                else // e - prev engines further: 256, or 256 - shift after the first tile
-                    host_entry_apply(radix + (e - prev) * MRG_RADIX_WORDS, x);
-                g.tile_states.insert(g.tile_states.end(), x, x + 6);
-                prev = e;
-                e    = end;
+                const size_t grid = t * MRG_TILE - c.shift;
+                const size_t end  = std::min(e < wrap ? std::min(grid, wrap) : grid, lanes); // > e
+                g.itiles.push_back(inter_tile{si, (uint32_t)e | (uint32_t)(end - e - 1) << 17});
+                t += end == grid ? 1 : 0;
+                e = end;
             }
         }
         g.bytes_out += b.n * (size_t)s.esz;
     }
-    // Philox tiles once the group's size (and so its tuned tile size, if any) is known
+    // Schedules once the groups' sizes are known.  A batch for a single launch takes the
+    // smallest Philox tiles (256 vecs: one chunk per wavefront) that leave it half the
+    // launch's tiles, so that a block's serial work is short; any other the tuned ones.
+    auto philox_tiles = [&](uint32_t tile) {
+        size_t n = 0;
+        for(const auto& g : L.groups)
+            for(const auto& c : g.ccalls)
+                n += c.vec_n / tile + 1;
+        return n;
+    };
+    size_t inter = 0;
+    for(const auto& g : L.groups)
+        inter += g.itiles.size();
+    uint32_t small = 0;
+    if(fine && inter + philox_tiles(CTR_TILE_VECS) <= SMALL_TILES / 2)
+        for(small = 256; inter + philox_tiles(small) > SMALL_TILES / 2;)
+            small *= 2;
     for(auto& g : L.groups)
+    {
+        std::lock_guard<std::mutex> lock(g_tune_mtx);
+        auto                        it = g_tuned.find(tune_key(g));
+        if(it != g_tuned.end())
+        {
+            g.blocks    = it->second.blocks;
+            g.tile_vecs = it->second.tile_vecs;
+        }
+        if(small != 0)
+            g.tile_vecs = small;
         if(g.philox)
-        {
-            {
-                std::lock_guard<std::mutex> lock(g_tune_mtx);
-                auto                        it = g_tuned.find(tune_key(g));
-                if(it != g_tuned.end())
-                {
-                    g.blocks    = it->second.blocks;
-                    g.tile_vecs = it->second.tile_vecs;
-                }
-            }
             g.tiles = counter_tiles(g, g.tile_vecs);
-        }
-        else
-        {
-            std::lock_guard<std::mutex> lock(g_tune_mtx);
-            auto                        it = g_tuned.find(tune_key(g));
-            if(it != g_tuned.end())
-                g.blocks = it->second.blocks;
-        }
+    }
     L.place();
     return ROCRAND_STATUS_SUCCESS;
 }
@@ -902,7 +1058,7 @@ rocrand_status tune(rocrand_batch_plan_st& p, bool& relayout)
     relayout                            = false;
     for(auto& g : p.groups)
     {
-        if(g.tiles.empty())
+        if(g.ntiles() == 0)
             continue;
         const auto key = tune_key(g);
         {
@@ -924,8 +1080,8 @@ rocrand_status tune(rocrand_batch_plan_st& p, bool& relayout)
         for(size_t tc = 0; tc < ntile_cands; tc++)
         {
             const uint32_t    tile   = g.philox ? ctr_tiles[tc] : g.tile_vecs;
-            const batch_tile* tiles  = g.d_tiles;
-            uint32_t          ntiles = (uint32_t)g.tiles.size();
+            const void*       tiles  = g.d_tiles;
+            uint32_t          ntiles = g.ntiles();
             device_block      tmp;
             if(g.philox && tile != g.tile_vecs)
             {
@@ -934,7 +1090,7 @@ rocrand_status tune(rocrand_batch_plan_st& p, bool& relayout)
                     return ROCRAND_STATUS_ALLOCATION_FAILED;
                 if(hipMemcpy(tmp.p, tt.data(), tt.size() * sizeof(batch_tile), hipMemcpyHostToDevice) != hipSuccess)
                     return ROCRAND_STATUS_INTERNAL_ERROR;
-                tiles  = static_cast<const batch_tile*>(tmp.p);
+                tiles  = tmp.p;
                 ntiles = (uint32_t)tt.size();
             }
             for(uint32_t c : grids)
@@ -975,6 +1131,11 @@ rocrand_status tune(rocrand_batch_plan_st& p, bool& relayout)
 
 } // namespace
 
+namespace rr
+{
+void collect_batch_staging() { pool().collect(); }
+} // namespace rr
+
 extern "C" {
 
 rocrand_status ROCRANDAPI rocrand_batch_plan_create(rocrand_batch_plan*         plan,
@@ -991,28 +1152,30 @@ rocrand_status ROCRANDAPI rocrand_batch_plan_create(rocrand_batch_plan*         
         p         = new rocrand_batch_plan_st();
         p->stream = stream;
         // lay the batch out (with the cached schedules) and upload its descriptor image
+        bool small = false; // one launch, nothing to tune
         auto lay_out = [&]() {
             batch_layout   L;
             rocrand_status r = build(L, streams, count);
             if(r != ROCRAND_STATUS_SUCCESS)
                 return r;
-            std::vector<char> image(L.bytes);
+            std::vector<char> image(L.upload);
             if(hipMalloc(reinterpret_cast<void**>(&p->d_image), L.bytes) != hipSuccess)
             {
                 p->d_image = nullptr;
                 return ROCRAND_STATUS_ALLOCATION_FAILED;
             }
             L.pack(image.data(), p->d_image);
+            if(hipMemcpy(p->d_image, image.data(), L.upload, hipMemcpyHostToDevice) != hipSuccess
+               || L.make_states(p->d_image, p->tables, stream) != hipSuccess
+               || hipStreamSynchronize(stream) != hipSuccess)
+                return ROCRAND_STATUS_INTERNAL_ERROR;
             p->groups = std::move(L.groups);
-            return hipMemcpy(p->d_image, image.data(), L.bytes, hipMemcpyHostToDevice) == hipSuccess
-                       ? ROCRAND_STATUS_SUCCESS
-                       : ROCRAND_STATUS_INTERNAL_ERROR;
+            small     = batch_tiles(p->groups) <= SMALL_TILES;
+            return ROCRAND_STATUS_SUCCESS;
         };
-        rocrand_status st = lay_out();
-        if(st == ROCRAND_STATUS_SUCCESS && get_device_tables(p->tables) != hipSuccess)
-            st = ROCRAND_STATUS_INTERNAL_ERROR;
+        rocrand_status st = get_device_tables(p->tables) == hipSuccess ? lay_out() : ROCRAND_STATUS_INTERNAL_ERROR;
         bool relayout = false;
-        if(st == ROCRAND_STATUS_SUCCESS)
+        if(st == ROCRAND_STATUS_SUCCESS && !small)
             st = tune(*p, relayout);
         if(st == ROCRAND_STATUS_SUCCESS && relayout)
         {
@@ -1123,7 +1286,8 @@ rocrand_status ROCRANDAPI rocrand_generate_batched(const rocrand_batch_stream* s
         if(pool().acquire(device, L.bytes, blk, ev) != hipSuccess)
             return ROCRAND_STATUS_ALLOCATION_FAILED;
         L.pack(blk.host, blk.dev);
-        const bool ok = hipMemcpyAsync(blk.dev, blk.host, L.bytes, hipMemcpyHostToDevice, stream) == hipSuccess
+        const bool ok = hipMemcpyAsync(blk.dev, blk.host, L.upload, hipMemcpyHostToDevice, stream) == hipSuccess
+                        && L.make_states(blk.dev, tables, stream) == hipSuccess
                         && run_groups(L.groups, tables, stream) == hipSuccess;
         if(hipEventRecord(ev, stream) != hipSuccess)
         {
@@ -1160,6 +1324,12 @@ rocrand_status ROCRANDAPI rocrand_generate_batched_noalloc(const rocrand_batch_s
             return st;
         if(L.groups.empty())
             return ROCRAND_STATUS_SUCCESS;
+        if(L.bytes > NOALLOC_SCRATCH_BYTES) // a small batch's tiles may be larger
+        {
+            L = batch_layout{};
+            if((st = build(L, streams, count, false)) != ROCRAND_STATUS_SUCCESS)
+                return st;
+        }
         if(L.bytes > NOALLOC_SCRATCH_BYTES)
             return ROCRAND_STATUS_OUT_OF_RANGE; // descriptors beyond the fixed scratch array
         device_tables tables{};
@@ -1168,10 +1338,10 @@ rocrand_status ROCRANDAPI rocrand_generate_batched_noalloc(const rocrand_batch_s
             return ROCRAND_STATUS_INTERNAL_ERROR;
         // Descriptors are packed in host memory and copied into the scratch array on the
         // stream; a copy from pageable memory has read the host buffer when it returns.
-        std::vector<char> image(L.bytes);
+        std::vector<char> image(L.upload);
         L.pack(image.data(), dev);
-        if(hipMemcpyAsync(dev, image.data(), L.bytes, hipMemcpyHostToDevice, stream) != hipSuccess
-           || run_groups(L.groups, tables, stream) != hipSuccess)
+        if(hipMemcpyAsync(dev, image.data(), L.upload, hipMemcpyHostToDevice, stream) != hipSuccess
+           || L.make_states(dev, tables, stream) != hipSuccess || run_groups(L.groups, tables, stream) != hipSuccess)
             return ROCRAND_STATUS_LAUNCH_FAILURE;
     }
     catch(const std::bad_alloc&)

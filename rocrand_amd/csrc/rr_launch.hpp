@@ -135,11 +135,9 @@ struct device_tables
 // Returns the tables of the current device (built and uploaded on first use).
 hipError_t get_device_tables(device_tables& t);
 
-// Host copies of the same tables (used by host-side seeding helpers and tests).
-const uint32_t* host_mrg_table(int which_engine /*32 or 31*/, int sub /*0 step,1 subsequence*/);
-// Host copy of the subsequence radix table (MRG_RADIX_LO + MRG_RADIX_HI entries of
-// MRG_RADIX_WORDS words: X^e for e < 512, then X^(512 h) for h < 256, X = A^(2^76) or A^(2^72)).
-const uint32_t* host_mrg_radix(int which_engine /*32 or 31*/);
-const uint32_t* host_gf2_table(int xorwow /*1 xorwow, 0 lfsr*/, int seq);
+// Returns the descriptor blocks of finished rocrand_generate_batched calls to their pool.
+// A caller that made such calls on streams of its own calls this between draining and
+// destroying them.
+void collect_batch_staging();
 
 } // namespace rr

@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include "rr_arena.hpp"
+#include "rr_launch.hpp"
 
 #include <deque>
 #include <map>
@@ -228,6 +229,7 @@ struct rocrand_server_st
     {
         for(hipStream_t s : streams)
             (void)hipStreamSynchronize(s);
+        rr::collect_batch_staging();
         for(auto& kv : sessions)
         {
             if(kv.second.gen)

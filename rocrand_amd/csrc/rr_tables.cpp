@@ -259,26 +259,4 @@ hipError_t get_device_tables(device_tables& t)
     return hipSuccess;
 }
 
-const uint32_t* host_mrg_table(int which_engine, int sub)
-{
-    const host_tables& h = host();
-    if(which_engine == 32)
-        return sub ? h.mrg32_sub.data() : h.mrg32_step.data();
-    return sub ? h.mrg31_sub.data() : h.mrg31_step.data();
-}
-
-const uint32_t* host_mrg_radix(int which_engine)
-{
-    const host_tables& h = host();
-    return which_engine == 32 ? h.mrg32_subr.data() : h.mrg31_subr.data();
-}
-
-const uint32_t* host_gf2_table(int xorwow, int seq)
-{
-    const host_tables& h = host();
-    if(xorwow)
-        return seq ? h.xorwow_seq.data() : h.xorwow_jump.data();
-    return seq ? h.lfsr_seq.data() : h.lfsr_jump.data();
-}
-
 } // namespace rr

@@ -1,0 +1,87 @@
+"""Batches whose tiles fall on the edges of their paths, each stream against its plain call:
+MRG32k3a engines that wrap at, before and after a tile's end, misaligned outputs, one launch
+for a small batch and one per group for a larger one, streams without values."""
+import ctypes
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+from rocrand_amd import rocrand as R  # noqa: E402
+
+S = 131072
+DT = {R.BATCH_UINT: torch.int32, R.BATCH_UNIFORM_FLOAT: torch.float32, R.BATCH_UNIFORM_DOUBLE: torch.float64,
+      R.BATCH_NORMAL_FLOAT: torch.float32, R.BATCH_NORMAL_DOUBLE: torch.float64,
+      R.BATCH_LOG_NORMAL_FLOAT: torch.float32, R.BATCH_LOG_NORMAL_DOUBLE: torch.float64, R.BATCH_POISSON: torch.int32}
+
+
+def _plain(rng, kind, seed, offset, view, a, b):
+    g = R.PRNG(rng, seed=seed, offset=offset)
+    if kind == R.BATCH_UINT:
+        g.generate(view)
+    elif kind in (R.BATCH_UNIFORM_FLOAT, R.BATCH_UNIFORM_DOUBLE):
+        g.uniform(view)
+    elif kind in (R.BATCH_NORMAL_FLOAT, R.BATCH_NORMAL_DOUBLE):
+        g.normal(view, a, b)
+    elif kind in (R.BATCH_LOG_NORMAL_FLOAT, R.BATCH_LOG_NORMAL_DOUBLE):
+        g.lognormal(view, a, b)
+    else:
+        g.poisson(view, a)
+
+
+def _check(streams):
+    """streams: (rng, kind, seed, offset, n, shift); the one-shot call, the no-allocation call and a plan."""
+    want, got = [], []
+    for rng, kind, seed, offset, n, shift in streams:
+        for out in (want, got):
+            buf = torch.zeros(n + 16, dtype=DT[kind], device="cuda")
+            out.append(buf[shift:shift + n])
+    par = [(4.0, 0.0) if k == R.BATCH_POISSON else (0.5, 2.0) for _, k, *_ in streams]
+    for (rng, kind, seed, offset, n, _), v, (a, b) in zip(streams, want, par):
+        if n:
+            _plain(rng, kind, seed, offset, v, a, b)
+    arr = (R.BatchStream * len(streams))(*[
+        R.BatchStream(rng, kind, seed, offset, n, a, b, v.data_ptr())
+        for (rng, kind, seed, offset, n, _), v, (a, b) in zip(streams, got, par)])
+    L = R.load()
+    calls = [lambda: R.check_rocrand(L.rocrand_generate_batched(arr, len(arr), None)),
+             lambda: R.check_rocrand(L.rocrand_generate_batched_noalloc(arr, len(arr), None))]
+    plan = ctypes.c_void_p()
+    R.check_rocrand(L.rocrand_batch_plan_create(ctypes.byref(plan), arr, len(arr), None))
+    calls += [lambda: R.check_rocrand(L.rocrand_batch_plan_launch(plan))] * 3
+    for call in calls:
+        for v in got:
+            v.zero_()
+        call()
+        torch.cuda.synchronize()
+        for i, (g, w) in enumerate(zip(got, want)):
+            assert torch.equal(g.view(torch.uint8), w.view(torch.uint8)), (i, streams[i])
+    R.check_rocrand(L.rocrand_batch_plan_destroy(plan))
+
+
+@pytest.mark.parametrize("kind", sorted(DT))
+def test_mrg32k3a_wraps_at_tile_edges(kind):
+    streams = []
+    for k, left in enumerate((1, 255, 256, 257, 511, 512)):  # engines before the wrap
+        for shift in (0, 1, 3):
+            start = S - left
+            streams.append((R.MRG32K3A, kind, 100 + k, 5 * S + start, 2 * 777 + k, shift))
+    streams.append((R.MRG32K3A, kind, 7, 0, 300, 0))
+    streams.append((R.MRG32K3A, kind, 8, S - 1, 1, 1))
+    _check(streams)
+
+
+def test_small_and_large_batches():
+    for count in (1, 3, 200):
+        streams = []
+        for i in range(count):
+            rng = R.PHILOX4_32_10 if i % 2 else R.MRG32K3A
+            n = (0, 1, 5, 1023, 1024, 1025, 40001)[i % 7]
+            streams.append((rng, sorted(DT)[(i // 2) % 8], i, i * 7919, n, i % 3))
+        _check(streams)
+    # past one launch's tiles: every kind, engines that all wrap and take several steps
+    streams = [(R.MRG32K3A if i % 2 else R.PHILOX4_32_10, sorted(DT)[(i // 2) % 8], i, (1 << 20) + 7 + i, 3 * S + 5 + i,
+                i % 4) for i in range(40)]
+    _check(streams)
