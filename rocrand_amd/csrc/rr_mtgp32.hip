@@ -9,22 +9,31 @@
 // ring, the recurrence parameters and the tempering table of its parameter set;
 // every generator masks with the first set's mask (rocrand_mtgp32.h:381).
 //
-// The ring lives in LDS for the whole call, twice: word i at ring[i] and ring[i + 1024],
-// so a step's reads at off + t + {0, 1, pos - 1, pos} (off < 1024, t < 256, pos <= 95)
-// need no wrap-around masks and share one address (the two pairs differ by immediate
-// offsets from it and from pos - 1).  Every write goes to both copies.  One barrier per
-// block-step suffices: a step reads ring[off .. off+350] and writes ring[off+351 ..
-// off+606] (indices mod 1024), so reads and writes of one step never alias, and the next
-// step's reads see this step's writes after the barrier.
+// The ring lives in LDS for the whole call, turned so that the call starts at word 0, and four
+// block-steps go once around it.  The main loop runs them unrolled, so that every LDS address
+// is a register that never changes plus an immediate.  A step reads words w = off + t + {0, 1,
+// pos - 1, pos} unmasked (w <= 768 + 255 + 95): words 0 to 94 have a second copy behind the
+// ring, written by the one step of four that wraps.  One barrier per block-step suffices: a
+// step reads ring[off .. off+350] and writes ring[off+351 .. off+606] (indices mod 1024), so
+// reads and writes of one step never alias, and the next step's reads see this step's writes
+// after the barrier.
 //
 // The recurrence table of every parameter set is GF(2)-linear in its 4-bit index
 // (tbl[i ^ j] = tbl[i] ^ tbl[j], tbl[0] = 0: MTGP is an F2-linear generator; the host
 // checks it for all 512 sets when it builds the states), so its lookup, which sits on
 // the step's critical path (ring reads -> new word -> ring write -> barrier), is the XOR
-// of the entries at 1, 2, 4 and 8 selected by the index bits: about ten VALU operations
+// of the entries at 1, 2, 4 and 8 selected by the index bits: eight VALU operations
 // on block-uniform operands instead of a dependent LDS round trip.  The tempering
 // table's lookup only feeds the output; it stays an LDS read, issued as soon as the
-// ring reads return so that its latency overlaps the recurrence.
+// ring reads return so that its latency overlaps the recurrence (behind the barrier instead:
+// u32 3.00 -> 2.91 TB/s, Poisson 2.31 -> 2.13).
+//
+// 512 generators are two blocks a CU, and a block-step is as wide as the recurrence allows
+// (351 - 95 words), so two wavefronts a SIMD have to hide a step's LDS reads, write and
+// barrier.  Integers and uniforms are bound by that chain (170 ns a step), the transforms by
+// VALU issue on top of it.  With an 18-instruction step (28 with wrap-around masks and a copy
+// of every word): 2^26 values, normal f32 147.6 -> 118.6 us, u32 2.74 -> 3.00 TB/s, uniform
+// f64 2.97 -> 3.41, Poisson 1.90 -> 2.31.
 #include "rr_generator.hpp"
 
 #include <rocrand.h>
@@ -45,6 +54,8 @@ constexpr unsigned MTGP_BLOCK = 256;
 constexpr unsigned MTGP_N     = 351; // 11213 / 32 + 1
 constexpr unsigned MTGP_RING  = 1024;
 constexpr unsigned MTGP_MASKI = MTGP_RING - 1;
+constexpr unsigned MTGP_STEPS = MTGP_RING / MTGP_BLOCK; // block-steps once around the ring
+constexpr unsigned MTGP_COPY  = MTGP_N - MTGP_BLOCK;    // words that have a second copy
 
 // One generator's device state: ring, ring offset, parameters.
 struct mtgp_state
@@ -125,12 +136,19 @@ struct mtgp_call
     dist_params params;
 };
 
-// tbl[k & 15] of a GF(2)-linear 16-entry table from its entries at 1, 2, 4 and 8
-__host__ __device__ __forceinline__ uint32_t mtgp_lin16(uint32_t k, uint32_t e1, uint32_t e2, uint32_t e4,
-                                                        uint32_t e8)
+// acc ^ tbl[k & 15] of a GF(2)-linear 16-entry table from its entries at 1, 2, 4 and 8: a
+// sign-extending bit extraction and a v_bitop3 (a ^ (b & c)) each
+__device__ __forceinline__ uint32_t mtgp_lin16(uint32_t acc, uint32_t k, const uint32_t (&e)[4])
 {
-    return (e1 & (0u - (k & 1u))) ^ (e2 & (0u - ((k >> 1) & 1u))) ^ (e4 & (0u - ((k >> 2) & 1u)))
-           ^ (e8 & (0u - ((k >> 3) & 1u)));
+#pragma unroll
+    for(uint32_t i = 0; i < 4; i++)
+        acc = __builtin_amdgcn_bitop3_b32(acc, e[i], __builtin_amdgcn_sbfe(k, i, 1), 0x78);
+    return acc;
+}
+
+uint32_t host_lin16(uint32_t k, const uint32_t* tbl)
+{
+    return (k & 1 ? tbl[1] : 0) ^ (k & 2 ? tbl[2] : 0) ^ (k & 4 ? tbl[4] : 0) ^ (k & 8 ? tbl[8] : 0);
 }
 
 template<class D>
@@ -142,17 +160,14 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
     constexpr int BYTES = OUT * (int)sizeof(out_t);
     static_assert(BYTES == 2 || BYTES == 4 || BYTES == 8 || BYTES == 16, "vec size");
 
-    __shared__ uint32_t ring[2 * MTGP_RING];
+    __shared__ uint32_t ring[MTGP_RING + MTGP_COPY];
     __shared__ uint32_t ttbl[16];
 
     const uint32_t b = blockIdx.x, t = threadIdx.x;
     mtgp_state*    g = c.states + b;
+    const uint32_t off0 = g->offset;
     for(uint32_t i = t; i < MTGP_RING; i += MTGP_BLOCK)
-    {
-        const uint32_t w   = g->status[i];
-        ring[i]             = w;
-        ring[i + MTGP_RING] = w;
-    }
+        ring[i] = g->status[(i + off0) & MTGP_MASKI];
     const uint32_t pos = g->pos, sh1 = g->sh1, sh2 = g->sh2, mask = g->mask;
     if(t < 16)
         ttbl[t] = g->tmp[t];
@@ -167,30 +182,33 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
             lds_packed[i] = c.params.pt.packed[i];
         kp.pt.packed = lds_packed;
     }
-    const uint32_t p1 = g->tbl[1], p2 = g->tbl[2], p4 = g->tbl[4], p8 = g->tbl[8];
-    uint32_t       off = g->offset;
+    const uint32_t lin[4] = {g->tbl[1], g->tbl[2], g->tbl[4], g->tbl[8]};
     stage_tables<D>(kp.tab);
     __syncthreads();
 
-    // one block-step: this thread's tempered word
-    auto step = [&]() -> uint32_t {
-        const uint32_t* rp = ring + t + off;
-        uint32_t        X  = (rp[0] & mask) ^ rp[1];
-        uint32_t        Y  = rp[pos];
-        uint32_t        T  = rp[pos - 1];
-        X ^= X << sh1;
-        Y = X ^ (Y >> sh2);
+    // one block-step, the `ph`-th of its turn: this thread's tempered word
+    const uint32_t* const rx   = ring + t;
+    const uint32_t* const ry   = ring + t + pos;
+    uint32_t* const       wrap = ring + (t < MTGP_RING - MTGP_N - 2 * MTGP_BLOCK ? t + 2 * MTGP_BLOCK + MTGP_N
+                                                                                : t + 2 * MTGP_BLOCK + MTGP_N - MTGP_RING);
+    auto step = [&](uint32_t ph) -> uint32_t {
+        const uint32_t at = ph * MTGP_BLOCK;
+        uint32_t       X  = (rx[at] & mask) ^ rx[at + 1];
+        uint32_t       Y  = ry[at];
+        uint32_t       T  = ry[(int)at - 1];
+        X                 = __builtin_amdgcn_bitop3_b32(X, X << sh1, Y >> sh2, 0x96);
         T ^= T >> 16;
         T ^= T >> 8;
-        const uint32_t tt  = ttbl[T & 0x0f];
-        const uint32_t r   = Y ^ mtgp_lin16(Y, p1, p2, p4, p8);
-        uint32_t* const wp = ring + ((t + off + MTGP_N) & MTGP_MASKI);
-        wp[0]              = r;
-        wp[MTGP_RING]      = r;
-        const uint32_t o   = r ^ tt;
-        off = (off + MTGP_BLOCK) & MTGP_MASKI;
+        const uint32_t tt = ttbl[T & 0x0f];
+        const uint32_t r  = mtgp_lin16(X, X, lin);
+        if(ph == MTGP_STEPS - 1)
+            ring[t + at + MTGP_N - MTGP_RING] = r;
+        else
+            ring[t + at + MTGP_N] = r;
+        if(ph == MTGP_STEPS - 2)
+            *wrap = r; // the words just written behind the ring, at its start (others: the same word)
         __syncthreads();
-        return o;
+        return r ^ tt;
     };
 
     out_t* const data     = static_cast<out_t*>(c.data);
@@ -206,12 +224,7 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
     const size_t   base0 = (size_t)b * MTGP_BLOCK;
     const uint32_t steps = base0 < down ? (uint32_t)((down - base0 + stride - 1) / stride) : 0u;
     out_t*         bptr  = vec_data + base0 * OUT;
-    for(uint32_t k = 0; k < steps; k++, bptr += stride * OUT)
-    {
-#pragma unroll
-        for(int i = 0; i < IN; i++)
-            in[i] = step();
-        D::apply(in, o, kp);
+    auto store = [&]() {
         out_t* const dst = bptr + t * OUT;
         if constexpr(BYTES == 2)
             *reinterpret_cast<uint16_t*>(dst) = *reinterpret_cast<const uint16_t*>(o);
@@ -221,14 +234,36 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
             *reinterpret_cast<uint2*>(dst) = *reinterpret_cast<const uint2*>(o);
         else
             *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(o);
+        bptr += stride * OUT;
+    };
+    static_assert(MTGP_STEPS % IN == 0, "whole vecs a turn");
+    constexpr uint32_t PER = MTGP_STEPS / IN; // vecs a turn
+    uint32_t           k = 0, ph = 0;
+    for(; k + PER <= steps; k += PER)
+#pragma unroll
+        for(uint32_t v = 0; v < PER; v++)
+        {
+#pragma unroll
+            for(int i = 0; i < IN; i++)
+                in[i] = step(v * IN + i);
+            D::apply(in, o, kp);
+            store();
+        }
+    // fewer than a turn is left, and the two extra uses
+    auto next_vec = [&]() {
+        for(int i = 0; i < IN; i++, ph = (ph + 1) % MTGP_STEPS)
+            in[i] = step(ph);
+        D::apply(in, o, kp);
+    };
+    for(; k < steps; k++)
+    {
+        next_vec();
+        store();
     }
     size_t index = base0 + (size_t)steps * stride + t;
     if(index - t < up)
     {
-#pragma unroll
-        for(int i = 0; i < IN; i++)
-            in[i] = step();
-        D::apply(in, o, kp);
+        next_vec();
         if(index < c.vec_n)
             for(int j = 0; j < OUT; j++)
                 vec_data[index * OUT + j] = o[j];
@@ -236,10 +271,7 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
     }
     if(OUT > 1 && (c.head > 0 || c.tail > 0))
     {
-#pragma unroll
-        for(int i = 0; i < IN; i++)
-            in[i] = step();
-        D::apply(in, o, kp);
+        next_vec();
         if(index == up)
             for(uint32_t j = 0; j < (uint32_t)OUT; j++)
                 if(j < c.head)
@@ -251,9 +283,9 @@ __global__ __launch_bounds__(MTGP_BLOCK) void mtgp_kernel(mtgp_call c)
     }
 
     for(uint32_t i = t; i < MTGP_RING; i += MTGP_BLOCK)
-        g->status[i] = ring[i];
+        g->status[(i + off0) & MTGP_MASKI] = ring[i];
     if(t == 0)
-        g->offset = off;
+        g->offset = (off0 + ph * MTGP_BLOCK) & MTGP_MASKI;
 }
 
 template<class D>
@@ -305,8 +337,7 @@ rocrand_status device_params(const mtgp_param*& out)
             if(p[i].pos == 0 || p[i].pos + MTGP_BLOCK > MTGP_N)
                 return ROCRAND_STATUS_INTERNAL_ERROR;
             for(uint32_t k = 0; k < 16; k++)
-                if(p[i].tbl[k] != mtgp_lin16(k, p[i].tbl[1], p[i].tbl[2], p[i].tbl[4], p[i].tbl[8])
-                   || p[i].tmp[k] != mtgp_lin16(k, p[i].tmp[1], p[i].tmp[2], p[i].tmp[4], p[i].tmp[8]))
+                if(p[i].tbl[k] != host_lin16(k, p[i].tbl) || p[i].tmp[k] != host_lin16(k, p[i].tmp))
                     return ROCRAND_STATUS_INTERNAL_ERROR;
         }
         void* d = nullptr;
