@@ -378,9 +378,9 @@ struct mrg_consts<31>
 // conversion: the double with high word 0x43300000 and low word v is 2^52 + v exactly,
 // and fma(2^52 + v, k, -2^52 k) rounds (2^52 + v) k - 2^52 k = v k once (2^52 k is exact,
 // a power-of-two scaling of k).
-__device__ __forceinline__ double scale_u32(uint32_t v, double k)
+__host__ __device__ __forceinline__ double scale_u32(uint32_t v, double k)
 {
-    const double x = __hiloint2double(0x43300000, (int)v);
+    const double x = rr_bits_to_double(0x4330000000000000ull | v);
     return __builtin_fma(x, k, -0x1p52 * k);
 }
 
@@ -391,7 +391,7 @@ __device__ __forceinline__ uint32_t mrg_uint(uint32_t v)
     return (uint32_t)scale_u32(v - 1, mrg_consts<MRG>::uint_norm);
 }
 template<int MRG>
-__device__ __forceinline__ float mrg_f32(uint32_t v)
+__host__ __device__ __forceinline__ float mrg_f32(uint32_t v)
 {
     return (float)scale_u32(v, mrg_consts<MRG>::norm);
 }
@@ -512,8 +512,12 @@ __device__ __forceinline__ void box_muller_double(uint32_t a, uint32_t b, uint32
 //   angle: a = t - q P is exact for P = pi/128 rounded to double; sin and cos of q P as
 //     double-doubles, the products with a and the sums carried with their errors.
 // Relative error below 2^-58 before the rounding: within 0.52 ulp of the exact value, where
-// the reference's steps (log, sqrt, sin/cos and product, rounded one by one) may be 1.8
-// ulp off, and within 2 ulp of those.  115 VALU instructions with its uniforms and the
+// the reference's steps (log, sqrt, sin/cos and product, rounded one by one) may be 2.3
+// ulp off, and within 2 ulp of those.  Next to a quarter turn (an MRG's float angle is
+// exactly one for one pair in some 10^7) the small sine or cosine is the table entry's tail,
+// itself a rounded double, so that value is within 1 ulp (0.89 the largest of 2.6e7 there),
+// and the head's part of the radius' tail alone would leave it 40 ulp off: hence
+// (sn + se) tl and (cs + ce) tl.  117 VALU instructions with its uniforms and the
 // affine step; taking those steps one by one, each correctly rounded, costs 243 (XORWOW
 // normal f64, 2^27 values: 2.10 -> 3.57 TB/s, MRG32k3a 2.07 -> 3.56, Philox 1.98 -> 3.14).
 __host__ __device__ __forceinline__ void box_muller_pair_double(double u, double t, uint32_t qoff, double& r0,
@@ -569,8 +573,8 @@ __host__ __device__ __forceinline__ void box_muller_pair_double(double u, double
     ce                 = __builtin_fma(-Sl, a, ce - __builtin_fma(S, a, -p2) + Cl);
     // the products, rounded once
     const double  q0   = sn * th, q1 = cs * th;
-    r0 = q0 + __builtin_fma(se, th, __builtin_fma(sn, tl, __builtin_fma(sn, th, -q0)));
-    r1 = q1 + __builtin_fma(ce, th, __builtin_fma(cs, tl, __builtin_fma(cs, th, -q1)));
+    r0 = q0 + __builtin_fma(se, th, __builtin_fma(sn + se, tl, __builtin_fma(sn, th, -q0)));
+    r1 = q1 + __builtin_fma(ce, th, __builtin_fma(cs + ce, tl, __builtin_fma(cs, th, -q1)));
 }
 // The pair of four words: u = (v1 + 1) 2^-53 and w = (v2 + 1) 2^-52 rounded to double, each
 // from its word's halves in two exact fused operations and one rounding (rocrand_normal.h:76-96);
@@ -631,8 +635,8 @@ __device__ __forceinline__ void mrg_box_muller_double(uint32_t x, uint32_t y, do
 }
 // The pair of rocrand_normal.h:156-172 evaluated as double-doubles and rounded once.
 template<int MRG>
-__device__ __forceinline__ void mrg_normal_pair_double(uint32_t x, uint32_t y, double& r0, double& r1,
-                                                       const math_tables& tab)
+__host__ __device__ __forceinline__ void mrg_normal_pair_double(uint32_t x, uint32_t y, double& r0, double& r1,
+                                                                const math_tables& tab = math_tables{})
 {
     ROCRAND_AMD_FP_EXACT
     constexpr int SH = MRG == 32 ? 19 : 18;

@@ -6,7 +6,8 @@
  *
  * usage: normal_twin N
  * prints NAME COUNT VALUES  for the float functions' results that are not the correctly
- * rounded ones, and  NAME VALUES MAX_ERR_MICROULP BEYOND_2ULP_OF_LIBM  for the pairs.
+ * rounded ones, and  NAME VALUES MAX_ERR_MICROULP BEYOND_2ULP_OF_LIBM  for the pairs (the
+ * rows next to quarter turns with the reference's steps' own MAX_ERR_MICROULP behind).
  */
 #include <rocrand/rocrand_amd_math.h>
 
@@ -53,6 +54,87 @@ static uint32_t word(long i)
                                     0xffffffffu};
     constexpr long        n = sizeof(edge) / sizeof(edge[0]);
     return i < n ? edge[i] : (uint32_t)(next64() >> 13);
+}
+
+// The double pair at angle t, radius uniform u: worst error in ulp of exact and, in `beyond`,
+// the values more than 2 ulp from the reference's steps over this libm, whose own worst
+// error goes to `host`.
+static void pair_check(double u, double t, const double (&g)[2], double& worst, long& beyond, double& host)
+{
+    const double     hs = sqrt(-2.0 * log(u)), h[2] = {sin(t) * hs, cos(t) * hs};
+    const __float128 S = sqrtq(-2 * logq((__float128)u));
+    const __float128 e[2] = {sinq((__float128)t) * S, cosq((__float128)t) * S};
+    for(int j = 0; j < 2; j++)
+    {
+        beyond += ulps<double, int64_t>(g[j], h[j]) > 2;
+        if(e[j] != 0)
+        {
+            worst = fmax(worst, error<double>(g[j], e[j]));
+            host  = fmax(host, error<double>(h[j], e[j]));
+        }
+    }
+}
+static void pair_words(uint32_t a, uint32_t b, uint32_t c, uint32_t d, double& worst, long& beyond, double& host)
+{
+    double g[2];
+    normal_pair_double(a, b, c, d, g[0], g[1]);
+    const uint64_t v1 = (uint64_t)a ^ ((uint64_t)b << 21), v2 = (uint64_t)c ^ ((uint64_t)d << 21);
+    const double   u = R_2POW53_INV_DBL + (double)v1 * R_2POW53_INV_DBL;
+    const double   t = (R_2POW53_INV_DBL * 2.0 + (double)v2 * (R_2POW53_INV_DBL * 2.0)) * R_PI_DBL;
+    pair_check(u, t, g, worst, beyond, host);
+}
+template<int MRG>
+static void pair_mrg(uint32_t x, uint32_t y, double& worst, long& beyond, double& host)
+{
+    double g[2];
+    mrg_normal_pair_double<MRG>(x, y, g[0], g[1]);
+    const float u = (float)((double)x * mrg_consts<MRG>::norm), v = (float)((double)y * mrg_consts<MRG>::norm);
+    pair_check((double)u, (double)v * 2.0 * R_PI_DBL, g, worst, beyond, host);
+}
+
+// The double pair next to the multiples of a quarter turn, where the sine or cosine is as
+// small as the angle's own rounding: every w = (v2 + 1) 2^-52 within 256 steps of 0, 1/2,
+// 1, 3/2 and 2, and the MRG words next to those that round to these (a float angle is
+// exactly a quarter turn for a few hundred words), `n` radius words each.
+template<class F>
+static void quarter_row(const char* name, long count, F one)
+{
+    double worst = 0.0, host = 0.0;
+    long   beyond = 0, total = 0;
+    for(long i = 0; i < count; i++)
+        total += 2 * one(i, worst, beyond, host);
+    printf("%s %ld %ld %ld %ld\n", name, total, (long)(worst * 1e6), beyond, (long)(host * 1e6));
+}
+template<int MRG>
+static void mrg_quarter_row(const char* name, int n)
+{
+    constexpr uint64_t m1 = MRG == 32 ? 4294967087ull : 2147483647ull;
+    quarter_row(name, 5 * 601, [&](long i, double& worst, long& beyond, double& host) {
+        const int64_t y = (int64_t)((i / 601) * ((m1 + 1) / 4)) + i % 601 - 300;
+        if(y < 1 || y > (int64_t)m1)
+            return 0;
+        for(int k = 0; k < n; k++)
+            pair_mrg<MRG>(k == 0 ? 1u : k == 1 ? (uint32_t)m1 : 1u + (uint32_t)(next64() % m1), (uint32_t)y, worst,
+                          beyond, host);
+        return n;
+    });
+}
+static void quarter_rows(int n)
+{
+    quarter_row("quarter_words", 5 * 513, [&](long i, double& worst, long& beyond, double& host) {
+        const int64_t v2 = (int64_t)(i / 513) * (1ll << 51) - 1 + i % 513 - 256;
+        if(v2 < 0 || v2 >= 1ll << 53)
+            return 0;
+        const uint32_t d = (uint32_t)(v2 >> 32) << 11, c = (uint32_t)v2;
+        for(int k = 0; k < n; k++)
+        {
+            const uint64_t x = k == 0 ? 0 : k == 1 ? ~0ull : next64();
+            pair_words((uint32_t)x, (uint32_t)(x >> 32), c, d, worst, beyond, host);
+        }
+        return n;
+    });
+    mrg_quarter_row<32>("quarter_mrg32", n);
+    mrg_quarter_row<31>("quarter_mrg31", n);
 }
 
 int main(int argc, char** argv)
@@ -112,25 +194,10 @@ int main(int argc, char** argv)
     for(long i = 0; i < n; i++)
     {
         const uint32_t a = word(i), b = word(i / 15), c = word(i), d = word(i < 225 ? i % 15 : 99);
-        double         g[2];
-        normal_pair_double(a, b, c, d, g[0], g[1]);
-        const uint64_t v1 = (uint64_t)a ^ ((uint64_t)b << 21), v2 = (uint64_t)c ^ ((uint64_t)d << 21);
-        const double   u = R_2POW53_INV_DBL + (double)v1 * R_2POW53_INV_DBL;
-        const double   t = (R_2POW53_INV_DBL * 2.0 + (double)v2 * (R_2POW53_INV_DBL * 2.0)) * R_PI_DBL;
-        const double   hs = sqrt(-2.0 * log(u)), h[2] = {sin(t) * hs, cos(t) * hs};
-        const __float128 S = sqrtq(-2 * logq((__float128)u));
-        const __float128 e[2] = {sinq((__float128)t) * S, cosq((__float128)t) * S};
-        for(int j = 0; j < 2; j++)
-        {
-            beyond += ulps<double, int64_t>(g[j], h[j]) > 2;
-            if(e[j] != 0)
-            {
-                worst = fmax(worst, error<double>(g[j], e[j]));
-                host  = fmax(host, error<double>(h[j], e[j]));
-            }
-        }
+        pair_words(a, b, c, d, worst, beyond, host);
     }
     printf("pair_f64 %ld %ld %ld\nsteps_f64 %ld\n", 2 * n, (long)(worst * 1e6), beyond, (long)(host * 1e6));
+    quarter_rows((int)(n / 4000));
     printf("special %d %d %d %d\n", logf_unit(1.0f) == 0.0f, expf_acc(-200.0f) == 0.0f, isinf(expf_acc(200.0f)),
            isnan(expf_acc(NAN)));
     return 0;

@@ -135,6 +135,19 @@ def test_normals_error_against_exact_box_muller(name, rng, family):
     check("normal_f64", got, want, (0.0, 1.0))
 
 
+@pytest.mark.parametrize("vec_step,value", [(107, 258765), (115, 39347), (194, 174849)])
+def test_mrg32k3a_double_pair_at_a_quarter_turn(vec_step, value):
+    """Values 28308173, 30185907 and 51030785 of the stream under seed 12345: their float angle is
+    exactly a quarter turn, so the cosine or sine is the angle's own rounding error (about
+    1e-16) and the result has to keep its relative accuracy."""
+    n, offset = 2 * S, 2 * vec_step * S
+    got = _device(R.MRG32K3A, "normal_f64", n, 12345, offset, (0.0, 1.0))
+    _, want = O.OracleGen(O.MRG32K3A, seed=12345, offset=offset).generate("normal_f64", n, 0x1000, 0.0, 1.0)
+    assert 0.0 < abs(want[value]) < 1e-15
+    d = ulp_distance(got, want)
+    assert d.max() <= 2, (int(d.argmax()), got[d.argmax()], want[d.argmax()])
+
+
 CONFIG2 = [("philox", R.PHILOX4_32_10), ("threefry4x32", R.THREEFRY4_32_20), ("mrg32k3a", R.MRG32K3A),
            ("xorwow", R.XORWOW), ("lfsr113", R.LFSR113)]
 CONFIG2_KINDS = [("u32", torch.uint32, "generate", ()), ("uniform_f32", torch.float32, "uniform", ()),

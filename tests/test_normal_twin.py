@@ -40,3 +40,14 @@ def test_pairs(rows, name, most):
     assert beyond == 0
     # the steps rounded one by one are further off: the comparison is not vacuous
     assert rows["steps_f64"][0] >= 1_000_000
+
+
+@pytest.mark.parametrize("name", ["quarter_words", "quarter_mrg32", "quarter_mrg31"])
+def test_double_pair_next_to_quarter_turns(rows, name):
+    """There the small sine or cosine is a table entry rounded to a double (half an ulp), and
+    the result is rounded once (another half)."""
+    n, worst, beyond, steps = rows[name]
+    assert n > 400000
+    assert worst <= 1_000_000
+    assert beyond == 0
+    assert steps >= 1_500_000  # the steps rounded one by one are further off
