@@ -414,7 +414,7 @@ __device__ __forceinline__ double mrg_f64(uint32_t v)
 //     Newton step gives 2 sqrt(x) = t (3 - t y) to 2^-46, and as 3 - t y is 2 to 2^-23,
 //     2 sqrt(x) cos a = t (3 - a^2 - t y) to 2^-33: the cosine costs no product of its own.
 //     The doubling is the table's half; the radius keeps the sign of a zero.
-// The pair before its rounding is within 2^-30 of exact, so each output is within 0.505
+// The pair before its rounding is within 2^-31 of exact, so each output is within 0.508
 // ulp of the exact value, and within 2 ulp of the reference's float pipeline (logf, sqrtf,
 // sinf/cosf and the product: four roundings, rocrand_normal.h:51-66).  About 34 VALU
 // operations a pair (38 with sin and cos as sums of products with sin a and cos a and a

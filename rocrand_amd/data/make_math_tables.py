@@ -1,21 +1,6 @@
 """Write include/rocrand/rocrand_amd_mathtab.h: the tables of the float-argument logarithm
 (Box-Muller radius), sine and cosine (Box-Muller angle) and exponential (log-normal
-outputs) evaluated in double.  The first logarithm table and the first sine and cosine table
-serve arguments of any origin (tests/fastmath_twin.c); the transforms take the Box-Muller
-tables below, indexed by the bits their arguments came from.
-
-Logarithm, 64 entries: a positive normal float u is split as u = 2^k z with z in
-[0x3f330000, 0x3fb30000) (about [0.699, 1.398)), so that k = 0 around u = 1.  Entry i
-covers the z whose bit pattern minus 0x3f330000 has bits 17..22 equal to i; it holds
-invc = 1/c for the centre c of that interval (rounded to double) and logc = -ln(invc)
-rounded to double, with invc = 1 and logc = 0 exactly for the interval that contains 1.
-Then ln u = k ln 2 + logc + log1p(z invc - 1), |z invc - 1| < 2^-7.
-
-Sine and cosine, 64 entries: sin(k pi/32), cos(k pi/32) rounded to double (exact 0 and +-1
-at multiples of pi/2); with x = q pi/32 + r, |r| <= pi/64, k = q mod 64,
-sin x = sin(a_k) cos r + cos(a_k) sin r and cos x = cos(a_k) cos r - sin(a_k) sin r.  The
-reduction constant pi/32 is split into a head with its low 8 bits clear (exact products
-with q < 2^7) and the rounded remainder.
+outputs) evaluated in double, and of the double transforms.
 
 Exponential, 32 entries: 2^(j/32) rounded to double, j = 0..31; with x = (32 e + j) ln2/32
 + r, |r| <= ln2/64, exp x = 2^e 2^(j/32) exp(r).  The reduction constant ln2/32 is split
@@ -73,46 +58,11 @@ import mpmath
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 OUT = os.path.join(os.path.dirname(os.path.dirname(HERE)), "include", "rocrand", "rocrand_amd_mathtab.h")
-OFF = 0x3F330000
-N_LOG = 64
 N_EXP = 32
-N_SC = 64
-
-
-def f32(bits):
-    return struct.unpack("<f", struct.pack("<I", bits))[0]
-
-
-def log_entries():
-    one = 0x3F800000
-    out = []
-    for i in range(N_LOG):
-        lo_bits = OFF + (i << 17)
-        hi_bits = OFF + ((i + 1) << 17)
-        if lo_bits <= one < hi_bits:
-            out.append((1.0, 0.0))
-            continue
-        c = (mpmath.mpf(f32(lo_bits)) + mpmath.mpf(f32(hi_bits))) / 2
-        invc = float(1 / c)
-        logc = float(-mpmath.log(mpmath.mpf(invc)))
-        out.append((invc, logc))
-    return out
 
 
 def exp_entries():
     return [float(mpmath.power(2, mpmath.mpf(j) / N_EXP)) for j in range(N_EXP)]
-
-
-def sincos_entries():
-    out = []
-    for k in range(N_SC):
-        if k % (N_SC // 4) == 0:  # multiples of pi/2: exact values
-            q = k // (N_SC // 4)
-            out.append(([0.0, 1.0, 0.0, -1.0][q], [1.0, 0.0, -1.0, 0.0][q]))
-            continue
-        a = k * mpmath.pi / (N_SC // 2)
-        out.append((float(mpmath.sin(a)), float(mpmath.cos(a))))
-    return out
 
 
 BM_EMIN = 95  # biased exponent of 2^-32
@@ -260,12 +210,8 @@ def ln2_split():
 
 def main():
     mpmath.mp.prec = 200
-    log_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}}}," for a, b in log_entries())
     exp_rows = "\n".join(f"    {a.hex()}," for a in exp_entries())
     head, tail, inv = ln2_split()
-    sc_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}}}," for a, b in sincos_entries())
-    sc_head, sc_tail = split(mpmath.pi / (N_SC // 2), 8)
-    sc_inv = float((N_SC // 2) / mpmath.pi)
     dlog_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}, {c.hex()}, 0.0}}," for a, b, c in dlog_entries())
     dexp_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}}}," for a, b in dexp_entries())
     dsc_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}, {c.hex()}, {d.hex()}}}," for a, b, c, d in dsincos_entries())
@@ -297,13 +243,6 @@ def main():
 
 namespace rocrand_amd_engine
 {{
-constexpr uint32_t RR_LOGTAB_OFF  = 0x{OFF:08x}u;
-constexpr int      RR_LOGTAB_BITS = 6;
-// {{1/c, -ln(1/c)}}
-RR_MATH_TABLE const double2 rr_logtab[{N_LOG}] = {{
-{log_rows}
-}};
-
 constexpr int    RR_EXPTAB_BITS  = 5;
 constexpr double RR_EXP_INV_STEP = {inv.hex()}; // {N_EXP} / ln 2
 constexpr double RR_EXP_STEP_HI  = {head.hex()}; // ln 2 / {N_EXP}, low 16 bits clear
@@ -311,15 +250,6 @@ constexpr double RR_EXP_STEP_LO  = {tail.hex()}; // ln 2 / {N_EXP} - RR_EXP_STEP
 // 2^(j/{N_EXP})
 RR_MATH_TABLE const double rr_exptab[{N_EXP}] = {{
 {exp_rows}
-}};
-
-constexpr int    RR_SCTAB_BITS  = 6;
-constexpr double RR_SC_INV_STEP = {sc_inv.hex()}; // {N_SC // 2} / pi
-constexpr double RR_SC_STEP_HI  = {sc_head.hex()}; // pi / {N_SC // 2}, low 8 bits clear
-constexpr double RR_SC_STEP_LO  = {sc_tail.hex()}; // pi / {N_SC // 2} - RR_SC_STEP_HI
-// {{sin(k pi/{N_SC // 2}), cos(k pi/{N_SC // 2})}}
-RR_MATH_TABLE const double2 rr_sctab[{N_SC}] = {{
-{sc_rows}
 }};
 
 // Box-Muller pair: {{2^(127-e)/c, 2 ln(2^(127-e)/c)}} for biased exponents e = {BM_EMIN}..{BM_EMAX}

@@ -6,8 +6,8 @@
  *
  * usage: normal_twin N
  * prints NAME COUNT VALUES  for the float functions' results that are not the correctly
- * rounded ones, and  NAME VALUES MAX_ERR_MICROULP BEYOND_2ULP_OF_LIBM  for the pairs (the
- * rows next to quarter turns with the reference's steps' own MAX_ERR_MICROULP behind).
+ * rounded ones, and  NAME VALUES MAX_ERR_MICROULP BEYOND_2ULP_OF_LIBM  and the MAX_ERR_MICROULP
+ * of the reference's steps over this libm for the pairs.
  */
 #include <rocrand/rocrand_amd_math.h>
 
@@ -46,14 +46,59 @@ static double error(F got, __float128 exact)
     const F sp = nextafter(e, (F)INFINITY) - e;
     return (double)(fabsq((__float128)got - exact) / (__float128)sp);
 }
-// words at the ends of their range and next to the angle table's boundaries, then random
+// words at the ends of their range and next to the angle tables' boundaries (odd multiples
+// of 2^22 for the float pair, of 2^23 for the others), then random; the first EDGES^2
+// pairs are all pairs of the edges
+static const uint32_t edge[] = {0u,          1u,          0x1fffffu,   0x200000u,   0x3fffffu,   0x400000u,   0x400001u,
+                                0x7fffffu,   0x800000u,   0x3fffffffu, 0x40000000u, 0x7fbfffffu, 0x7fc00000u, 0x7fffffffu,
+                                0x80000000u, 0x803fffffu, 0x80400000u, 0xbfffffffu, 0xffbfffffu, 0xffc00000u, 0xffffff7fu,
+                                0xffffff80u, 0xfffffffeu, 0xffffffffu};
+constexpr long        EDGES  = sizeof(edge) / sizeof(edge[0]);
 static uint32_t word(long i)
 {
-    static const uint32_t edge[] = {0u, 1u, 0x1fffffu, 0x200000u, 0x7fffffu, 0x800000u, 0x3fffffffu, 0x40000000u,
-                                    0x7fffffffu, 0x80000000u, 0xbfffffffu, 0xffbfffffu, 0xffffff7fu, 0xffffff80u,
-                                    0xffffffffu};
-    constexpr long        n = sizeof(edge) / sizeof(edge[0]);
-    return i < n ? edge[i] : (uint32_t)(next64() >> 13);
+    return i < EDGES ? edge[i] : (uint32_t)(next64() >> 13);
+}
+static uint32_t word_x(long i) { return word(i < EDGES * EDGES ? i / EDGES : EDGES); }
+static uint32_t word_y(long i) { return word(i < EDGES * EDGES ? i % EDGES : EDGES); }
+
+// The float pair: rows as for the double pair below; a sign that differs from the steps'
+// (a radius of -0 keeps its sign) counts as beyond.
+template<class F>
+static void pair_f32_row(const char* name, long n, F uv)
+{
+    double worst = 0.0, host = 0.0;
+    long   beyond = 0;
+    for(long i = 0; i < n; i++)
+    {
+        float    u, v, g[2];
+        uint32_t qoff;
+        uv(word_x(i), word_y(i), u, v, qoff);
+        box_muller_dd<false>(u, v, qoff, g[0], g[1]);
+        const float       hs = sqrtf(-2.0f * logf(u)), h[2] = {sinf(v) * hs, cosf(v) * hs};
+        const long double S = sqrtl(-2.0L * logl((long double)u));
+        const __float128  e[2] = {(__float128)(sinl((long double)v) * S), (__float128)(cosl((long double)v) * S)};
+        for(int j = 0; j < 2; j++)
+        {
+            beyond += ulps<float, int32_t>(g[j], h[j]) > 2 || !signbit(g[j]) != !signbit(h[j]);
+            if(e[j] != 0)
+            {
+                worst = fmax(worst, error<float>(g[j], e[j]));
+                host  = fmax(host, error<float>(h[j], e[j]));
+            }
+        }
+    }
+    printf("%s %ld %ld %ld %ld\n", name, 2 * n, (long)(worst * 1e6), beyond, (long)(host * 1e6));
+}
+// mrg_box_muller's float uniform and angle of values in [1, m1]
+template<int MRG>
+static void mrg_uv(uint32_t x, uint32_t y, float& u, float& v, uint32_t& qoff)
+{
+    constexpr uint64_t m1 = MRG == 32 ? 4294967087ull : 2147483647ull;
+    x = x == 0xffffffffu ? (uint32_t)m1 : 1u + (uint32_t)((MRG == 32 ? x : x >> 1) % m1); // u = 1 among them
+    y = 1u + (uint32_t)((MRG == 32 ? y : y >> 1) % m1);
+    u    = (float)((double)x * mrg_consts<MRG>::norm);
+    v    = (float)((double)y * mrg_consts<MRG>::norm) * R_2PI;
+    qoff = ((y >> (MRG == 32 ? 19 : 18)) + 8u) & ~15u;
 }
 
 // The double pair at angle t, radius uniform u: worst error in ulp of exact and, in `beyond`,
@@ -169,34 +214,21 @@ int main(int argc, char** argv)
         bad += expf_acc(x) != (float)expl((long double)x);
     }
     printf("exp %ld %ld\n", bad, total);
-    double worst = 0.0;
+    pair_f32_row("pair_f32", 5 * n, [](uint32_t x, uint32_t y, float& u, float& v, uint32_t& qoff) {
+        u    = (float)x * R_2POW32_INV + R_2POW32_INV;
+        v    = R_2POW32_INV_2PI + (float)y * R_2POW32_INV_2PI;
+        qoff = ((y >> 19) + 8u) & ~15u;
+    });
+    pair_f32_row("pair_f32_mrg32", 5 * n, mrg_uv<32>);
+    pair_f32_row("pair_f32_mrg31", 5 * n, mrg_uv<31>);
+    double worst = 0.0, host = 0.0;
     long   beyond = 0;
     for(long i = 0; i < n; i++)
     {
-        const uint32_t x = word(i / 15), y = word(i % 225 < 15 && i < 225 ? i % 15 : 99);
-        const float    u = (float)x * R_2POW32_INV + R_2POW32_INV;
-        const float    v = R_2POW32_INV_2PI + (float)y * R_2POW32_INV_2PI;
-        float          g[2];
-        box_muller_dd<false>(u, v, ((y >> 19) + 8u) & ~15u, g[0], g[1]);
-        const float       hs = sqrtf(-2.0f * logf(u)), h[2] = {sinf(v) * hs, cosf(v) * hs};
-        const long double S = sqrtl(-2.0L * logl((long double)u));
-        const __float128  e[2] = {(__float128)(sinl((long double)v) * S), (__float128)(cosl((long double)v) * S)};
-        for(int j = 0; j < 2; j++)
-        {
-            beyond += ulps<float, int32_t>(g[j], h[j]) > 2;
-            worst = e[j] != 0 ? fmax(worst, error<float>(g[j], e[j])) : worst;
-        }
-    }
-    printf("pair_f32 %ld %ld %ld\n", 2 * n, (long)(worst * 1e6), beyond);
-    worst  = 0.0;
-    beyond = 0;
-    double host = 0.0;
-    for(long i = 0; i < n; i++)
-    {
-        const uint32_t a = word(i), b = word(i / 15), c = word(i), d = word(i < 225 ? i % 15 : 99);
+        const uint32_t a = word(i), b = word_x(i), c = word(i), d = word_y(i);
         pair_words(a, b, c, d, worst, beyond, host);
     }
-    printf("pair_f64 %ld %ld %ld\nsteps_f64 %ld\n", 2 * n, (long)(worst * 1e6), beyond, (long)(host * 1e6));
+    printf("pair_f64 %ld %ld %ld %ld\n", 2 * n, (long)(worst * 1e6), beyond, (long)(host * 1e6));
     quarter_rows((int)(n / 4000));
     printf("special %d %d %d %d\n", logf_unit(1.0f) == 0.0f, expf_acc(-200.0f) == 0.0f, isinf(expf_acc(200.0f)),
            isnan(expf_acc(NAN)));
