@@ -39,10 +39,10 @@ constexpr float  R_SQRT2          = 1.4142135f;
 //   neg2log (Box-Muller radius, u a positive normal float in [2^-32, 1]): one table load
 //        indexed by u's exponent and 6 leading mantissa bits, |u a - 1| < 2^-7, series to
 //        r^4 (relative error < 2^-30) or r^6 (< 2^-44);
-//   sin/cos of a Box-Muller angle: table entry from the word that the angle came from, the
-//        difference exact in float, series to a^5 / a^6 on |a| < 0.0124 (errors < 2^-47);
-//   expf_acc: reduction by ln2/32, 2^(j/32) from rocrand_amd_mathtab.h, series of
-//        exp(r) - 1 to r^5 on |r| < 0.0109, scaling by 2^e in double.
+//   sin/cos of a Box-Muller angle: table entry from the word that the angle came from,
+//        series to a^7 / a^6 on |a| < 0.0124 (relative error < 2^-51, also next to the zeros);
+//   exp_acc: reduction by ln2/32 in two parts, 2^(j/32) from rocrand_amd_mathtab.h, series of
+//        exp(r) - 1 to r^5 on |r| < 0.0109 (relative error < 2^-48), scaling by 2^e in double.
 // The r^6 log, sin/cos and exp round to the correctly rounded float result but next to a
 // rounding boundary (relative distance 2^-44 or less), so each differs from the host
 // libm's float result by at most the host's own error (< 1 ulp).
@@ -130,26 +130,37 @@ struct math_tables
     const double*  psc  = rr_psc_tab[0];
 };
 
-// sin and cos of a Box-Muller angle v, each rounded to float: qoff = 16 q selects q =
-// round(128 v / pi), which the callers take from the word the angle came from.
-__host__ __device__ __forceinline__ void sincosf_unit(float v, uint32_t qoff, float& s, float& c,
-                                                      const math_tables& tab = math_tables{})
+// sin and cos of a Box-Muller angle v: qoff = 16 q selects q = round(128 v / pi), which the
+// callers take from the word the angle came from.  The table's step is pi/128 as a double:
+// with a step of 15 bits (a = v - q P exact in float) the entries next to a quarter turn
+// cancel with a, and the small sine or cosine kept only 42 bits.
+__host__ __device__ __forceinline__ void sincos_unit(float v, uint32_t qoff, double& s, double& c,
+                                                     const math_tables& tab = math_tables{})
 {
     ROCRAND_AMD_FP_EXACT
     const double2 t  = *reinterpret_cast<const double2*>(reinterpret_cast<const char*>(tab.sc) + qoff);
-    const double  a  = (double)__builtin_fmaf(-(float)qoff, RR_BM_ANGLE_STEP * 0.0625f, v);
+    const double  a  = __builtin_fma((double)qoff, -RR_BM_ANGLE_STEP / 16, (double)v);
     const double  a2 = a * a;
-    const double  sa = __builtin_fma(a * a2, __builtin_fma(a2, 1.0 / 120, -1.0 / 6), a);
+    double        sa = __builtin_fma(a2, -1.0 / 5040, 1.0 / 120);
+    sa               = __builtin_fma(a * a2, __builtin_fma(a2, sa, -1.0 / 6), a);
     double        ca = __builtin_fma(a2, -1.0 / 720, 1.0 / 24);
     ca               = __builtin_fma(a2, __builtin_fma(a2, ca, -0.5), 1.0);
-    s                = (float)__builtin_fma(t.x, ca, t.y * sa);
-    c                = (float)__builtin_fma(t.y, ca, -(t.x * sa));
+    s                = __builtin_fma(t.x, ca, t.y * sa);
+    c                = __builtin_fma(t.y, ca, -(t.x * sa));
+}
+__host__ __device__ __forceinline__ void sincosf_unit(float v, uint32_t qoff, float& s, float& c,
+                                                      const math_tables& tab = math_tables{})
+{
+    double sd, cd;
+    sincos_unit(v, qoff, sd, cd, tab);
+    s = (float)sd;
+    c = (float)cd;
 }
 
-// exp of a float, rounded to float: x = (32 e + j) ln2/32 + r, exp x = 2^e 2^(j/32) exp(r)
+// exp of a float, rounded to float by expf_acc: x = (32 e + j) ln2/32 + r, exp x = 2^e 2^(j/32) exp(r)
 // with the 2^(j/32) table of rocrand_amd_mathtab.h.  Arguments are clamped to [-110, 100]
 // first (the float result is then 0 or +inf already); a NaN passes through the clamp.
-__host__ __device__ __forceinline__ float expf_acc(float xf, const math_tables& tab = math_tables{})
+__host__ __device__ __forceinline__ double exp_acc(float xf, const math_tables& tab = math_tables{})
 {
     ROCRAND_AMD_FP_EXACT
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -159,17 +170,22 @@ __host__ __device__ __forceinline__ float expf_acc(float xf, const math_tables& 
 #endif
     const float  kf = __builtin_rintf(xc * (float)RR_EXP_INV_STEP);
     const int    k  = (int)kf;
-    const double r  = __builtin_fma((double)kf, -(RR_EXP_STEP_HI + RR_EXP_STEP_LO), (double)xc);
+    const double kd = (double)kf;
+    const double r  = __builtin_fma(kd, -RR_EXP_STEP_LO, __builtin_fma(kd, -RR_EXP_STEP_HI, (double)xc));
     double       p  = __builtin_fma(r, 1.0 / 120, 1.0 / 24);
     p               = __builtin_fma(p, r, 1.0 / 6);
     p               = __builtin_fma(p, r, 0.5);
     p               = __builtin_fma(p, r, 1.0);
     const double t  = tab.ex[k & ((1 << RR_EXPTAB_BITS) - 1)];
 #if defined(__HIP_DEVICE_COMPILE__)
-    return (float)__builtin_amdgcn_ldexp(__builtin_fma(t * r, p, t), k >> RR_EXPTAB_BITS);
+    return __builtin_amdgcn_ldexp(__builtin_fma(t * r, p, t), k >> RR_EXPTAB_BITS);
 #else
-    return (float)__builtin_ldexp(__builtin_fma(t * r, p, t), k >> RR_EXPTAB_BITS);
+    return __builtin_ldexp(__builtin_fma(t * r, p, t), k >> RR_EXPTAB_BITS);
 #endif
+}
+__host__ __device__ __forceinline__ float expf_acc(float xf, const math_tables& tab = math_tables{})
+{
+    return (float)exp_acc(xf, tab);
 }
 
 // ---------------------------------------------------------------- double functions

@@ -18,12 +18,13 @@ holds only u = 1: its entry is a = 1, b = -0, which gives -2 ln 1 = -0 (the refe
 b = 0) instead of its centre: r = u - 1 is then exact and small with ln u, so -2 ln u
 keeps its relative accuracy where it approaches 0.
 
-Box-Muller sine and cosine, 257 entries: angles q P, q = 0..256, P = pi/128 rounded to a
-float of 15 significant bits (q P and v - q P are exact in float for the angles v the
-transform sees, |v - q P| < 0.0124); entry q holds sin(q P), cos(q P) rounded to double.
+Box-Muller sine and cosine, 257 entries: angles q P, q = 0..256, P = pi/128 rounded to
+double (v - q P rounds once, |v - q P| < 0.0124); entry q holds sin(q P), cos(q P) rounded to
+double, which at a quarter turn is at most 2.5e-16, so that the small sine or cosine next to
+one is v - q P itself and nothing cancels.
 
 Float normals, sine and cosine, 513 entries: angles q P, q = 0..512, P = pi/256 rounded to 15
-significant bits (q P and v - q P exact in float as above, |v - q P| < 0.0063); entry q holds
+significant bits (q P and v - q P are exact in float for the angles v the transform sees, |v - q P| < 0.0063); entry q holds
 sin(q P)/2, cos(q P)/2 rounded to double (the radius comes out doubled).
 
 Double-precision Box-Muller pair (evaluated as double-doubles and rounded once):
@@ -91,13 +92,8 @@ def bm_log_entries():
     return out
 
 
-def bm_angle_step():
-    m, e = mpmath.frexp(mpmath.pi / 128)
-    return float(mpmath.nint(m * 2**15) * mpmath.power(2, e - 15))
-
-
 def bm_sincos_entries():
-    p = mpmath.mpf(bm_angle_step())
+    p = mpmath.mpf(float(mpmath.pi / 128))
     return [(float(mpmath.sin(q * p)), float(mpmath.cos(q * p))) for q in range(257)]
 
 
@@ -220,7 +216,7 @@ def main():
     p64 = split3(mpmath.pi / 64, 8)            # q pi/64 exact for q < 2^8
     bm_log_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}}}," for a, b in bm_log_entries())
     bm_sc_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}}}," for a, b in bm_sincos_entries())
-    bm_p = bm_angle_step()
+    bm_p = float(mpmath.pi / 128)
     nsc_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}}}," for a, b in normal_sincos_entries())
     nsc_p = float(rounded_to(mpmath.pi / 256, 15))
     plog_rows = "\n".join(f"    {{{a.hex()}, {b.hex()}, {c.hex()}, 0.0}}," for a, b, c in pair_log_entries())
@@ -257,7 +253,7 @@ constexpr uint32_t RR_BM_EMIN = {BM_EMIN}u;
 RR_MATH_TABLE const double2 rr_bm_logtab[{(BM_EMAX - BM_EMIN + 1) * 64}] = {{
 {bm_log_rows}
 }};
-constexpr float RR_BM_ANGLE_STEP = {bm_p.hex()}f; // pi/128 to 15 bits
+constexpr double RR_BM_ANGLE_STEP = {bm_p.hex()}; // pi/128 rounded to double
 // {{sin(q RR_BM_ANGLE_STEP), cos(q RR_BM_ANGLE_STEP)}}, q = 0..256
 RR_MATH_TABLE const double2 rr_bm_sctab[257] = {{
 {bm_sc_rows}

@@ -182,6 +182,30 @@ static void quarter_rows(int n)
     mrg_quarter_row<31>("quarter_mrg31", n);
 }
 
+// log2 of the worst relative error of the doubles that are rounded to float, in hundredths
+static void steps_row()
+{
+    double ws = 0.0, we = 0.0;
+    auto   rel = [](double got, __float128 exact) { return (double)fabsq(((__float128)got - exact) / exact); };
+    auto   angle = [&](uint32_t y) {
+        const float v = R_2POW32_INV_2PI + (float)y * R_2POW32_INV_2PI;
+        double      s, c;
+        sincos_unit(v, ((y >> 20) + 8u) & ~15u, s, c);
+        ws = fmax(ws, fmax(rel(s, sinq((__float128)v)), rel(c, cosq((__float128)v))));
+    };
+    for(long i = 0; i < 200000; i++)
+        angle((uint32_t)(next64() >> 13));
+    for(uint32_t q = 0; q < 4; q++) // next to the quarter turns, and the table's boundaries
+        for(uint32_t k = 0; k < 2000; k++)
+            angle((q << 30) + 256 * k), angle((q << 30) - 1 - 256 * k), angle((uint32_t)(next64() >> 13) & 0xff000000u | 0x00800000u);
+    for(long i = 0; i < 400000; i++)
+    {
+        const float x = -105.0f + (float)i * (195.0f / 400000);
+        we = fmax(we, rel(exp_acc(x), expq((__float128)x)));
+    }
+    printf("steps %ld %ld\n", (long)(100 * log2(ws)), (long)(100 * log2(we)));
+}
+
 int main(int argc, char** argv)
 {
     const long n = argc > 1 ? atol(argv[1]) : 100000;
@@ -230,6 +254,7 @@ int main(int argc, char** argv)
     }
     printf("pair_f64 %ld %ld %ld %ld\n", 2 * n, (long)(worst * 1e6), beyond, (long)(host * 1e6));
     quarter_rows((int)(n / 4000));
+    steps_row();
     printf("special %d %d %d %d\n", logf_unit(1.0f) == 0.0f, expf_acc(-200.0f) == 0.0f, isinf(expf_acc(200.0f)),
            isnan(expf_acc(NAN)));
     return 0;

@@ -54,3 +54,12 @@ def test_double_pair_next_to_quarter_turns(rows, name):
     assert worst <= 1_000_000
     assert beyond == 0
     assert steps >= 1_500_000  # the steps rounded one by one are further off
+
+
+def test_doubles_before_their_rounding_to_float(rows):
+    """The worst relative errors (100 log2) of the doubles that sincosf_unit and expf_acc round:
+    sin and cos a few roundings of 2^-53 (next to their zeros too), exp the r^6/720 that its
+    series leaves out at |r| = 0.0109 (2^-48.6) and a few roundings."""
+    sincos, exp = rows["steps"]
+    assert sincos <= -5100
+    assert exp <= -4840
