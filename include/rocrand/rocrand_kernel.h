@@ -8,10 +8,9 @@
  * skipahead_subsequence, skipahead_sequence, rocrand_uniform*, rocrand_normal*,
  * rocrand_log_normal*, rocrand_poisson* and rocrand_discrete*.  A state initialised with
  * (seed, subsequence, offset) produces the words of the reference state initialised the
- * same way; the engine arithmetic and the float transforms are the library's own
- * (rocrand_amd_engines.h, rocrand_amd_math.h), so a thread's float normals equal the bulk
- * generator's for the same words; its double normals take the reference's steps one by one
- * (the log-normals share them), within 2 ulp of the bulk generator's.  Jump matrices: rocrand_amd_jumptables.h.
+ * same way; the engine arithmetic and the transforms are the library's own
+ * (rocrand_amd_engines.h, rocrand_amd_math.h), so a thread's normals and log-normals equal the
+ * bulk generator's for the same words.  Jump matrices: rocrand_amd_jumptables.h.
  *
  * Sobol32/64 and their scrambled forms take the caller's direction vectors and scramble
  * constants (rocrand_get_direction_vectors32/64, rocrand_get_scramble_constants32/64).
@@ -1230,14 +1229,20 @@ __host__ __device__ __forceinline__ float2 box_muller(unsigned long long v)
 {
     return box_muller<LN>((unsigned int)v, (unsigned int)(v >> 32));
 }
-// rocrand_normal.h:76-96
+// rocrand_normal.h:76-96.  LN as above: the log-normals (and the normal approximation of
+// Poisson) take the reference's steps (log, sqrt, sin/cos, product, each rounded), the normals the
+// pair evaluated as double-doubles and rounded once.
+template<bool LN = false>
 __host__ __device__ __forceinline__ double2 box_muller_double(unsigned int a, unsigned int b, unsigned int c,
                                                               unsigned int d)
 {
     ROCRAND_AMD_FP_EXACT
 #if defined(__HIP_DEVICE_COMPILE__)
     double r0, r1;
-    ::rocrand_amd_engine::box_muller_double(a, b, c, d, r0, r1);
+    if constexpr(LN)
+        ::rocrand_amd_engine::box_muller_double(a, b, c, d, r0, r1);
+    else
+        ::rocrand_amd_engine::normal_pair_double(a, b, c, d, r0, r1);
     return double2{r0, r1};
 #else
     const unsigned long long v1 = (unsigned long long)a ^ ((unsigned long long)b << 21);
@@ -1248,11 +1253,16 @@ __host__ __device__ __forceinline__ double2 box_muller_double(unsigned int a, un
     return double2{sin(w * RPID) * s, cos(w * RPID) * s};
 #endif
 }
-__host__ __device__ __forceinline__ double2 box_muller_double(uint4 v) { return box_muller_double(v.x, v.y, v.z, v.w); }
+template<bool LN = false>
+__host__ __device__ __forceinline__ double2 box_muller_double(uint4 v)
+{
+    return box_muller_double<LN>(v.x, v.y, v.z, v.w);
+}
+template<bool LN = false>
 __host__ __device__ __forceinline__ double2 box_muller_double(ulonglong2 v)
 {
-    return box_muller_double((unsigned int)v.x, (unsigned int)(v.x >> 32), (unsigned int)v.y,
-                             (unsigned int)(v.y >> 32));
+    return box_muller_double<LN>((unsigned int)v.x, (unsigned int)(v.x >> 32), (unsigned int)v.y,
+                                 (unsigned int)(v.y >> 32));
 }
 // rocrand_normal.h:138-172
 template<int MRG, bool LN = false>
@@ -1273,13 +1283,16 @@ __host__ __device__ __forceinline__ float2 mrg_box_muller(unsigned int x, unsign
     return float2{sinf(v) * s, cosf(v) * s};
 #endif
 }
-template<int MRG>
+template<int MRG, bool LN = false>
 __host__ __device__ __forceinline__ double2 mrg_box_muller_double(unsigned int x, unsigned int y)
 {
     ROCRAND_AMD_FP_EXACT
 #if defined(__HIP_DEVICE_COMPILE__)
     double r0, r1;
-    ::rocrand_amd_engine::mrg_box_muller_double<MRG>(x, y, r0, r1);
+    if constexpr(LN)
+        ::rocrand_amd_engine::mrg_box_muller_double<MRG>(x, y, r0, r1);
+    else
+        ::rocrand_amd_engine::mrg_normal_pair_double<MRG>(x, y, r0, r1);
     return double2{r0, r1};
 #else
     const double u = (double)mrg_f32<MRG>(x);
@@ -1433,21 +1446,21 @@ __host__ __device__ __forceinline__ float2 bm2(mrg_engine<MRG>* s)
     const unsigned int b = s->next();
     return mrg_box_muller<MRG, LN>(a, b);
 }
-template<int MRG>
+template<bool LN = false, int MRG>
 __host__ __device__ __forceinline__ double2 bmd2(mrg_engine<MRG>* s)
 {
     const unsigned int a = s->next();
     const unsigned int b = s->next();
-    return mrg_box_muller_double<MRG>(a, b);
+    return mrg_box_muller_double<MRG, LN>(a, b);
 }
-template<class S>
+template<bool LN = false, class S>
 __host__ __device__ __forceinline__ double2 bmd2_words(S* s)
 {
     const unsigned int a = rocrand(s);
     const unsigned int b = rocrand(s);
     const unsigned int c = rocrand(s);
     const unsigned int d = rocrand(s);
-    return box_muller_double(a, b, c, d);
+    return box_muller_double<LN>(a, b, c, d);
 }
 } // namespace amd_detail
 } // namespace rocrand_device
@@ -1693,8 +1706,9 @@ namespace rocrand_device
 {
 namespace amd_detail
 {
-// The Box-Muller pairs of rocrand_normal2 with the log-normal variate (box_muller<true>),
-// and rocrand_normal's single value sharing the state's Box-Muller cache.
+// The Box-Muller pairs of rocrand_normal2 and rocrand_normal_double2 with the log-normal
+// variate (box_muller<true>, box_muller_double<true>), and the single values sharing the
+// state's Box-Muller caches.
 __host__ __device__ __forceinline__ float2 normal2_ln(rocrand_state_philox4x32_10* s) { return bm2<true>(s); }
 __host__ __device__ __forceinline__ float2 normal2_ln(rocrand_state_xorwow* s) { return bm2<true>(s); }
 __host__ __device__ __forceinline__ float2 normal2_ln(rocrand_state_mrg32k3a* s) { return bm2<true>(s); }
@@ -1722,10 +1736,48 @@ __host__ __device__ __forceinline__ float2 normal2_ln(rocrand_state_threefry4x64
     const unsigned long long b = rocrand(s);
     return box_muller<true>((unsigned int)a, (unsigned int)b);
 }
+__host__ __device__ __forceinline__ double2 normal_double2_ln(rocrand_state_philox4x32_10* s)
+{
+    return box_muller_double<true>(rocrand4(s));
+}
+__host__ __device__ __forceinline__ double2 normal_double2_ln(rocrand_state_xorwow* s) { return bmd2_words<true>(s); }
+__host__ __device__ __forceinline__ double2 normal_double2_ln(rocrand_state_mrg32k3a* s) { return bmd2<true>(s); }
+__host__ __device__ __forceinline__ double2 normal_double2_ln(rocrand_state_mrg31k3p* s) { return bmd2<true>(s); }
+__host__ __device__ __forceinline__ double2 normal_double2_ln(rocrand_state_lfsr113* s) { return bmd2_words<true>(s); }
+__host__ __device__ __forceinline__ double2 normal_double2_ln(rocrand_state_threefry2x32_20* s)
+{
+    const uint2 a = rocrand2(s);
+    const uint2 b = rocrand2(s);
+    return box_muller_double<true>(a.x, a.y, b.x, b.y);
+}
+__host__ __device__ __forceinline__ double2 normal_double2_ln(rocrand_state_threefry2x64_20* s)
+{
+    return box_muller_double<true>(rocrand2(s));
+}
+__host__ __device__ __forceinline__ double2 normal_double2_ln(rocrand_state_threefry4x32_20* s)
+{
+    return box_muller_double<true>(rocrand4(s));
+}
+__host__ __device__ __forceinline__ double2 normal_double2_ln(rocrand_state_threefry4x64_20* s)
+{
+    const unsigned long long a = rocrand(s);
+    const unsigned long long b = rocrand(s);
+    return box_muller_double<true>(ulonglong2{a, b});
+}
+// States without a cache: one word through the inverse error function.
+template<class S>
+__host__ __device__ __forceinline__ double normal_double_ln(S* state)
+{
+    return rocrand_normal_double(state);
+}
 #define ROCRAND_AMD_NORMAL_LN(STATE)                                                                         \
     __host__ __device__ __forceinline__ float normal_ln(STATE* state)                                        \
     {                                                                                                        \
         ROCRAND_AMD_BM_FLOAT(state, normal2_ln(state))                                                       \
+    }                                                                                                        \
+    __host__ __device__ __forceinline__ double normal_double_ln(STATE* state)                                \
+    {                                                                                                        \
+        ROCRAND_AMD_BM_DOUBLE(state, normal_double2_ln(state))                                               \
     }
 ROCRAND_AMD_NORMAL_LN(rocrand_state_philox4x32_10)
 ROCRAND_AMD_NORMAL_LN(rocrand_state_mrg32k3a)
@@ -1766,7 +1818,7 @@ __host__ __device__ __forceinline__ double ln_d(double mean, double stddev, doub
     __host__ __device__ __forceinline__ double2 rocrand_log_normal_double2(STATE* state, double mean,        \
                                                                            double stddev)                    \
     {                                                                                                        \
-        const double2 r = rocrand_normal_double2(state);                                                     \
+        const double2 r = rocrand_device::amd_detail::normal_double2_ln(state);                              \
         return double2{rocrand_device::amd_detail::ln_d(mean, stddev, r.x),                                  \
                        rocrand_device::amd_detail::ln_d(mean, stddev, r.y)};                                 \
     }
@@ -1780,7 +1832,8 @@ __host__ __device__ __forceinline__ double ln_d(double mean, double stddev, doub
     __host__ __device__ __forceinline__ double rocrand_log_normal_double(STATE* state, double mean,          \
                                                                          double stddev)                      \
     {                                                                                                        \
-        return rocrand_device::amd_detail::ln_d(mean, stddev, rocrand_normal_double(state));                 \
+        return rocrand_device::amd_detail::ln_d(mean, stddev,                                                \
+                                                rocrand_device::amd_detail::normal_double_ln(state));        \
     }
 ROCRAND_AMD_LN_CACHED(rocrand_state_philox4x32_10)
 ROCRAND_AMD_LN_CACHED(rocrand_state_mrg32k3a)
@@ -1838,7 +1891,7 @@ __host__ __device__ __forceinline__ double2 rocrand_log_normal_double2(rocrand_s
                                                                        double mean, double stddev)
 {
     using namespace rocrand_device::amd_detail;
-    const double2 r = rocrand_normal_double2(state);
+    const double2 r = normal_double2_ln(state);
     return double2{ln_d(mean, stddev, r.x), ln_d(mean, stddev, r.y)};
 }
 #define ROCRAND_AMD_LN_SOBOL(STATE)                                                                          \
@@ -1870,9 +1923,10 @@ __host__ __device__ __forceinline__ double4 rocrand_log_normal_double4(rocrand_s
                                                                        double mean, double stddev)
 {
     using namespace rocrand_device::amd_detail;
-    const double4 r = rocrand_normal_double4(state);
-    return double4{ln_d(mean, stddev, r.x), ln_d(mean, stddev, r.y), ln_d(mean, stddev, r.z),
-                   ln_d(mean, stddev, r.w)};
+    const double2 r1 = normal_double2_ln(state);
+    const double2 r2 = normal_double2_ln(state);
+    return double4{ln_d(mean, stddev, r1.x), ln_d(mean, stddev, r1.y), ln_d(mean, stddev, r2.x),
+                   ln_d(mean, stddev, r2.y)};
 }
 
 // ---------------------------------------------------------------- Poisson (rocrand_poisson.h)
@@ -1941,7 +1995,7 @@ template<class S, class R = unsigned int>
 __host__ __device__ __forceinline__ R poisson_huge(S* state, double lambda)
 {
     ROCRAND_AMD_FP_EXACT
-    const double n = rocrand_normal_double(state);
+    const double n = normal_double_ln(state);
     return (R)round(sqrt(lambda) * n + lambda);
 }
 template<class S>
@@ -2105,7 +2159,7 @@ __device__ __forceinline__ double2 rocrand_log_normal_double2(rocrand_state_mtgp
                                                               double stddev)
 {
     using namespace rocrand_device::amd_detail;
-    const double2 r = rocrand_normal_double2(state);
+    const double2 r = bmd2_words<true>(state);
     return double2{ln_d(mean, stddev, r.x), ln_d(mean, stddev, r.y)};
 }
 __device__ __forceinline__ unsigned int rocrand_poisson(rocrand_state_mtgp32* state, double lambda)

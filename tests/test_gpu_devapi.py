@@ -9,7 +9,8 @@ sequence of tests/devapi/program.h (tests/devapi/libdevapi_gpu.so).
   inverse-error-function normals and log-normals within the bars of parity_checks.py
   (the device's transcendentals are correctly rounded, the host libm's are not always).
 * Philox4x32-10 and ThreeFry 2x32 / 4x32 states at (seed, 0, offset) yield the bulk
-  generator's output for that seed (rocrand_generate, legacy ordering).
+  generator's output for that seed (rocrand_generate, legacy ordering); normals and
+  log-normals equal the bulk generator's for the same words bit for bit.
 """
 import os
 import sys
@@ -163,6 +164,31 @@ def test_device_states_continue_the_bulk_stream(gpu, engine, rng):
     off = np.arange(threads, dtype=np.uint64) * calls
     got = gpu.run(engine, C.F["WORD"], np.zeros(threads, np.uint64), off, calls, seed=seed)[:, :, 0]
     assert np.array_equal(got.astype(np.uint32).ravel(), bulk.cpu().numpy())
+
+
+@pytest.mark.parametrize("engine,rng", [("philox", "PHILOX4_32_10"), ("threefry4x32", "THREEFRY4_32_20"),
+                                         ("mrg32k3a", "MRG32K3A"), ("mrg31k3p", "MRG31K3P"), ("xorwow", "XORWOW")])
+@pytest.mark.parametrize("fn,call", [("NORMAL2", "normal"), ("NORMAL_D2", "normal"), ("LOGN2", "lognormal"),
+                                     ("LOGN_D2", "lognormal")])
+def test_device_normals_equal_the_bulk_generator(gpu, engine, rng, fn, call):
+    """The pairs of a thread's states equal the bulk generator's for the same words, bit for bit:
+    counter engines from word 2 i or 4 i on, interleaved engine i in subsequence i."""
+    import torch
+
+    from rocrand_amd import rocrand as R
+
+    n, double = 4096, "_D" in fn
+    i = np.arange(n, dtype=np.uint64)
+    counter = engine in ("philox", "threefry4x32")
+    off = i * np.uint64(4 if double else 2) if counter else np.zeros_like(i)
+    print(f"case {engine} {fn}", flush=True)
+    got = gpu.run(engine, C.F[fn], np.zeros_like(i) if counter else i, off, 1, a=0.0, b=1.0)[:, 0, :2].ravel()
+    bulk = torch.empty(2 * n, dtype=torch.float64 if double else torch.float32, device="cuda")
+    getattr(R.PRNG(getattr(R, rng), seed=C.SEED), call)(bulk, 0.0, 1.0)
+    torch.cuda.synchronize()
+    want = bulk.cpu().numpy()
+    got = got.view(np.float64) if double else got.astype(np.uint32).view(np.float32)
+    assert np.array_equal(got, want), np.flatnonzero(got != want)[:4]
 
 
 @pytest.mark.parametrize("engine,rng,bits", [("sobol32", "SOBOL32", 32), ("sobol64", "SOBOL64", 64)])
