@@ -3,7 +3,7 @@
 // Each stream is the output of one fresh generator's single generate call (see
 // include/rocrand_batched.h).  Streams are grouped by (engine, output kind); a group is
 // one persistent kernel whose blocks walk a list of tiles:
-//   * Philox: a tile is up to 1024 consecutive vecs of one stream, computed exactly as
+//   * Philox: a tile is a run of consecutive vecs of one stream, computed exactly as
 //     the per-call kernels do (rr_counter_dev.hpp), so outputs match the plain path bit
 //     for bit; the stream's head and tail go to its first tile;
 //   * MRG32k3a: a tile is up to 256 of a stream's engines.  A lane initialises its engine
@@ -15,7 +15,9 @@
 //     engines a stream uses are set up: min(S, vec_n + 1) instead of S per call.
 // The plan records the group launches in a HIP graph once; a launch replays it.  The
 // grid size of each group is chosen by timing a few candidates on the first plan of a
-// given shape (kept in a process-wide cache).
+// given shape (kept in a process-wide cache).  A batch of little work takes one launch for
+// all its groups (rr_batch_schedule.hpp).
+#include "rr_batch_schedule.hpp"
 #include "rr_counter_dev.hpp"
 #include "rr_generator.hpp"
 #include "rr_interleaved_dev.hpp"
@@ -34,9 +36,6 @@ namespace rr
 {
 namespace
 {
-
-constexpr uint32_t CTR_TILE_VECS = 4096; // 4 wavefronts x 16 chunks of 64
-constexpr uint32_t MRG_TILE      = 256;
 
 struct batch_tile
 {
@@ -367,7 +366,7 @@ launcher pick_launcher(bool philox, out_kind k)
 #undef RR_PICK
 }
 
-// All groups of a small batch in one launch, one tile per block.
+// All groups of a batch of little work in one launch, one tile per block.
 struct small_batch
 {
     struct part
@@ -430,7 +429,7 @@ struct group
     void*                     d_calls   = nullptr;
     void*                     d_tiles   = nullptr;
     const uint32_t*           d_states  = nullptr;
-    uint32_t                  blocks    = 2048;
+    uint32_t                  blocks    = 8192; // before tuning (2048: 2% to 10% slower from 512 MiB on, every kind)
     uint32_t                  tile_vecs = CTR_TILE_VECS; // Philox: vecs per tile
     uint32_t                  lds_bytes = 0; // largest Poisson table of the group, packed
     uint32_t ntiles() const { return (uint32_t)(philox ? tiles.size() : itiles.size()); }
@@ -489,6 +488,7 @@ struct batch_layout
     uint32_t                               nitiles = 0;
     size_t                                 upload = 0; // bytes made on the host
     size_t                                 bytes  = 0;
+    bool                                   single = false; // one launch for all groups
 
     static size_t align(size_t x) { return (x + 255) / 256 * 256; }
 
@@ -590,25 +590,8 @@ struct batch_layout
     }
 };
 
-// A batch of at most this many tiles goes in one launch (batch_small_kernel): its groups
-// would not fill the chip one by one, and six launches of 10 us each, in a row, are what
-// 256 streams of 10^2.5 to 10^5 values took.  They now take 9.5 us for the states and 33 us
-// for the one launch; the whole call went from 304 to 66 us, most of that host work.
-// Above, a group's own launch fills the chip and has its own tuned grid.
-constexpr uint32_t SMALL_TILES = 8192;
-
-uint64_t batch_tiles(const std::vector<group>& groups)
+hipError_t run_single(const std::vector<group>& groups, const device_tables& tables, hipStream_t s)
 {
-    uint64_t n = 0;
-    for(const auto& g : groups)
-        n += g.ntiles();
-    return n;
-}
-
-hipError_t run_small(const std::vector<group>& groups, const device_tables& tables, hipStream_t s, bool& done)
-{
-    if(batch_tiles(groups) > SMALL_TILES)
-        return hipSuccess;
     small_batch b{};
     uint32_t    total = 0, lds = 0;
     for(const auto& g : groups)
@@ -619,7 +602,6 @@ hipError_t run_small(const std::vector<group>& groups, const device_tables& tabl
         lds            = std::max(lds, g.lds_bytes);
         b.parts[b.n++] = {g.d_calls, g.d_tiles, g.d_states, total, (uint32_t)g.kind + (g.philox ? 0u : 32u)};
     }
-    done = true;
     if(total == 0)
         return hipSuccess;
     hipLaunchKernelGGL(batch_small_kernel, dim3(total), dim3(256), lds, s, b, tables);
@@ -631,13 +613,12 @@ hipError_t run_group(const group& g, const device_tables& tables, hipStream_t s)
     return g.fn(g.d_calls, g.d_tiles, g.d_states, g.ntiles(), std::min(g.blocks, g.ntiles()), g.lds_bytes, tables, s);
 }
 
-hipError_t run_groups(const std::vector<group>& groups, const device_tables& tables, hipStream_t s)
+hipError_t run_groups(const batch_layout& L, const device_tables& tables, hipStream_t s)
 {
-    bool       done = false;
-    hipError_t e    = run_small(groups, tables, s, done);
-    if(e != hipSuccess || done)
-        return e;
-    for(const auto& g : groups)
+    if(L.single)
+        return run_single(L.groups, tables, s);
+    hipError_t e = hipSuccess;
+    for(const auto& g : L.groups)
         if(g.ntiles() != 0 && (e = run_group(g, tables, s)) != hipSuccess)
             return e;
     return hipSuccess;
@@ -675,15 +656,11 @@ struct fork_join
     }
 };
 
-// run_groups under capture, each group on its side stream between fork and join.
+// A launch per group under capture, each on its side stream between fork and join.
 hipError_t run_groups_forked(const std::vector<group>& groups, const device_tables& tables, hipStream_t cap,
                              const fork_join& fj)
 {
-    bool       done = false;
-    hipError_t e    = run_small(groups, tables, cap, done);
-    if(e != hipSuccess || done)
-        return e;
-    e = hipEventRecord(fj.fork, cap);
+    hipError_t e = hipEventRecord(fj.fork, cap);
     for(size_t i = 0; i < groups.size() && e == hipSuccess; i++)
     {
         const group& g = groups[i];
@@ -839,6 +816,7 @@ struct rocrand_batch_plan_st
 {
     hipStream_t        stream = 0;
     std::vector<group> groups;
+    bool               single  = false; // one launch for all groups
     char*              d_image = nullptr;
     device_tables      tables{};
     hipGraph_t         graph    = nullptr;
@@ -862,8 +840,8 @@ struct rocrand_batch_plan_st
 namespace
 {
 
-// Validates the streams and lays out the batch on the host (no device calls).  `fine` lets
-// a small batch take smaller Philox tiles.
+// Validates the streams and lays out the batch on the host (no device calls).  Without `fine`
+// no Philox tile is smaller than CTR_TILE_VECS (a smaller image).
 rocrand_status build(batch_layout& L, const rocrand_batch_stream* streams, size_t count, bool fine = true)
 {
     // Poisson alias tables, one per distinct lambda (poisson.hpp:110-161, discrete.hpp:189-265)
@@ -983,34 +961,33 @@ rocrand_status build(batch_layout& L, const rocrand_batch_stream* streams, size_
         }
         g.bytes_out += b.n * (size_t)s.esz;
     }
-    // Schedules once the groups' sizes are known.  A batch for a single launch takes the
-    // smallest Philox tiles (256 vecs: one chunk per wavefront) that leave it half the
-    // launch's tiles, so that a block's serial work is short; any other the tuned ones.
-    auto philox_tiles = [&](uint32_t tile) {
+    // Schedules, once the groups' sizes are known
+    size_t bytes = 0, inter = 0;
+    for(const auto& g : L.groups)
+        bytes += g.bytes_out, inter += g.itiles.size();
+    const batch_launch how = batch_schedule(L.groups.size(), bytes, inter, [&](uint32_t vecs) {
         size_t n = 0;
         for(const auto& g : L.groups)
             for(const auto& c : g.ccalls)
-                n += c.vec_n / tile + 1;
+                n += c.vec_n / vecs + 1;
         return n;
-    };
-    size_t inter = 0;
-    for(const auto& g : L.groups)
-        inter += g.itiles.size();
-    uint32_t small = 0;
-    if(fine && inter + philox_tiles(CTR_TILE_VECS) <= SMALL_TILES / 2)
-        for(small = 256; inter + philox_tiles(small) > SMALL_TILES / 2;)
-            small *= 2;
+    });
+    L.single = how.single;
     for(auto& g : L.groups)
     {
-        std::lock_guard<std::mutex> lock(g_tune_mtx);
-        auto                        it = g_tuned.find(tune_key(g));
-        if(it != g_tuned.end())
+        g.tile_vecs = how.tile;
+        if(!L.single)
         {
-            g.blocks    = it->second.blocks;
-            g.tile_vecs = it->second.tile_vecs;
+            std::lock_guard<std::mutex> lock(g_tune_mtx);
+            auto                        it = g_tuned.find(tune_key(g));
+            if(it != g_tuned.end())
+            {
+                g.blocks    = it->second.blocks;
+                g.tile_vecs = it->second.tile_vecs;
+            }
         }
-        if(small != 0)
-            g.tile_vecs = small;
+        if(!fine)
+            g.tile_vecs = std::max(g.tile_vecs, CTR_TILE_VECS);
         if(g.philox)
             g.tiles = counter_tiles(g, g.tile_vecs);
     }
@@ -1152,7 +1129,6 @@ rocrand_status ROCRANDAPI rocrand_batch_plan_create(rocrand_batch_plan*         
         p         = new rocrand_batch_plan_st();
         p->stream = stream;
         // lay the batch out (with the cached schedules) and upload its descriptor image
-        bool small = false; // one launch, nothing to tune
         auto lay_out = [&]() {
             batch_layout   L;
             rocrand_status r = build(L, streams, count);
@@ -1169,13 +1145,13 @@ rocrand_status ROCRANDAPI rocrand_batch_plan_create(rocrand_batch_plan*         
                || L.make_states(p->d_image, p->tables, stream) != hipSuccess
                || hipStreamSynchronize(stream) != hipSuccess)
                 return ROCRAND_STATUS_INTERNAL_ERROR;
+            p->single = L.single;
             p->groups = std::move(L.groups);
-            small     = batch_tiles(p->groups) <= SMALL_TILES;
             return ROCRAND_STATUS_SUCCESS;
         };
         rocrand_status st = get_device_tables(p->tables) == hipSuccess ? lay_out() : ROCRAND_STATUS_INTERNAL_ERROR;
         bool relayout = false;
-        if(st == ROCRAND_STATUS_SUCCESS && !small)
+        if(st == ROCRAND_STATUS_SUCCESS && !p->single) // one launch has nothing to tune
             st = tune(*p, relayout);
         if(st == ROCRAND_STATUS_SUCCESS && relayout)
         {
@@ -1208,7 +1184,8 @@ rocrand_status ROCRANDAPI rocrand_batch_plan_create(rocrand_batch_plan*         
                 st = ROCRAND_STATUS_INTERNAL_ERROR;
             else if(st == ROCRAND_STATUS_SUCCESS)
             {
-                const hipError_t le = run_groups_forked(p->groups, p->tables, cap, fj);
+                const hipError_t le = p->single ? run_single(p->groups, p->tables, cap)
+                                                : run_groups_forked(p->groups, p->tables, cap, fj);
                 const hipError_t ce = hipStreamEndCapture(cap, &p->graph);
                 if(le != hipSuccess || ce != hipSuccess
                    || hipGraphInstantiate(&p->exec, p->graph, nullptr, nullptr, 0) != hipSuccess)
@@ -1288,7 +1265,7 @@ rocrand_status ROCRANDAPI rocrand_generate_batched(const rocrand_batch_stream* s
         L.pack(blk.host, blk.dev);
         const bool ok = hipMemcpyAsync(blk.dev, blk.host, L.upload, hipMemcpyHostToDevice, stream) == hipSuccess
                         && L.make_states(blk.dev, tables, stream) == hipSuccess
-                        && run_groups(L.groups, tables, stream) == hipSuccess;
+                        && run_groups(L, tables, stream) == hipSuccess;
         if(hipEventRecord(ev, stream) != hipSuccess)
         {
             // the block cannot be tracked: wait for the stream, then recycle it
@@ -1324,7 +1301,7 @@ rocrand_status ROCRANDAPI rocrand_generate_batched_noalloc(const rocrand_batch_s
             return st;
         if(L.groups.empty())
             return ROCRAND_STATUS_SUCCESS;
-        if(L.bytes > NOALLOC_SCRATCH_BYTES) // a small batch's tiles may be larger
+        if(L.bytes > NOALLOC_SCRATCH_BYTES) // its tiles may be larger
         {
             L = batch_layout{};
             if((st = build(L, streams, count, false)) != ROCRAND_STATUS_SUCCESS)
@@ -1341,7 +1318,7 @@ rocrand_status ROCRANDAPI rocrand_generate_batched_noalloc(const rocrand_batch_s
         std::vector<char> image(L.upload);
         L.pack(image.data(), dev);
         if(hipMemcpyAsync(dev, image.data(), L.upload, hipMemcpyHostToDevice, stream) != hipSuccess
-           || L.make_states(dev, tables, stream) != hipSuccess || run_groups(L.groups, tables, stream) != hipSuccess)
+           || L.make_states(dev, tables, stream) != hipSuccess || run_groups(L, tables, stream) != hipSuccess)
             return ROCRAND_STATUS_LAUNCH_FAILURE;
     }
     catch(const std::bad_alloc&)

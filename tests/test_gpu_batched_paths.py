@@ -1,6 +1,7 @@
 """Batches whose tiles fall on the edges of their paths, each stream against its plain call:
 MRG32k3a engines that wrap at, before and after a tile's end, misaligned outputs, one launch
-for a small batch and one per group for a larger one, streams without values."""
+for a batch of several groups and little work and one per group for any other, streams
+without values."""
 import ctypes
 
 import pytest
@@ -85,3 +86,18 @@ def test_small_and_large_batches():
     streams = [(R.MRG32K3A if i % 2 else R.PHILOX4_32_10, sorted(DT)[(i // 2) % 8], i, (1 << 20) + 7 + i, 3 * S + 5 + i,
                 i % 4) for i in range(40)]
     _check(streams)
+
+
+@pytest.mark.parametrize("rng,kind", [(R.PHILOX4_32_10, R.BATCH_UNIFORM_FLOAT), (R.PHILOX4_32_10, R.BATCH_NORMAL_DOUBLE),
+                                      (R.MRG32K3A, R.BATCH_NORMAL_FLOAT)])
+def test_one_group(rng, kind):
+    for n in (3, 4099, (1 << 17) + 1, (1 << 20) + 5):
+        _check([(rng, kind, i, i * 7919, n + i, i) for i in range(4)])
+
+
+def test_batches_next_to_the_limit_of_one_launch():
+    """512 MiB of output: 12 streams of two kinds just within it and just past it."""
+    n = (512 << 20) // 48
+    for extra in (-6, 6):
+        _check([(R.MRG32K3A if i % 2 else R.PHILOX4_32_10, (R.BATCH_UINT, R.BATCH_UNIFORM_FLOAT)[(i // 2) % 2], i, i, n + extra,
+                 0) for i in range(12)])
