@@ -1134,6 +1134,8 @@ rocrand_status ROCRANDAPI rocrand_batch_plan_create(rocrand_batch_plan*         
             rocrand_status r = build(L, streams, count);
             if(r != ROCRAND_STATUS_SUCCESS)
                 return r;
+            if(get_device_tables(p->tables) != hipSuccess)
+                return ROCRAND_STATUS_INTERNAL_ERROR;
             std::vector<char> image(L.upload);
             if(hipMalloc(reinterpret_cast<void**>(&p->d_image), L.bytes) != hipSuccess)
             {
@@ -1149,8 +1151,8 @@ rocrand_status ROCRANDAPI rocrand_batch_plan_create(rocrand_batch_plan*         
             p->groups = std::move(L.groups);
             return ROCRAND_STATUS_SUCCESS;
         };
-        rocrand_status st = get_device_tables(p->tables) == hipSuccess ? lay_out() : ROCRAND_STATUS_INTERNAL_ERROR;
-        bool relayout = false;
+        rocrand_status st       = lay_out();
+        bool           relayout = false;
         if(st == ROCRAND_STATUS_SUCCESS && !p->single) // one launch has nothing to tune
             st = tune(*p, relayout);
         if(st == ROCRAND_STATUS_SUCCESS && relayout)

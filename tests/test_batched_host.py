@@ -1,5 +1,5 @@
 """What the batched calls decide on the host (include/rocrand_batched.h): which batches fit the
-no-allocation call's array."""
+no-allocation call's array, and the status of streams that no call takes."""
 import ctypes
 
 import pytest
@@ -9,7 +9,7 @@ from rocrand_amd import rocrand as R
 torch = pytest.importorskip("torch")
 
 S = 131072
-OUT_OF_RANGE = 104
+TYPE_ERROR, OUT_OF_RANGE = 103, 104
 
 
 # Batches of MRG32k3a streams whose engines wrap (offset S - 1 or S - 100), cut into one tile
@@ -23,3 +23,20 @@ OUT_OF_RANGE = 104
 def test_batches_that_fit_the_no_allocation_array(rng, kind, offset, n, count):
     arr = (R.BatchStream * count)(*[R.BatchStream(rng, kind, i, offset, n, 0.0, 1.0, 0x1004) for i in range(count)])
     assert R.load().rocrand_generate_batched_noalloc(arr, count, None) != OUT_OF_RANGE
+
+
+@pytest.mark.parametrize("stream,want", [
+    ((R.XORWOW, R.BATCH_UINT, 1, 0, 10, 0.0, 1.0, 0x1000), TYPE_ERROR),
+    ((R.MRG32K3A, 8, 1, 0, 10, 0.0, 1.0, 0x1000), TYPE_ERROR),
+    ((R.PHILOX4_32_10, R.BATCH_UINT, 1, 0, 10, 0.0, 1.0, None), OUT_OF_RANGE),
+    ((R.PHILOX4_32_10, R.BATCH_POISSON, 1, 0, 10, 0.0, 1.0, 0x1000), OUT_OF_RANGE),
+    ((R.MRG32K3A, R.BATCH_POISSON, 1, 0, 10, float("nan"), 1.0, 0x1000), OUT_OF_RANGE)])
+def test_streams_are_checked_before_the_device_is_asked(stream, want):
+    """Every call names the stream's fault, also where there is no device."""
+    L = R.load()
+    arr = (R.BatchStream * 1)(R.BatchStream(*stream))
+    plan = ctypes.c_void_p()
+    assert L.rocrand_batch_plan_create(ctypes.byref(plan), arr, 1, None) == want
+    assert not plan
+    assert L.rocrand_generate_batched(arr, 1, None) == want
+    assert L.rocrand_generate_batched_noalloc(arr, 1, None) == want
