@@ -71,8 +71,10 @@ ROCRANDAPI rocrand_status rocrand_batch_plan_destroy(rocrand_batch_plan plan);
 /* One-shot: validates and lays out the batch and launches it without a graph,
  * asynchronously on `stream` (like any rocrand_generate_* call).  The descriptors go
  * through pooled pinned and device memory that is recycled once the launch has
- * completed, so repeated calls neither allocate in steady state nor wait for the device;
- * `streams` may be reused as soon as the call returns. */
+ * completed, so repeated calls neither allocate in steady state nor wait for the device
+ * (where the only memory of the size was last used on a stream that has been destroyed, a
+ * call waits for the device once instead of allocating); `streams` may be reused as soon as
+ * the call returns.  A captured call's memory stays with the graph. */
 ROCRANDAPI rocrand_status rocrand_generate_batched(const rocrand_batch_stream* streams,
                                                    size_t                      count,
                                                    hipStream_t                 stream);

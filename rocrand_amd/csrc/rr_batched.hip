@@ -21,6 +21,7 @@
 #include "rr_counter_dev.hpp"
 #include "rr_generator.hpp"
 #include "rr_interleaved_dev.hpp"
+#include "rr_staging.hpp"
 
 #include <rocrand_batched.h>
 
@@ -675,103 +676,6 @@ hipError_t run_groups_forked(const std::vector<group>& groups, const device_tabl
     return e;
 }
 
-// Device blocks with pinned host twins for the one-shot call's descriptor images,
-// recycled once the call that used them has completed (its event has fired).  Blocks
-// come in power-of-two sizes from 64 KiB and stay allocated for the process lifetime,
-// so a steady stream of calls allocates nothing and never waits for the device.
-class staging_pool
-{
-public:
-    struct block
-    {
-        char*  dev  = nullptr;
-        char*  host = nullptr;
-        size_t size = 0;
-        int    device = 0;
-    };
-
-    hipError_t acquire(int device, size_t bytes, block& b, hipEvent_t& ev)
-    {
-        size_t size = 64 << 10;
-        while(size < bytes)
-            size *= 2;
-        std::lock_guard<std::mutex> lock(mu_);
-        reclaim();
-        auto& fl = free_[std::make_pair(device, size)];
-        if(!fl.empty())
-        {
-            b = fl.back();
-            fl.pop_back();
-        }
-        else
-        {
-            b        = block{};
-            b.size   = size;
-            b.device = device;
-            hipError_t e = hipMalloc(reinterpret_cast<void**>(&b.dev), size);
-            if(e != hipSuccess)
-                return e;
-            e = hipHostMalloc(reinterpret_cast<void**>(&b.host), size, hipHostMallocDefault);
-            if(e != hipSuccess)
-            {
-                (void)hipFree(b.dev);
-                return e;
-            }
-        }
-        auto& evs = events_[device];
-        if(!evs.empty())
-        {
-            ev = evs.back();
-            evs.pop_back();
-            return hipSuccess;
-        }
-        return hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-    }
-
-    // Hands the block back once `ev` (recorded after the block's last use) has fired.
-    void release_after(const block& b, hipEvent_t ev)
-    {
-        std::lock_guard<std::mutex> lock(mu_);
-        pending_.push_back(std::make_pair(b, ev));
-    }
-
-    // Takes back the blocks whose events have fired (a caller whose streams are drained and
-    // about to be destroyed: an event cannot be asked once its stream is gone).
-    void collect()
-    {
-        std::lock_guard<std::mutex> lock(mu_);
-        reclaim();
-    }
-
-private:
-    void reclaim()
-    {
-        size_t keep = 0;
-        for(size_t i = 0; i < pending_.size(); i++)
-        {
-            const hipError_t e = hipEventQuery(pending_[i].second);
-            if(e == hipSuccess)
-            {
-                const block& b = pending_[i].first;
-                free_[std::make_pair(b.device, b.size)].push_back(b);
-                events_[b.device].push_back(pending_[i].second);
-                continue;
-            }
-            // An event whose stream is gone or is being captured cannot be asked: its block
-            // stays out of use, and the error is not left for the next launch to report.
-            if(e != hipErrorNotReady)
-                (void)hipGetLastError();
-            pending_[keep++] = pending_[i];
-        }
-        pending_.resize(keep);
-    }
-
-    std::mutex                                        mu_;
-    std::map<std::pair<int, size_t>, std::vector<block>> free_;
-    std::map<int, std::vector<hipEvent_t>>            events_;
-    std::vector<std::pair<block, hipEvent_t>>         pending_;
-};
-
 staging_pool& pool()
 {
     static staging_pool* p = new staging_pool(); // lives to process exit
@@ -1259,23 +1163,32 @@ rocrand_status ROCRANDAPI rocrand_generate_batched(const rocrand_batch_stream* s
             return ROCRAND_STATUS_INTERNAL_ERROR;
         // Descriptors go through a pooled pinned buffer and a pooled device block, both
         // released to the pool when the event recorded after the kernels has fired: the
-        // call returns without waiting for the device.
+        // call returns without waiting for the device.  Under capture the graph's copy node
+        // and kernels keep them.
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        const bool captured = stream != nullptr && hipStreamIsCapturing(stream, &capture) == hipSuccess
+                              && capture != hipStreamCaptureStatusNone;
         staging_pool::block blk;
         hipEvent_t          ev = nullptr;
-        if(pool().acquire(device, L.bytes, blk, ev) != hipSuccess)
+        if(pool().acquire(device, L.bytes, captured, blk, ev) != hipSuccess)
             return ROCRAND_STATUS_ALLOCATION_FAILED;
         L.pack(blk.host, blk.dev);
         const bool ok = hipMemcpyAsync(blk.dev, blk.host, L.upload, hipMemcpyHostToDevice, stream) == hipSuccess
                         && L.make_states(blk.dev, tables, stream) == hipSuccess
                         && run_groups(L, tables, stream) == hipSuccess;
-        if(hipEventRecord(ev, stream) != hipSuccess)
+        if(captured)
+            pool().leave_to_graph(blk, ev);
+        else
         {
-            // the block cannot be tracked: wait for the stream, then recycle it
-            (void)hipStreamSynchronize(stream);
-            (void)hipEventRecord(ev, 0);
-            (void)hipEventSynchronize(ev);
+            if(hipEventRecord(ev, stream) != hipSuccess)
+            {
+                // the block cannot be tracked: wait for the stream, then recycle it
+                (void)hipStreamSynchronize(stream);
+                (void)hipEventRecord(ev, 0);
+                (void)hipEventSynchronize(ev);
+            }
+            pool().release_after(blk, ev);
         }
-        pool().release_after(blk, ev);
         if(!ok)
             return ROCRAND_STATUS_LAUNCH_FAILURE;
     }

@@ -101,3 +101,70 @@ def test_batches_next_to_the_limit_of_one_launch():
     for extra in (-6, 6):
         _check([(R.MRG32K3A if i % 2 else R.PHILOX4_32_10, (R.BATCH_UINT, R.BATCH_UNIFORM_FLOAT)[(i // 2) % 2], i, i, n + extra,
                  0) for i in range(12)])
+
+
+def test_empty_batches():
+    """No streams, or only streams without values: every call succeeds and writes nothing."""
+    _check([])
+    _check([(R.MRG32K3A, R.BATCH_UINT, 1, 5, 0, 0), (R.PHILOX4_32_10, R.BATCH_NORMAL_FLOAT, 1, 5, 0, 1)])
+
+
+def _request(count, seed):
+    """`count` mixed streams, their outputs, and the values that plain calls give."""
+    specs = [(R.MRG32K3A if i % 2 else R.PHILOX4_32_10, R.BATCH_UNIFORM_FLOAT, seed + i, i * 7919, 257 + i % 3) for i in range(count)]
+    got = [torch.zeros(s[4], dtype=torch.float32, device="cuda") for s in specs]
+    want = [torch.zeros_like(v) for v in got]
+    for (rng, kind, sd, off, _), w in zip(specs, want):
+        _plain(rng, kind, sd, off, w, 0.0, 0.0)
+    arr = (R.BatchStream * count)(*[R.BatchStream(*s, 0.0, 0.0, v.data_ptr()) for s, v in zip(specs, got)])
+    torch.cuda.synchronize()
+    return arr, got, want
+
+
+def test_one_shot_calls_on_streams_that_are_destroyed():
+    """A program that makes a stream, calls, waits and destroys the stream, again and again: right
+    values, no status but success and no block more for each call."""
+    from test_gpu_graphs import Hip
+
+    hip, L = Hip(), R.load()
+    arr, got, want = _request(3000, 1)  # a descriptor image of about 1 MiB
+    free = None
+    for turn in range(40):
+        s = hip.stream()
+        for v in got[:4]:
+            v.zero_()
+        torch.cuda.synchronize()
+        assert L.rocrand_generate_batched(arr, len(arr), s) == 0
+        hip.check(hip.lib.hipStreamSynchronize(s))
+        hip.check(hip.lib.hipStreamDestroy(s))
+        assert all(torch.equal(g, w) for g, w in zip(got[:4], want[:4])), turn
+        if turn == 3:
+            free = torch.cuda.mem_get_info()[0]
+    assert all(torch.equal(g, w) for g, w in zip(got, want))
+    assert free - torch.cuda.mem_get_info()[0] < 8 << 20
+
+
+def test_captured_one_shot_call():
+    """Every replay of a captured call, with other calls between them."""
+    from test_gpu_graphs import Hip
+
+    hip, L = Hip(), R.load()
+    arr, got, want = _request(8, 100)
+    other, got2, want2 = _request(9, 200)
+    s = hip.stream()
+    for calls in (2, 1):  # the third finds both blocks done and leaves one to capture with
+        for _ in range(calls):
+            R.check_rocrand(L.rocrand_generate_batched(arr, len(arr), s))
+        hip.check(hip.lib.hipStreamSynchronize(s))
+    graph, exe = hip.capture(s, lambda: R.check_rocrand(L.rocrand_generate_batched(arr, len(arr), s)))
+    for _ in range(4):
+        for v in got + got2:
+            v.zero_()
+        torch.cuda.synchronize()
+        R.check_rocrand(L.rocrand_generate_batched(other, len(other), s))
+        hip.launch(s, exe)
+        R.check_rocrand(L.rocrand_generate_batched(other, len(other), s))
+        hip.check(hip.lib.hipStreamSynchronize(s))
+        assert all(torch.equal(g, w) for g, w in zip(got + got2, want + want2))
+    hip.destroy(graph, exe)
+    hip.check(hip.lib.hipStreamDestroy(s))
