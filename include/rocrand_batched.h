@@ -82,7 +82,8 @@ ROCRANDAPI rocrand_status rocrand_generate_batched(const rocrand_batch_stream* s
  * device or pinned memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  Same streams, same outputs as rocrand_generate_batched; the
  * descriptors go into a fixed 16 MiB array in device memory, one per GPU, held until the
- * process ends, and no allocation routine is called.  OUT_OF_RANGE when a batch's
+ * process ends, and no allocation routine is called (a captured call leaves the host copy
+ * of its descriptors, which every replay reads, to the graph).  OUT_OF_RANGE when a batch's
  * descriptors exceed that array (about 10^6 tiles of 16 Ki values, or fewer streams
  * with large Poisson tables).  Every call on a GPU shares that GPU's array: calls that
  * overlap on one GPU (issued on different streams) race; calls in order on one stream

@@ -29,6 +29,7 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <tuple>
 #include <vector>
@@ -676,6 +677,12 @@ hipError_t run_groups_forked(const std::vector<group>& groups, const device_tabl
     return e;
 }
 
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    return s != nullptr && hipStreamIsCapturing(s, &c) == hipSuccess && c != hipStreamCaptureStatusNone;
+}
+
 staging_pool& pool()
 {
     static staging_pool* p = new staging_pool(); // lives to process exit
@@ -1165,9 +1172,7 @@ rocrand_status ROCRANDAPI rocrand_generate_batched(const rocrand_batch_stream* s
         // released to the pool when the event recorded after the kernels has fired: the
         // call returns without waiting for the device.  Under capture the graph's copy node
         // and kernels keep them.
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        const bool captured = stream != nullptr && hipStreamIsCapturing(stream, &capture) == hipSuccess
-                              && capture != hipStreamCaptureStatusNone;
+        const bool          captured = capturing(stream);
         staging_pool::block blk;
         hipEvent_t          ev = nullptr;
         if(pool().acquire(device, L.bytes, captured, blk, ev) != hipSuccess)
@@ -1229,10 +1234,12 @@ rocrand_status ROCRANDAPI rocrand_generate_batched_noalloc(const rocrand_batch_s
         if(get_device_tables(tables) != hipSuccess || (dev = scratch_address()) == nullptr)
             return ROCRAND_STATUS_INTERNAL_ERROR;
         // Descriptors are packed in host memory and copied into the scratch array on the
-        // stream; a copy from pageable memory has read the host buffer when it returns.
-        std::vector<char> image(L.upload);
-        L.pack(image.data(), dev);
-        if(hipMemcpyAsync(dev, image.data(), L.upload, hipMemcpyHostToDevice, stream) != hipSuccess
+        // stream; a copy from pageable memory has read the host buffer when it returns, but
+        // a captured copy reads it at every replay: it stays for the graph then.
+        auto image = std::make_unique<std::vector<char>>(L.upload);
+        L.pack(image->data(), dev);
+        char* const host = capturing(stream) ? image.release()->data() : image->data();
+        if(hipMemcpyAsync(dev, host, L.upload, hipMemcpyHostToDevice, stream) != hipSuccess
            || L.make_states(dev, tables, stream) != hipSuccess || run_groups(L, tables, stream) != hipSuccess)
             return ROCRAND_STATUS_LAUNCH_FAILURE;
     }

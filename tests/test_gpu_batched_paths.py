@@ -144,26 +144,27 @@ def test_one_shot_calls_on_streams_that_are_destroyed():
     assert free - torch.cuda.mem_get_info()[0] < 8 << 20
 
 
-def test_captured_one_shot_call():
-    """Every replay of a captured call, with other calls between them."""
+@pytest.mark.parametrize("name", ["rocrand_generate_batched", "rocrand_generate_batched_noalloc"])
+def test_captured_one_shot_call(name):
+    """Every replay of a captured call, with other calls (and other host allocations) between them."""
     from test_gpu_graphs import Hip
 
-    hip, L = Hip(), R.load()
+    hip, generate = Hip(), getattr(R.load(), name)
     arr, got, want = _request(8, 100)
     other, got2, want2 = _request(9, 200)
     s = hip.stream()
     for calls in (2, 1):  # the third finds both blocks done and leaves one to capture with
         for _ in range(calls):
-            R.check_rocrand(L.rocrand_generate_batched(arr, len(arr), s))
+            R.check_rocrand(generate(arr, len(arr), s))
         hip.check(hip.lib.hipStreamSynchronize(s))
-    graph, exe = hip.capture(s, lambda: R.check_rocrand(L.rocrand_generate_batched(arr, len(arr), s)))
+    graph, exe = hip.capture(s, lambda: R.check_rocrand(generate(arr, len(arr), s)))
     for _ in range(4):
         for v in got + got2:
             v.zero_()
         torch.cuda.synchronize()
-        R.check_rocrand(L.rocrand_generate_batched(other, len(other), s))
+        R.check_rocrand(generate(other, len(other), s))
         hip.launch(s, exe)
-        R.check_rocrand(L.rocrand_generate_batched(other, len(other), s))
+        R.check_rocrand(generate(other, len(other), s))
         hip.check(hip.lib.hipStreamSynchronize(s))
         assert all(torch.equal(g, w) for g, w in zip(got + got2, want + want2))
     hip.destroy(graph, exe)
