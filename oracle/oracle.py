@@ -250,6 +250,17 @@ def poisson_table(lam):
     return off.value, prob[:size].copy(), alias[:size].copy()
 
 
+def poisson_cdf(lam):
+    """The running sums over the same values as poisson_table's (the quasi-random method's table)."""
+    size, off, p = ctypes.c_uint(0), ctypes.c_uint(0), ctypes.POINTER(ctypes.c_double)()
+    f = lib().orc_poisson_cdf
+    f.argtypes = [ctypes.c_double, ctypes.POINTER(ctypes.c_uint), ctypes.POINTER(ctypes.c_uint),
+                  ctypes.POINTER(ctypes.POINTER(ctypes.c_double))]
+    if f(lam, ctypes.byref(size), ctypes.byref(off), ctypes.byref(p)):
+        raise MemoryError("orc_poisson_cdf")
+    return np.ctypeslib.as_array(p, (size.value,)).copy()  # the oracle's few KiB stay allocated
+
+
 def discrete_tables(weights):
     """(prob, alias, cdf) of rocrand_create_discrete_distribution for `weights`."""
     w = np.ascontiguousarray(weights, dtype=np.float64)
