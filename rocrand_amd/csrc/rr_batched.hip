@@ -62,12 +62,13 @@ static_assert(INTERLEAVED_ENGINES == 1u << 17, "span layout");
 struct inter_call
 {
     uint32_t    seeded[6];
-    uint32_t    start;           // offset mod S
-    uint8_t     shift;           // vecs between the last 128-byte line boundary and vec 0
-    uint8_t     mis, head, tail; // below a vec's outputs
-    uint64_t    steps;           // offset / S
+    uint32_t    start; // offset mod S
+    uint16_t    shift; // vecs between the last 128-byte line boundary and vec 0
+    uint16_t    mis;
+    uint64_t    steps; // offset / S
     void*       data;
     size_t      n, vec_n;
+    uint32_t    head, tail;
     dist_params params;
 };
 
@@ -845,15 +846,15 @@ rocrand_status build(batch_layout& L, const rocrand_batch_stream* streams, size_
             c.start    = (uint32_t)(b.offset % INTERLEAVED_ENGINES);
             c.data     = b.output;
             c.n        = b.n;
-            c.mis      = (uint8_t)((s.out_w - (addr / s.esz) % s.out_w) % s.out_w);
-            c.head     = (uint8_t)std::min<size_t>(b.n, c.mis);
-            c.tail     = (uint8_t)((b.n - c.head) % s.out_w);
+            c.mis      = (uint16_t)((s.out_w - (addr / s.esz) % s.out_w) % s.out_w);
+            c.head     = (uint32_t)std::min<size_t>(b.n, c.mis);
+            c.tail     = (uint32_t)((b.n - c.head) % s.out_w);
             c.vec_n    = (b.n - c.head) / s.out_w;
             c.params   = prm;
             {
                 const uintptr_t vaddr  = addr + (uintptr_t)c.mis * s.esz;
                 const unsigned  vbytes = s.out_w * s.esz;
-                c.shift = (uint8_t)(128u % vbytes == 0 ? (vaddr / vbytes) % (128u / vbytes) : 0u);
+                c.shift = (uint16_t)(128u % vbytes == 0 ? (vaddr / vbytes) % (128u / vbytes) : 0u);
             }
             L.icalls.push_back(c);
             const bool   extra = s.out_w > 1 && (c.head > 0 || c.tail > 0);

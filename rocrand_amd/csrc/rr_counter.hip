@@ -3,10 +3,11 @@
 // The output map is described in rr_counter_dev.hpp.  The reference's grid is not this
 // kernel's grid: any schedule that computes that map is equivalent.
 //
-// Schedule: one vec per lane over a grid that covers the whole call (up to 4 for the
-// transforms that stage tables), so the resident wavefronts always write one contiguous
-// front of the output (16-byte stores, 1 KiB per wavefront).  A grid-stride loop over a small grid spreads the
-// concurrent stores over the whole buffer and was measured 1.5x slower on MI355X.
+// Schedule: one vec per lane over a grid that covers the whole call (4 or 8 for the
+// transforms that stage tables, 8 from a mid-block start), so the resident wavefronts always
+// write one contiguous front of the output (16-byte stores, 1 KiB per wavefront).  A
+// grid-stride loop over a small grid spreads the concurrent stores over the whole buffer and
+// was measured 1.5x slower on MI355X.
 #include "rr_counter_dev.hpp"
 
 namespace rr

@@ -123,8 +123,8 @@ __global__ __launch_bounds__(64) void mtgp_seed_kernel(mtgp_state* states, const
 
 // d_params of the current device, checked and uploaded on the first call there: the kernel
 // evaluates the recurrence table from its entries at 1, 2, 4 and 8 (the tempering table is
-// linear too and checked with it), and its unmasked ring reads reach off + 255 + pos with
-// off < 1024.
+// linear too and checked with it), and its unmasked ring reads reach word 768 + 255 + pos,
+// which the 95 words copied behind the ring hold for pos <= 95.
 rocrand_status device_params(const mtgp_param*& out);
 
 struct mtgp_call
