@@ -533,9 +533,9 @@ __device__ __forceinline__ void box_muller_double(uint32_t a, uint32_t b, uint32
 // exactly one for one pair in some 10^7) the small sine or cosine is the table entry's tail,
 // itself a rounded double, so that value is within 1 ulp (0.89 the largest of 2.6e7 there),
 // and the head's part of the radius' tail alone would leave it 40 ulp off: hence
-// (sn + se) tl and (cs + ce) tl.  117 VALU instructions with its uniforms and the
-// affine step; taking those steps one by one, each correctly rounded, costs 243 (XORWOW
-// normal f64, 2^27 values: 2.10 -> 3.57 TB/s, MRG32k3a 2.07 -> 3.56, Philox 1.98 -> 3.14).
+// (sn + se) tl and (cs + ce) tl.  117 VALU instructions with its uniforms and the affine
+// step; taking those steps one by one, each correctly rounded, costs 243 (2^28 normal f64
+// values: XORWOW 2.08 -> 3.51 TB/s, MRG32k3a 2.06 -> 3.51, Philox 2.01 -> 3.09).
 __host__ __device__ __forceinline__ void box_muller_pair_double(double u, double t, uint32_t qoff, double& r0,
                                                                 double& r1, const math_tables& tab)
 {
