@@ -109,6 +109,9 @@ struct rocrand_generator_base_type
     virtual rocrand_status set_dimensions(unsigned int d);
     rocrand_status         set_stream(hipStream_t s);
     virtual rocrand_status init() = 0;
+    // Waits, after init(), for what it left to the stream where a later call on another
+    // stream may rely on it.
+    virtual rocrand_status settle() { return ROCRAND_STATUS_SUCCESS; }
 
     // Entry for every rocrand_generate_*: host generators stage through device memory.
     rocrand_status generate(rr::out_kind k, void* data, size_t n, const rr::gen_args& args);
@@ -121,6 +124,8 @@ struct rocrand_generator_base_type
     rocrand_status initialize()
     {
         rocrand_status st = init();
+        if(st == ROCRAND_STATUS_SUCCESS)
+            st = settle();
         if(st == ROCRAND_STATUS_SUCCESS && host_mode == 0)
             st = m_poisson.reserve();
         return st;

@@ -387,6 +387,21 @@ public:
         if(hipGetLastError() != hipSuccess)
             return ROCRAND_STATUS_LAUNCH_FAILURE;
         m_initialized = true;
+        m_seeding     = true;
+        return ROCRAND_STATUS_SUCCESS;
+    }
+
+    // An explicit set-up returns with the states made, whatever stream the generate calls then
+    // run on (set-up had copied them and waited).  A capturing stream cannot be waited for.
+    rocrand_status settle() override
+    {
+        hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+        if(!m_seeding
+           || (stream != nullptr && hipStreamIsCapturing(stream, &c) == hipSuccess && c != hipStreamCaptureStatusNone))
+            return ROCRAND_STATUS_SUCCESS;
+        if(hipStreamSynchronize(stream) != hipSuccess)
+            return ROCRAND_STATUS_LAUNCH_FAILURE;
+        m_seeding = false;
         return ROCRAND_STATUS_SUCCESS;
     }
 
@@ -432,7 +447,7 @@ protected:
         if((st = init()) != ROCRAND_STATUS_SUCCESS)
             return st;
         if(data == nullptr)
-            return ROCRAND_STATUS_SUCCESS;
+            return settle();
         const uintptr_t addr = reinterpret_cast<uintptr_t>(data);
         c.mis    = (s.out_w - (addr / s.esz) % s.out_w) % s.out_w;
         c.head   = (uint32_t)std::min<size_t>(n, c.mis);
@@ -441,6 +456,7 @@ protected:
         c.states = static_cast<mtgp_state*>(m_states);
         c.data   = data;
         c.n      = n;
+        m_seeding = false; // the call's own work follows the seeding on its stream
         if(dispatch(k, c, stream) != hipSuccess)
             return ROCRAND_STATUS_LAUNCH_FAILURE;
         return ROCRAND_STATUS_SUCCESS;
@@ -449,6 +465,7 @@ protected:
 private:
     unsigned long long m_seed        = 0;
     bool               m_initialized = false;
+    bool               m_seeding     = false; // seeded since the last wait or generate call
     void*              m_states      = nullptr;
 };
 

@@ -94,3 +94,24 @@ def test_mtgp32_states_under_new_seeds():
         torch.cuda.synchronize()
         assert np.array_equal(got.cpu().numpy(), _want(O.MTGP32, n, seed=seed))
 
+
+@pytest.mark.parametrize("call", ["initialize", "generate_null"])
+def test_mtgp32_set_up_returns_with_the_states_made(call):
+    """Set up on a busy stream, then used on another one without a wait between them."""
+    n, seed = 512 * 256 + 3, 42
+    busy, other = torch.cuda.Stream(), torch.cuda.Stream()
+    work = torch.empty(1 << 28, device="cuda")
+    torch.cuda.synchronize()
+    p = R.PRNG(R.PHILOX4_32_10, stream=busy)
+    for _ in range(20):  # 3 ms of stores
+        p.uniform(work)
+    g = R.PRNG(R.MTGP32, seed=seed, stream=busy)
+    if call == "initialize":
+        g.initialize()
+    else:
+        assert R.load().rocrand_generate(g._gen, None, 0) == 0
+    g.stream = other
+    buf = torch.empty(n, dtype=torch.uint32, device="cuda")
+    g.generate(buf)
+    torch.cuda.synchronize()
+    assert np.array_equal(buf.cpu().numpy(), _want(O.MTGP32, n, seed=seed))
